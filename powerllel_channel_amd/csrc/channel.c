@@ -435,10 +435,13 @@ int pll_channel_run(pll_channel *c, pll_ppe *ppe, int nsteps, double *u, double 
     const int fmask = (c->is_forced[0] ? 1 : 0) | (c->is_forced[1] ? 2 : 0);
     /* The projecting RK1 issues more loads per value than RK1 and correctVel
      * together and needs enough workgroups to hide them: at 768x384x256
-     * (4608 tiles) the chain is 2% faster per step, at 192x192x128 (288
-     * tiles) 10% slower, so small grids take the per-step path. */
+     * (4608 64 x 4 x 64 tiles) the chain is 2% faster per step, at
+     * 192x192x128 (288 tiles) 10% slower, so small grids take the per-step
+     * path. */
     const char *pc = getenv("PLL_RUN_CHAIN"); /* tuning: 0 never, 1 always */
-    const int big = pll_rk_blocks(&c->g) >= 2048;
+    const long long t64 = (long long)((c->g.nx + 63) / 64) * ((c->g.ny + 3) / 4) *
+                          ((c->g.nz + 63) / 64);
+    const int big = t64 >= 2048;
     const int chain = !c->is_forced[2] && pll_ppe_refinement(ppe) < 0 &&
                       (pc ? atoi(pc) != 0 : big);
     int rc;
