@@ -201,11 +201,11 @@ int pll_channel_step(pll_channel *c, pll_ppe *ppe, double *u, double *v,
                      void *stream);
 /* nsteps calls of pll_channel_step (src/main.f90:131-212 without the
  * per-step checks and output), with the same results bit for bit.  With the
- * FP64 solve, w not forced and a large grid (at least 2048 RK tiles of
- * 64 x 4 x 64 cells), each step's projection (correctVel, forcing, boundary
- * fill) is formed inside the next step's RK1 and RK2 as they read the
- * velocity, which saves one pass over the fields per step; the run works in
- * place and allocates no device memory. */
+ * FP64 solve and w not forced, each step's projection (correctVel, forcing,
+ * boundary fill) is formed as the next step reads the velocity, and RK1 and
+ * RK2 of that step are one pass; (u, v, w) and the work space (u1, v1, w1)
+ * take the steps' velocity in turn, so what the latter hold after the call is
+ * unspecified.  The run allocates no device memory. */
 int pll_channel_run(pll_channel *c, pll_ppe *ppe, int nsteps, double *u,
                     double *v, double *w, double *u1, double *v1, double *w1,
                     double *p, void *stream);

@@ -167,7 +167,8 @@ int pll_channel_correct_vel(pll_channel *c, const double *p, double *u, double *
                             void *stream)
 {
     CHK_C(c);
-    return kl(pll_launch_correct_vel(&c->g, p, u, v, w, 0, 0.0, 0.0, NULL, (hipStream_t)stream),
+    const double *q[3] = {u, v, w};
+    return kl(pll_launch_correct_vel(&c->g, p, q, u, v, w, 0, 0.0, 0.0, NULL, (hipStream_t)stream),
               "correct_vel");
 }
 
@@ -345,7 +346,8 @@ static int step_impl(pll_channel *c, pll_ppe *ppe, double *u, double *v, double 
         if ((rc = pll_channel_bc_p(c, p, stream))) return rc;
     }
     if (fuse || none) {
-        if ((rc = kl(pll_launch_correct_vel(&c->g, p, u, v, w, fuse ? fmask : 0, c->vel_force[0],
+        const double *q[3] = {u, v, w};
+        if ((rc = kl(pll_launch_correct_vel(&c->g, p, q, u, v, w, fuse ? fmask : 0, c->vel_force[0],
                                             c->vel_force[1], fuse ? c->scal + 4 : NULL, s),
                      "correct_vel")))
             return rc;
@@ -362,69 +364,54 @@ int pll_channel_step(pll_channel *c, pll_ppe *ppe, double *u, double *v, double 
     return step_impl(c, ppe, u, v, w, u1, v1, w1, p, NULL, stream);
 }
 
-/* A step of a chain up to its pressure solve, in place on X = (u, v, w):
- * proj == 0: X is projected (the caller's state), plain RK1 and RK2;
- * proj == 1: X is the previous step's RK2 output, unprojected (its boundary
- * fill not made either), and p that step's pressure: RK1 projects every
- * value it reads (pll_launch_rk1_corr, writing only the RK1 stage) and RK2
- * projects its old value at each cell as it reads it (pll_launch_rk2_proj),
- * both from p and the forcing means of the previous step.  Then the forcing
- * means of the new RK2 output and the FP64 solve with calcRHS formed in its
- * x transform.  The projection of X and its boundary fill are left to the
- * next step (or to the chain's final projection). */
-static int chain_step(pll_channel *c, pll_ppe *ppe, int proj, double *const *X, double *u1,
-                      double *v1, double *w1, double *p, int fmask, hipStream_t s)
-{
-    const int nb = pll_rk_blocks(&c->g);
-    const double *mean = fmask ? c->scal + 4 : NULL;
-    const double dti = 1.0 / c->g.dt;
-    int rc;
-    if (!proj) {
-        if ((rc = kl(pll_launch_rk1(&c->g, X[0], X[1], X[2], u1, v1, w1, NULL, s), "rk1")))
-            return rc;
-        if ((rc = kl(pll_launch_rk2(&c->g, X[0], X[1], X[2], u1, v1, w1, fmask ? c->part : NULL,
-                                    fmask, NULL, 1, s),
-                     "rk2")))
-            return rc;
-    } else {
-        if ((rc = kl(pll_launch_rk1_corr(&c->g, X[0], X[1], X[2], p, NULL, NULL, NULL, u1, v1,
-                                         w1, fmask, c->vel_force[0], c->vel_force[1], mean, s),
-                     "rk1 (projecting)")))
-            return rc;
-        if ((rc = kl(pll_launch_rk2_proj(&c->g, X[0], X[1], X[2], u1, v1, w1, p,
-                                         fmask ? c->part : NULL, fmask, c->vel_force[0],
-                                         c->vel_force[1], mean, s),
-                     "rk2 (projecting)")))
-            return rc;
-    }
-    for (int d = 0; d < 2; d++)
-        if ((fmask >> d) & 1)
-            if ((rc = kl(pll_launch_mean_final(nb, c->part + (size_t)d * nb, c->scal + 4 + d,
-                                               c->g.nx, c->g.ny, s),
-                         "mean final")))
-                return rc;
-    /* no boundary fill of X: the solve's calcRHS and the next step's RK1
-     * read the values the fill would leave from the interior */
-    pll_div_src q = {X[0], X[1], X[2], c->g.dzf_inv, dti, dti * c->g.dx_inv,
-                     dti * c->g.dy_inv, 1};
-    return pll_ppe_solve_div(ppe, &q, p, s);
-}
-
-/* m steps whose projections are carried into the next step's RK1 and RK2:
- * step n leaves its RK2 output and pressure p unprojected in place; the
- * next step's RK1 and RK2 read both and project every value they read.
- * After the last step the final projection (correctVel + forcing + boundary
- * fill) is made in place.  Same kernels and roundings as m calls of
- * step_impl. */
+/* m steps whose projections are carried into the next step.  Step 0 takes
+ * the caller's state (whatever its ghost cells hold) through RK1 and RK2 in
+ * place.  Every later step reads the previous step's RK2 output X, neither
+ * projected nor filled, and that step's pressure p: one kernel projects each
+ * value as it reads it and makes RK1 and RK2 of it (pll_launch_rk12), into
+ * the other of the two sets (u, v, w) and (u1, v1, w1).  Each step then
+ * reduces the forcing means of its RK2 output and solves with calcRHS formed
+ * in the x transform, which like the next step takes the values the boundary
+ * fill would leave from the interior.  After the last step the projection
+ * (correctVel + forcing + boundary fill) goes to (u, v, w).  Same roundings
+ * as m calls of step_impl. */
 static int run_chain(pll_channel *c, pll_ppe *ppe, int m, double *u, double *v, double *w,
                      double *u1, double *v1, double *w1, double *p, int fmask, hipStream_t s)
 {
-    double *X[3] = {u, v, w};
+    double *const A[3] = {u, v, w}, *const B[3] = {u1, v1, w1};
+    double *const *X = A;
     const double *mean = fmask ? c->scal + 4 : NULL;
+    double *part = fmask ? c->part : NULL;
+    const double dti = 1.0 / c->g.dt;
+    const int nb = pll_rk_blocks(&c->g);
     int rc;
-    for (int i = 0; i < m; i++)
-        if ((rc = chain_step(c, ppe, i > 0, X, u1, v1, w1, p, fmask, s))) return rc;
-    if ((rc = kl(pll_launch_correct_vel(&c->g, p, u, v, w, fmask, c->vel_force[0],
+    for (int i = 0; i < m; i++) {
+        if (i == 0) {
+            if ((rc = kl(pll_launch_rk1(&c->g, u, v, w, u1, v1, w1, NULL, s), "rk1")) ||
+                (rc = kl(pll_launch_rk2(&c->g, u, v, w, u1, v1, w1, part, fmask, NULL, 1, s),
+                         "rk2")))
+                return rc;
+        } else {
+            const double *q[3] = {X[0], X[1], X[2]};
+            double *const *Y = X == A ? B : A;
+            if ((rc = kl(pll_launch_rk12(&c->g, q, Y, p, part, fmask, c->vel_force[0],
+                                         c->vel_force[1], mean, NULL, s),
+                         "rk1 + rk2")))
+                return rc;
+            X = Y;
+        }
+        for (int d = 0; d < 2; d++)
+            if ((fmask >> d) & 1)
+                if ((rc = kl(pll_launch_mean_final(nb, c->part + (size_t)d * nb, c->scal + 4 + d,
+                                                   c->g.nx, c->g.ny, s),
+                             "mean final")))
+                    return rc;
+        const pll_div_src q = {X[0], X[1], X[2], c->g.dzf_inv, dti, dti * c->g.dx_inv,
+                               dti * c->g.dy_inv, 1};
+        if ((rc = pll_ppe_solve_div(ppe, &q, p, s))) return rc;
+    }
+    const double *q[3] = {X[0], X[1], X[2]};
+    if ((rc = kl(pll_launch_correct_vel(&c->g, p, q, u, v, w, fmask, c->vel_force[0],
                                         c->vel_force[1], mean, s),
                  "correct_vel")))
         return rc;
@@ -440,19 +427,15 @@ int pll_channel_run(pll_channel *c, pll_ppe *ppe, int nsteps, double *u, double 
     if (!u || !v || !w || !u1 || !v1 || !w1 || !p) return pll_set_error(PLL_EINVAL, "NULL field");
     hipStream_t s = (hipStream_t)stream;
     const int fmask = (c->is_forced[0] ? 1 : 0) | (c->is_forced[1] ? 2 : 0);
-    /* The projecting RK1 issues more loads per value than RK1 and correctVel
-     * together and needs enough workgroups to hide them: at 768x384x256
-     * (4608 64 x 4 x 64 tiles) the chain is 2% faster per step, at
-     * 192x192x128 (288 tiles) 10% slower, so small grids take the per-step
-     * path. */
-    const char *pc = getenv("PLL_RUN_CHAIN"); /* tuning: 0 never, 1 always */
-    const long long t64 = (long long)((c->g.nx + 63) / 64) * ((c->g.ny + 3) / 4) *
-                          ((c->g.nz + 63) / 64);
-    const int big = t64 >= 2048;
-    const int chain = !c->is_forced[2] && pll_ppe_refinement(ppe) < 0 &&
-                      (pc ? atoi(pc) != 0 : big);
+    /* From the second step on the chain moves 152 N bytes per step (RK1 + RK2
+     * from the unprojected velocity 56, calcRHS + x transform 32, the rest of
+     * the solve 64) where step_impl moves 272 N, in two launches less; per step,
+     * as steps and as a chain of ten, 192x192x128 326 -> 291 us, 64x64x64 the
+     * same, 384x384x192 1.73 -> 1.27 ms, 768x384x256 4.6 -> 3.0 ms. */
+    const char *pc = getenv("PLL_RUN_CHAIN"); /* tuning: 0 never */
+    const int chain = !c->is_forced[2] && pll_ppe_refinement(ppe) < 0 && !(pc && atoi(pc) == 0);
     int rc;
-    if (!chain || nsteps < 3) {
+    if (!chain || nsteps < 2) {
         for (int i = 0; i < nsteps; i++)
             if ((rc = step_impl(c, ppe, u, v, w, u1, v1, w1, p, NULL, stream))) return rc;
         return PLL_OK;

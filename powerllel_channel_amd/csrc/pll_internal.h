@@ -182,16 +182,6 @@ typedef struct {
 int pll_launch_rk1(const pll_grid_dev *g, const double *u, const double *v,
                    const double *w, double *u1, double *v1, double *w1,
                    const double *const *body, hipStream_t s);
-/* RK1 from an unprojected velocity (u, v, w: the previous RK2 output after its
- * boundary fill; p: its pressure with ghosts): every value read is projected
- * on load as correctVel + forceVel (fmask bits with vfu, vfv and the device
- * means mean[0..1]; mean NULL: no forcing) + updateBoundVel would leave it;
- * the projected interior is written to (nu, nv, nw), the RK1 result to
- * (u1, v1, w1). */
-int pll_launch_rk1_corr(const pll_grid_dev *g, const double *u, const double *v,
-                        const double *w, const double *p, double *nu, double *nv, double *nw,
-                        double *u1, double *v1, double *w1, int fmask, double vfu, double vfv,
-                        const double *mean, hipStream_t s);
 /* mpart non-NULL and fmask != 0: also the Mean_h partial sums of the new u
  * (fmask bit 0) and v (bit 1), pll_rk_blocks(g) of each, u's first. */
 /* fill != 0: (u1, v1, w1) have no boundary fill; RK2 reads the values the
@@ -199,20 +189,25 @@ int pll_launch_rk1_corr(const pll_grid_dev *g, const double *u, const double *v,
 int pll_launch_rk2(const pll_grid_dev *g, double *u, double *v, double *w,
                    const double *u1, const double *v1, const double *w1, double *mpart,
                    int fmask, const double *const *body, int fill, hipStream_t s);
-/* RK2 of a multi-step run in place on (u, v, w), the previous step's
- * unprojected RK2 output, projected with p (and the forcing shift from mean)
- * as it is read; Mean_h partials into mpart as pll_launch_rk2 */
-int pll_launch_rk2_proj(const pll_grid_dev *g, double *u, double *v, double *w,
-                        const double *u1, const double *v1, const double *w1,
-                        const double *p, double *mpart, int fmask, double vfu,
-                        double vfv, const double *mean, hipStream_t s);
 int pll_rk_blocks(const pll_grid_dev *g);
+/* ntx, nty, nkc, planes per k chunk and XCD numbering of the RK2 tiles */
+void pll_rk_tiling(const pll_grid_dev *g, int rk[5]);
+/* RK1 and RK2 of a step in one pass (rk_fused.hip): q the velocity, o the RK2
+ * output (other arrays than q).  p NULL: q is projected and its boundary fill
+ * is made.  p non-NULL: q is the previous step's unprojected RK2 output and p
+ * its pressure; every value is projected as it is read (with the forcing
+ * shift from the device means mean[0..1]).  mpart as pll_launch_rk2; body (p
+ * NULL only) as pll_launch_rk1. */
+int pll_launch_rk12(const pll_grid_dev *g, const double *const q[3], double *const o[3],
+                    const double *p, double *mpart, int fmask, double vfu, double vfv,
+                    const double *mean, const double *const *body, hipStream_t s);
 int pll_launch_calc_rhs(const pll_grid_dev *g, const double *u, const double *v,
                         const double *w, double *p, hipStream_t s);
-/* mean non-NULL and fmask != 0: then also q += vel_force - mean[d] for the
- * forced components (bit 0 u with vfu, bit 1 v with vfv). */
-int pll_launch_correct_vel(const pll_grid_dev *g, const double *p, double *u,
-                           double *v, double *w, int fmask, double vfu, double vfv,
+/* (u, v, w) := q corrected, q = the same arrays or others; mean non-NULL and
+ * fmask != 0: then also += vel_force - mean[d] for the forced components
+ * (bit 0 u with vfu, bit 1 v with vfv). */
+int pll_launch_correct_vel(const pll_grid_dev *g, const double *p, const double *const q[3],
+                           double *u, double *v, double *w, int fmask, double vfu, double vfv,
                            const double *mean, hipStream_t s);
 /* partial sums of q*dzflzi per (j,k) row into part[ny*nz]; then a single
  * workgroup reduces them to out[0] = sum / nx / ny (Mean_h). */

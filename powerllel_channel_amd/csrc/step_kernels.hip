@@ -72,32 +72,7 @@ struct Body {
 
 __device__ __forceinline__ int wrap(int i, int n) { return i == 0 ? n : (i == n + 1 ? 1 : i); }
 
-// CORR (RK1 of a multi-step run): the velocity q is the previous step's RK2
-// output after its boundary fill, not yet projected.  Every value the
-// stencil reads is formed on load as correctVel (with the forcing shift) and
-// updateBoundVel would have left it, in the same roundings (k_correct,
-// k_bc_vel), from q and the pressure p with its ghosts; the projected
-// interior values are also written to (nu, nv, nw).
-struct Corr {
-    const double *p;
-    double *nu, *nv, *nw;
-    double dtdxi, dtdyi;
-    int fmask;
-    double vfu, vfv;
-    const double *mean;
-};
-
-// The projecting RK1 (CORR) uses tiles of 64 x 8 columns: its pressure tiles
-// add to the halo, so taller tiles pay (768x384x256: 4.60 -> 4.47 ms per step),
-// while the other RK kernels are faster with 64 x 4 (4.74 vs 4.82 ms).
-constexpr int RK_TY_CORR = 8;
 constexpr int LTX = RK_TX + 2;
-// CORR: pressure tiles one cell wider on the high x and y sides (p(i+1),
-// p(j+1) of every velocity tile cell)
-constexpr int PTX = LTX + 1;
-
-// periodic index of a pressure tile cell: 0 -> n, n + 1 -> 1, n + 2 -> 2
-__device__ __forceinline__ int wrap_p(int i, int n) { return i == 0 ? n : (i > n ? i - n : i); }
 
 // FILL: q's boundary fill has not been made; the values it would leave
 // (k_bc_vel) are read from the interior instead of the ghost cells.
@@ -110,28 +85,20 @@ __device__ __forceinline__ int wrap_p(int i, int n) { return i == 0 ? n : (i > n
 // values of plane k are loaded before the prefetch of plane k+2, so that
 // waiting for them leaves the prefetch in flight.
 // Occupancy hints: the FULL RK1 kernels at 4 waves per SIMD; the general RK2
-// kernels without a body force at 5 (96 VGPRs, no spills: the forced RK2 of
-// pll_channel_run had 100 and 4 waves; step 4.365 -> 4.350 ms at 768x384x256);
-// the PROJO RK2 at 4 (at 5 it spills).
-// PROJO (RK2 of a multi-step run): o is the previous step's RK2 output, not
-// yet projected; its projected value at the cell (correctVel with the forcing
-// shift, and w = 0 on the top interior row as updateBoundVel leaves it) is
-// formed as it is read, from o and p, in the roundings of the projecting RK1,
-// so that RK1 need not write the projected field.
-template <bool SECOND, bool MEAN, bool BODY, bool CORR = false, int TY = RK_TY, bool FILL = false,
-          bool FULL = false, bool PROJO = false>
-__global__ void __launch_bounds__(RK_TX *TY, ((FULL && !SECOND) || PROJO ? 4 : (SECOND && !FULL && !BODY ? 5 : 1))) k_rk(G g, Tiles t, const double *__restrict__ qu,
+// kernels without a body force at 5 (96 VGPRs, no spills: 100 and 4 waves
+// without it; step 4.365 -> 4.350 ms at 768x384x256).
+template <bool SECOND, bool MEAN, bool BODY, bool FILL, bool FULL>
+__global__ void __launch_bounds__(RK_TX *RK_TY, (FULL && !SECOND ? 4 : (SECOND && !FULL && !BODY ? 5 : 1))) k_rk(G g, Tiles t, const double *__restrict__ qu,
                                                      const double *__restrict__ qv,
                                                      const double *__restrict__ qw,
                                                      double *__restrict__ ou,
                                                      double *__restrict__ ov,
                                                      double *__restrict__ ow,
                                                      double *__restrict__ mpart, int fmask,
-                                                     Body fb, Corr cr = Corr{})
+                                                     Body fb)
 {
-    constexpr int LTY = TY + 2, LPL = LTX * LTY, NT = RK_TX * TY;
+    constexpr int TY = RK_TY, LTY = TY + 2, LPL = LTX * LTY, NT = RK_TX * TY;
     constexpr int NLD = (LPL + NT - 1) / NT;
-    constexpr int PTY = LTY + 1, LPP = PTX * PTY, NLP = (LPP + NT - 1) / NT;
     __shared__ double tl[2][3][LPL];
     int tx, ty, kc;
     rk_tile(t, tx, ty, kc);
@@ -157,73 +124,12 @@ __global__ void __launch_bounds__(RK_TX *TY, ((FULL && !SECOND) || PROJO ? 4 : (
         gii[r] = gk[r] ? wrap(gi, g.nx) : 1;
         gjj[r] = gk[r] ? wrap(gj, g.ny) : 1;
     }
-    // CORR: projected value of field f at interior (i, j, k), as k_correct
-    const double shu = ((CORR || PROJO) && (cr.fmask & 1)) ? cr.vfu - cr.mean[0] : 0.0;
-    const double shv = ((CORR || PROJO) && (cr.fmask & 2)) ? cr.vfv - cr.mean[1] : 0.0;
-    auto proj = [&](int f, int ii, int jj, int kk) -> double {
-        const long long e0 = ii + sy * jj + sz * kk;
-        const double pc = cr.p[e0];
-        if (f == 0) {
-            double un = qu[e0] - (cr.p[e0 + 1] - pc) * cr.dtdxi;
-            if (cr.fmask & 1) un = un + shu;
-            return un;
-        }
-        if (f == 1) {
-            double vn = qv[e0] - (cr.p[e0 + sy] - pc) * cr.dtdyi;
-            if (cr.fmask & 2) vn = vn + shv;
-            return vn;
-        }
-        return qw[e0] - (cr.p[e0 + sz] - pc) * g.dt * g.dzc_inv[kk];
-    };
-    // ... and as k_bc_vel then leaves it at haloed (gi, gj, kk) (ii, jj wrapped)
-    auto filled = [&](int f, int ii, int jj, int kk) -> double {
-        if (kk == 0 || kk == g.nz + 1) {
-            if (f == 2) return 0.0;
-            const double bc = f == 0 ? 0.0 - g.u_crf : 0.0;
-            return 2.0 * bc - proj(f, ii, jj, kk == 0 ? 1 : g.nz);
-        }
-        if (f == 2 && kk == g.nz) return 0.0;
-        return proj(f, ii, jj, kk);
-    };
     double pre[3][NLD];
-    // CORR: the plane's raw velocity (at the wrapped source cells) is loaded
-    // ahead like pre; the pressure goes through two LDS tiles, p of the source
-    // plane and of the plane above (w's projection), the latter loaded ahead
-    // into pnext; the projection is formed when the plane is written to LDS
-    __shared__ double tp[CORR ? 2 : 1][CORR ? LPP : 1];
-    long long gpo[NLP];
-    bool gpk[NLP];
-    double pnext[NLP];
-    int kpre = 0, pcur = 0;
-    if (CORR) {
-#pragma unroll
-        for (int r = 0; r < NLP; ++r) {
-            const int q = FULL ? min(tid + r * NT, LPP - 1) : tid + r * NT;
-            const int row = q / PTX, col = q - row * PTX;
-            const int gi = i0 + col, gj = j0 + row;
-            gpk[r] = FULL || (q < LPP && gi <= g.nx + 2 && gj <= g.ny + 2);
-            gpo[r] = gpk[r] ? wrap_p(gi, g.nx) + sy * wrap_p(gj, g.ny) : 0;
-            // p of the chunk's first plane, for its first projection
-            if (FULL || q < LPP) tp[0][q] = gpk[r] ? cr.p[gpo[r] + sz * k0] : 0.0;
-        }
-    }
+    int kpre = 0;
     // interior: 1 <= kp <= nz - 1 is known (no wall rule applies to the plane)
     auto fetch = [&](int kp, bool interior = false) {
         kpre = kp;
-        if (CORR) {
-            const int ks = interior ? kp : (kp == 0 ? 1 : (kp == g.nz + 1 ? g.nz : kp));
-            const bool above = interior || (kp >= 1 && kp <= g.nz - 1);
-#pragma unroll
-            for (int r = 0; r < NLD; ++r) {
-                const long long e0 = gii[r] + sy * gjj[r] + sz * ks;
-                pre[0][r] = gk[r] ? qu[e0] : 0.0;
-                pre[1][r] = gk[r] ? qv[e0] : 0.0;
-                pre[2][r] = gk[r] ? qw[e0] : 0.0;
-            }
-#pragma unroll
-            for (int r = 0; r < NLP; ++r)
-                pnext[r] = (above && gpk[r]) ? cr.p[gpo[r] + sz * (kp + 1)] : 0.0;
-        } else if (FILL) {
+        if (FILL) {
             const int ks = kp == 0 ? 1 : (kp == g.nz + 1 ? g.nz : kp);
 #pragma unroll
             for (int f = 0; f < 3; ++f)
@@ -240,49 +146,7 @@ __global__ void __launch_bounds__(RK_TX *TY, ((FULL && !SECOND) || PROJO ? 4 : (
     // interior: the plane put lies strictly inside (1 <= kp <= nz - 1), so no
     // wall rule of the fill applies (the FULL loop's planes but the last two)
     auto put = [&](int b, bool interior = false) {
-        if (CORR) {
-            // projection (k_correct) of the plane's source values, then the
-            // fill (k_bc_vel) for the wall planes and w's wall row.  tp[pcur]
-            // holds p of the source plane ks; p of the plane above goes to the
-            // other tile and becomes the source plane's p for the next put
-            const int kp = kpre;
-            const int ks = interior ? kp : (kp == 0 ? 1 : (kp == g.nz + 1 ? g.nz : kp));
-            const bool wall = !interior && (kp == 0 || kp == g.nz + 1);
-            const bool above = interior || (kp >= 1 && kp <= g.nz - 1);
-            const double dzi = pll::zm(g.dzc_inv, ks), bcu = 0.0 - g.u_crf;
-            if (above) {
-#pragma unroll
-                for (int r = 0; r < NLP; ++r) {
-                    const int q = FULL ? min(tid + r * NT, LPP - 1) : tid + r * NT;
-                    if (FULL || q < LPP) tp[pcur ^ 1][q] = pnext[r];
-                }
-            }
-            __syncthreads();
-            const double *Pc = tp[pcur], *Pn = tp[pcur ^ 1];
-#pragma unroll
-            for (int r = 0; r < NLD; ++r) {
-                const int q = tid + r * NT;
-                const int row = q / LTX, col = q - row * LTX;
-                const int o = q < LPL ? row * PTX + col : 0;
-                const double pc = Pc[o];
-                double un = pre[0][r] - (Pc[o + 1] - pc) * cr.dtdxi;
-                if (cr.fmask & 1) un = un + shu;
-                double vn = pre[1][r] - (Pc[o + PTX] - pc) * cr.dtdyi;
-                if (cr.fmask & 2) vn = vn + shv;
-                double wn = above ? pre[2][r] - (Pn[o] - pc) * g.dt * dzi : 0.0;
-                if (wall) {
-                    un = 2.0 * bcu - un;
-                    vn = 2.0 * 0.0 - vn;
-                    wn = 0.0;
-                } else if (!interior && kp == g.nz) {
-                    wn = 0.0;
-                }
-                pre[0][r] = un;
-                pre[1][r] = vn;
-                pre[2][r] = wn;
-            }
-            if (above) pcur ^= 1;
-        } else if (FILL && !interior) {
+        if (FILL && !interior) {
             const int kp = kpre;
             if (kp == 0 || kp == g.nz + 1) {
                 const double bcu = 0.0 - g.u_crf;
@@ -307,7 +171,6 @@ __global__ void __launch_bounds__(RK_TX *TY, ((FULL && !SECOND) || PROJO ? 4 : (
     };
     fetch(k0);
     put(0);
-    if (CORR) __syncthreads();  // put(0)'s pressure reads are done before put(1) writes a tile
     fetch(k0 + 1);
     put(1);
     long long e = i + sy * j + sz * k0;
@@ -329,12 +192,6 @@ __global__ void __launch_bounds__(RK_TX *TY, ((FULL && !SECOND) || PROJO ? 4 : (
             w00m = fq(qw, 2, i, j);
             wp0m = fq(qw, 2, wrap(i + 1, g.nx), j);
             w0pm = fq(qw, 2, i, wrap(j + 1, g.ny));
-        } else if (CORR) {
-            u00m = filled(0, i, j, k0 - 1);
-            v00m = filled(1, i, j, k0 - 1);
-            w00m = filled(2, i, j, k0 - 1);
-            wp0m = filled(2, wrap(i + 1, g.nx), j, k0 - 1);
-            w0pm = filled(2, i, wrap(j + 1, g.ny), k0 - 1);
         } else {
             u00m = qu[e - sz];
             v00m = qv[e - sz];
@@ -372,20 +229,8 @@ __global__ void __launch_bounds__(RK_TX *TY, ((FULL && !SECOND) || PROJO ? 4 : (
             fw = fw + fb.w[ek];
         }
         if (SECOND) {
-            double ou0, ov0, ow0;
-            if constexpr (PROJO) {
-                // the expressions of proj() on o
-                const double pc = cr.p[ek];
-                ou0 = ou[ek] - (cr.p[ek + 1] - pc) * cr.dtdxi;
-                if (cr.fmask & 1) ou0 = ou0 + shu;
-                ov0 = ov[ek] - (cr.p[ek + sy] - pc) * cr.dtdyi;
-                if (cr.fmask & 2) ov0 = ov0 + shv;
-                ow0 = k == g.nz ? 0.0 : ow[ek] - (cr.p[ek + sz] - pc) * g.dt * g.dzc_inv[k];
-            } else {
-                ou0 = old ? old[0] : ou[ek];
-                ov0 = old ? old[1] : ov[ek];
-                ow0 = old ? old[2] : ow[ek];
-            }
+            const double ou0 = old ? old[0] : ou[ek], ov0 = old ? old[1] : ov[ek],
+                         ow0 = old ? old[2] : ow[ek];
             const double un = (n.u000 + g.dt * fu + ou0) * 0.5;
             const double vn = (n.v000 + g.dt * fv + ov0) * 0.5;
             ou[ek] = un;
@@ -402,11 +247,6 @@ __global__ void __launch_bounds__(RK_TX *TY, ((FULL && !SECOND) || PROJO ? 4 : (
             ou[ek] = n.u000 + g.dt * fu;
             ov[ek] = n.v000 + g.dt * fv;
             ow[ek] = n.w000 + g.dt * fw;
-            if (CORR && cr.nu) {
-                cr.nu[ek] = n.u000;
-                cr.nv[ek] = n.v000;
-                cr.nw[ek] = n.w000;
-            }
         }
         u00m = n.u000;
         v00m = n.v000;
@@ -482,13 +322,13 @@ __global__ void __launch_bounds__(RK_TX *TY, ((FULL && !SECOND) || PROJO ? 4 : (
 // next step's p(k)).  FORCE: then forceVel's shift q += vel_force - mean for
 // the components in fmask (bit 0 u, bit 1 v), with the means in mean[0..1],
 // in the same two roundings as correctVel followed by forceVel.
+// Reads (qu, qv, qw) and writes (u, v, w), which may be the same arrays.
 template <bool FORCE>
 __global__ void __launch_bounds__(RK_TX *RK_TY) k_correct(G g, Tiles t, const double *__restrict__ p,
-                                                          double *__restrict__ u,
-                                                          double *__restrict__ v,
-                                                          double *__restrict__ w, double dtdxi,
-                                                          double dtdyi, int fmask, double vfu,
-                                                          double vfv,
+                                                          const double *qu, const double *qv,
+                                                          const double *qw, double *u, double *v,
+                                                          double *w, double dtdxi, double dtdyi,
+                                                          int fmask, double vfu, double vfv,
                                                           const double *__restrict__ mean)
 {
     int tx, ty, kc;
@@ -507,13 +347,14 @@ __global__ void __launch_bounds__(RK_TX *RK_TY) k_correct(G g, Tiles t, const do
     double pc = p[e];
     for (int k = k0; k <= k1; ++k, e += sz) {
         const double pz = p[e + sz];
-        double un = u[e] - (p[e + 1] - pc) * dtdxi;
-        double vn = v[e] - (p[e + sy] - pc) * dtdyi;
+        double un = qu[e] - (p[e + 1] - pc) * dtdxi;
+        double vn = qv[e] - (p[e + sy] - pc) * dtdyi;
+        const double wn = qw[e] - (pz - pc) * g.dt * g.dzc_inv[k];
         if (FORCE && (fmask & 1)) un = un + fu;
         if (FORCE && (fmask & 2)) vn = vn + fv;
         u[e] = un;
         v[e] = vn;
-        w[e] = w[e] - (pz - pc) * g.dt * g.dzc_inv[k];
+        w[e] = wn;
         pc = pz;
     }
 }
@@ -836,6 +677,16 @@ Tiles rk_tiles(const G &g, int ty = RK_TY)
 
 }  // namespace
 
+extern "C" void pll_rk_tiling(const pll_grid_dev *gd, int rk[5])
+{
+    const Tiles t = rk_tiles(make_g(gd));
+    rk[0] = t.ntx;
+    rk[1] = t.nty;
+    rk[2] = t.nkc;
+    rk[3] = t.kc;
+    rk[4] = t.xcd;
+}
+
 extern "C" int pll_rk_blocks(const pll_grid_dev *gd)
 {
     const Tiles t = rk_tiles(make_g(gd));
@@ -855,9 +706,8 @@ int with_flags(bool a, bool b, bool c, F &&f)
     return -1;
 }
 
-// Grids whose RK tiles all lie inside take the FULL kernels for RK1 and the
-// projecting RK1 (768x384x256, same-process A/B: projecting RK1 1.698 ->
-// 1.542 ms, RK1 unchanged); RK2's FULL form needs 145 VGPRs (3 waves per SIMD
+// Grids whose RK tiles all lie inside take the FULL kernel for RK1
+// (768x384x256: 0.94 ms either way); RK2's FULL form needs 145 VGPRs (3 waves per SIMD
 // against 4) and runs 1.314 ms against 1.304, so RK2 keeps the general form
 // unless PLL_RK2_FULL=1.  PLL_RK_FULL=0 takes the general kernels everywhere.
 // (read at every launch, so that one process can time both forms)
@@ -878,41 +728,10 @@ extern "C" int pll_launch_rk1(const pll_grid_dev *gd, const double *u, const dou
     const dim3 grid((unsigned)(t.ntx * t.nty * t.nkc)), blk(RK_TX * RK_TY);
     const Body fb = body ? Body{body[0], body[1], body[2]} : Body{nullptr, nullptr, nullptr};
     return with_flags(false, body != nullptr, full_tiles(g, RK_TY), [&](auto, auto B, auto F) {
-        hipLaunchKernelGGL((k_rk<false, false, decltype(B)::value, false, RK_TY, false,
-                                 decltype(F)::value>),
-                           grid, blk, 0, s, g, t, u, v, w, u1, v1, w1, nullptr, 0, fb, Corr{});
+        hipLaunchKernelGGL((k_rk<false, false, decltype(B)::value, false, decltype(F)::value>),
+                           grid, blk, 0, s, g, t, u, v, w, u1, v1, w1, nullptr, 0, fb);
         return ok();
     });
-}
-
-extern "C" int pll_launch_rk1_corr(const pll_grid_dev *gd, const double *u, const double *v,
-                                   const double *w, const double *p, double *nu, double *nv,
-                                   double *nw, double *u1, double *v1, double *w1, int fmask,
-                                   double vfu, double vfv, const double *mean, hipStream_t s)
-{
-    const G g = make_g(gd);
-    const Tiles t = rk_tiles(g, RK_TY_CORR);
-    const dim3 grid((unsigned)(t.ntx * t.nty * t.nkc)), blk(RK_TX * RK_TY_CORR);
-    Corr cr;
-    cr.p = p;
-    cr.nu = nu;
-    cr.nv = nv;
-    cr.nw = nw;
-    cr.dtdxi = g.dt * g.dx_inv;  // as pll_launch_correct_vel
-    cr.dtdyi = g.dt * g.dy_inv;
-    cr.fmask = mean ? fmask : 0;
-    cr.vfu = vfu;
-    cr.vfv = vfv;
-    cr.mean = mean;
-    if (full_tiles(g, RK_TY_CORR))
-        hipLaunchKernelGGL((k_rk<false, false, false, true, RK_TY_CORR, false, true>), grid, blk, 0,
-                           s, g, t, u, v, w, u1, v1, w1, nullptr, 0,
-                           Body{nullptr, nullptr, nullptr}, cr);
-    else
-        hipLaunchKernelGGL((k_rk<false, false, false, true, RK_TY_CORR, false, false>), grid, blk,
-                           0, s, g, t, u, v, w, u1, v1, w1, nullptr, 0,
-                           Body{nullptr, nullptr, nullptr}, cr);
-    return ok();
 }
 
 extern "C" int pll_launch_rk2(const pll_grid_dev *gd, double *u, double *v, double *w,
@@ -927,48 +746,15 @@ extern "C" int pll_launch_rk2(const pll_grid_dev *gd, double *u, double *v, doub
     const bool mean = mpart && fmask;
     return with_flags(mean, body != nullptr, fill != 0, [&](auto M, auto B, auto F) {
         if (full_tiles(g, RK_TY, true))
-            hipLaunchKernelGGL((k_rk<true, decltype(M)::value, decltype(B)::value, false, RK_TY,
-                                     decltype(F)::value, true>),
+            hipLaunchKernelGGL((k_rk<true, decltype(M)::value, decltype(B)::value, decltype(F)::value, true>),
                                grid, blk, 0, s, g, t, u1, v1, w1, u, v, w, mean ? mpart : nullptr,
-                               mean ? fmask : 0, fb, Corr{});
+                               mean ? fmask : 0, fb);
         else
-            hipLaunchKernelGGL((k_rk<true, decltype(M)::value, decltype(B)::value, false, RK_TY,
-                                     decltype(F)::value, false>),
+            hipLaunchKernelGGL((k_rk<true, decltype(M)::value, decltype(B)::value, decltype(F)::value, false>),
                                grid, blk, 0, s, g, t, u1, v1, w1, u, v, w, mean ? mpart : nullptr,
-                               mean ? fmask : 0, fb, Corr{});
+                               mean ? fmask : 0, fb);
         return ok();
     });
-}
-
-// RK2 of a multi-step run, in place: o = (u, v, w) is the previous step's
-// unprojected RK2 output, projected at each cell as it is read (PROJO), and
-// is overwritten with the new velocity; q = the RK1 stage; the boundary values
-// of the RK1 stage are read from its interior (FILL).
-extern "C" int pll_launch_rk2_proj(const pll_grid_dev *gd, double *u, double *v, double *w,
-                                   const double *u1, const double *v1, const double *w1,
-                                   const double *p, double *mpart, int fmask, double vfu,
-                                   double vfv, const double *mean, hipStream_t s)
-{
-    const G g = make_g(gd);
-    const Tiles t = rk_tiles(g);
-    const dim3 grid((unsigned)(t.ntx * t.nty * t.nkc)), blk(RK_TX * RK_TY);
-    Corr cr;
-    cr.p = p;
-    cr.nu = cr.nv = cr.nw = nullptr;
-    cr.dtdxi = g.dt * g.dx_inv;  // as pll_launch_correct_vel
-    cr.dtdyi = g.dt * g.dy_inv;
-    cr.fmask = mean ? fmask : 0;
-    cr.vfu = vfu;
-    cr.vfv = vfv;
-    cr.mean = mean;
-    const Body fb{nullptr, nullptr, nullptr};
-    if (mpart && fmask)
-        hipLaunchKernelGGL((k_rk<true, true, false, false, RK_TY, true, false, true>), grid, blk, 0,
-                           s, g, t, u1, v1, w1, u, v, w, mpart, fmask, fb, cr);
-    else
-        hipLaunchKernelGGL((k_rk<true, false, false, false, RK_TY, true, false, true>), grid, blk,
-                           0, s, g, t, u1, v1, w1, u, v, w, nullptr, 0, fb, cr);
-    return ok();
 }
 
 extern "C" int pll_launch_calc_rhs(const pll_grid_dev *gd, const double *u, const double *v,
@@ -982,8 +768,9 @@ extern "C" int pll_launch_calc_rhs(const pll_grid_dev *gd, const double *u, cons
     return ok();
 }
 
-extern "C" int pll_launch_correct_vel(const pll_grid_dev *gd, const double *p, double *u,
-                                      double *v, double *w, int fmask, double vfu, double vfv,
+extern "C" int pll_launch_correct_vel(const pll_grid_dev *gd, const double *p,
+                                      const double *const q[3], double *u, double *v,
+                                      double *w, int fmask, double vfu, double vfv,
                                       const double *mean, hipStream_t s)
 {
     const G g = make_g(gd);
@@ -993,7 +780,7 @@ extern "C" int pll_launch_correct_vel(const pll_grid_dev *gd, const double *p, d
     const bool force = mean && fmask;
     return with_flags(force, false, false, [&](auto Fo, auto, auto) {
         hipLaunchKernelGGL(k_correct<decltype(Fo)::value>, grid, dim3(RK_TX * RK_TY), 0, s, g, t, p,
-                           u, v, w, dtdxi, dtdyi, force ? fmask : 0, vfu, vfv,
+                           q[0], q[1], q[2], u, v, w, dtdxi, dtdyi, force ? fmask : 0, vfu, vfv,
                            force ? mean : nullptr);
         return ok();
     });

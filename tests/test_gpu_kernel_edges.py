@@ -39,3 +39,35 @@ def test_stencil_chunks_bitwise(orc, cuda, shape):
     torch.cuda.synchronize()
     for a, b in zip(d[:6], (u, v, w, u1, v1, w1)):
         assert np.array_equal(a.cpu().numpy(), b)
+
+
+# RK1 + RK2 in one pass (64 x 12 tiles): tiles cut by the grid's edge in x and
+# y, grids narrower than the halo, k chunks of one plane and more with short
+# ends, few planes
+@pytest.mark.parametrize("shape,forced,u_crf,n", [
+    ((4, 4, 2), (True, False, False), 0.0, 3),
+    ((10, 6, 3), (True, True, False), 0.3, 4),
+    ((66, 26, 17), (False, False, False), 0.2, 3),
+    ((128, 24, 65), (True, False, False), 0.0, 2),
+    ((256, 256, 34), (True, False, False), 0.1, 3),
+    ((200, 140, 29), (False, True, False), 0.0, 4)])
+def test_run_equals_steps_edges(orc, cuda, shape, forced, u_crf, n):
+    """pll_channel_run against as many calls of pll_channel_step, bit for bit
+    (u, v, w with their ghosts and the pressure)."""
+    import torch
+    from powerllel_channel_amd import PoissonSolver
+    nx, ny, nz = shape
+    print(f"[run = steps] {shape} forced={forced} u_crf={u_crf} n={n}", flush=True)
+    g, G, ch, (u, v, w, *_) = _channel(orc, nx, ny, nz, u_crf=u_crf, is_forced=forced,
+                                       vel_force=(1.0, 0.2, 0.0), dt=1e-4)
+    orc.bc_vel(G, u, v, w, u_crf)
+    z = np.zeros(g.shape)
+    s = PoissonSolver(nx, ny, nz, g.dx, g.dy, g.dzf)
+    a, b = _dev(torch, cuda, u, v, w, z, z, z, z), _dev(torch, cuda, u, v, w, z, z, z, z)
+    ch.run(s, n, *a)
+    for _ in range(n):
+        ch.step(s, *b)
+    torch.cuda.synchronize()
+    for q in (0, 1, 2, 6):
+        assert torch.isfinite(b[q]).all()
+        assert torch.equal(a[q], b[q]), q
