@@ -71,3 +71,37 @@ def test_run_equals_steps_edges(orc, cuda, shape, forced, u_crf, n):
     for q in (0, 1, 2, 6):
         assert torch.isfinite(b[q]).all()
         assert torch.equal(a[q], b[q]), q
+
+
+# 64 x 4 tiles over the haloed box: sizes that fill them exactly (62 + 2 by
+# 2 + 2), exceed them by one cell, and leave short k chunks
+@pytest.mark.parametrize("shape", [(62, 2, 5), (63, 3, 4), (64, 6, 37), (130, 23, 16), (3, 2, 2)])
+def test_rk_vjp_transposes_jvp(cuda, shape):
+    """<J dq, l> = <dq, J^T l> over the haloed arrays (l on the interior), and
+    the alpha, a0, beta combination.  Both sums have positive and negative
+    terms of size ~1; 1e-12 of the sum of their magnitudes."""
+    import torch
+    from powerllel_channel_amd import Channel
+    from powerllel_channel_amd.mesh import Grid
+    nx, ny, nz = shape
+    print(f"[rk vjp] {shape}", flush=True)
+    g = Grid(nx, ny, nz, 0.1 * nx, 0.1 * ny, 2.0, 2.0)
+    ch = Channel(nx, ny, nz, g.lx, g.ly, g.lz, g.dzf, 1e-2, 1e-3, u_crf=0.3)
+    gen = torch.Generator().manual_seed(3)
+    q, d, lam, x = [[torch.randn(g.shape, generator=gen, dtype=torch.float64).to(cuda)
+                     for _ in range(3)] for _ in range(4)]
+    jd = [torch.zeros_like(t) for t in q]
+    ch.rk_jvp(q, d, jd)
+    o = [t.clone() for t in x]
+    ch.rk_vjp(q, lam, o, 1.0, 0.0, 0.0)
+    inner = (slice(1, -1),) * 3
+    lhs = sum(float((a[inner] * b[inner]).sum()) for a, b in zip(jd, lam))
+    rhs = sum(float((a * b).sum()) for a, b in zip(d, o))
+    mag = sum(float((a * b).abs().sum()) for a, b in zip(d, o))
+    assert abs(lhs - rhs) <= 1e-12 * mag
+    c = [t.clone() for t in x]
+    ch.rk_vjp(q, lam, c, 0.25, 1.5, -0.5)
+    for a, b, l, y in zip(c, o, lam, x):
+        want = 0.25 * b - 0.5 * y
+        want[inner] += 1.5 * l[inner]
+        assert float((a - want).abs().max()) <= 1e-14 * float(b.abs().max() + y.abs().max() + 2.0)
