@@ -31,7 +31,8 @@ struct pll_adjoint {
     double *ck;              /* nck checkpoints x 3 fields */
     double *seg;             /* every states x 3 fields */
     double *u1, *p;          /* 3 fields, 1 field */
-    double *lam, *lam1, *lamp, *grad, *body; /* 3, 3, 1, 3, 3 fields */
+    double *lam, *lam1, *lamp, *body; /* 3, 3, 1, 3 fields */
+    double *jpart, *tot;     /* device: partial sums of lam, the 3 sums */
     double *wsum;            /* device: 2 nsteps wall sums */
     double *part;            /* device: partials for the wall sums */
     double *hsum;            /* host: 2 nsteps */
@@ -55,8 +56,8 @@ static int launch(int rc, const char *what)
 int pll_adjoint_destroy(pll_adjoint *a)
 {
     if (!a) return PLL_OK;
-    void *bufs[] = {a->ck, a->seg, a->u1, a->p, a->lam, a->lam1, a->lamp, a->grad, a->body,
-                    a->wsum, a->part};
+    void *bufs[] = {a->ck, a->seg, a->u1, a->p, a->lam, a->lam1, a->lamp, a->body,
+                    a->wsum, a->part, a->jpart, a->tot};
     for (size_t i = 0; i < sizeof bufs / sizeof bufs[0]; i++)
         if (bufs[i]) hipFree(bufs[i]);
     free(a->hsum);
@@ -101,7 +102,9 @@ int pll_adjoint_create(pll_adjoint **out, pll_channel *ch, pll_ppe *ppe, int nst
         (rc = dalloc(a, &a->seg, 3 * a->fbytes * (size_t)a->every)) ||
         (rc = dalloc(a, &a->u1, 3 * a->fbytes)) || (rc = dalloc(a, &a->p, a->fbytes)) ||
         (rc = dalloc(a, &a->lam, 3 * a->fbytes)) || (rc = dalloc(a, &a->lam1, 3 * a->fbytes)) ||
-        (rc = dalloc(a, &a->lamp, a->fbytes)) || (rc = dalloc(a, &a->grad, 3 * a->fbytes)) ||
+        (rc = dalloc(a, &a->lamp, a->fbytes)) ||
+        (rc = dalloc(a, &a->jpart, sizeof(double) * 3 * (size_t)pll_jtv_fold_blocks(g))) ||
+        (rc = dalloc(a, &a->tot, sizeof(double) * 3)) ||
         (rc = dalloc(a, &a->body, 3 * a->fbytes)) ||
         (rc = dalloc(a, &a->wsum, sizeof(double) * 2 * (size_t)nsteps)) ||
         (rc = dalloc(a, &a->part, sizeof(double) * 2 * (size_t)g->ny))) {
@@ -186,55 +189,62 @@ int pll_adjoint_forward(pll_adjoint *a, const double *u0, const double *v0, cons
 
 /* dJ/du on the wall planes for one state: (1/nsteps) * 1/2 * re_inv /
  * (nx ny dzf(kw)/2) */
-static int seed(pll_adjoint *a, hipStream_t s)
+static void seed(const pll_adjoint *a, double *cb, double *ct)
 {
     const pll_grid_dev *g = pll_channel_grid(a->ch);
     const double *dzf = pll_channel_dzf_host(a->ch);
     const double nxy = (double)g->nx * g->ny;
-    const double cb = g->re_inv / (a->nsteps * nxy * dzf[1]);
-    const double ct = g->re_inv / (a->nsteps * nxy * dzf[g->nz]);
-    return launch(pll_launch_wall_seed(g, fld(a, a->lam, 0), cb, ct, s), "wall seed");
+    *cb = g->re_inv / (a->nsteps * nxy * dzf[1]);
+    *ct = g->re_inv / (a->nsteps * nxy * dzf[g->nz]);
 }
 
-/* lam (adjoint of the state after step n) -> adjoint of the state before it;
- * U is that state, its RK1 stage is recomputed into u1. */
-static int step_adj(pll_adjoint *a, double *U, hipStream_t s)
+/* lam (adjoint of the state U_{n+1}, folded) -> adjoint of the state U_n
+ * with J's reading of U_n added; U is U_n, its RK1 stage is recomputed into
+ * u1.  Every adjoint field lives on the interior: the transposed boundary
+ * fills are part of the passes on either side of them.
+ *   lamp = transposed correctVel of lam, solved
+ *   lam* = lam (forcing transposed) + transposed calcRHS of lamp
+ *   RK2, u* = (u1 + dt (f(u1) + b) + u) / 2:  l1 = lam* / 2 + dt/2 J(u1)^T lam*
+ *   RK1, u1 = u + dt (f(u) + b):  lam = lam* / 2 + l1 + dt J(u)^T l1 + dJ/dU_n
+ *   grad += dt/2 lam* + dt l1
+ * The sums of the new lam (for its transposed forcing) come out of the last
+ * pass; fmask 0: lam has had its forcing transposed already.  last: the
+ * adjoint of U_n is not wanted. */
+static int step_adj(pll_adjoint *a, const double *U, double *const Gr[3], int fmask, int last,
+                    hipStream_t s)
 {
     pll_channel *ch = a->ch;
     const pll_grid_dev *g = pll_channel_grid(ch);
+    const size_t nf = a->fbytes / sizeof(double);
     double *L[3] = {fld(a, a->lam, 0), fld(a, a->lam, 1), fld(a, a->lam, 2)};
     double *L1[3] = {fld(a, a->lam1, 0), fld(a, a->lam1, 1), fld(a, a->lam1, 2)};
-    double *Gr[3] = {fld(a, a->grad, 0), fld(a, a->grad, 1), fld(a, a->grad, 2)};
-    const double *Uc[3] = {fld(a, U, 0), fld(a, U, 1), fld(a, U, 2)};
+    const double *Lc[3] = {L[0], L[1], L[2]}, *L1c[3] = {L1[0], L1[1], L1[2]};
+    const double *Uc[3] = {U, U + nf, U + 2 * nf};
     double *U1[3] = {fld(a, a->u1, 0), fld(a, a->u1, 1), fld(a, a->u1, 2)};
-    const double *B[3] = {fld(a, a->body, 0), fld(a, a->body, 1), fld(a, a->body, 2)};
-    int rc;
-    /* stage recomputation: u1 = RK1(u) with its boundary fill */
-    if ((rc = launch(pll_launch_rk1(g, Uc[0], Uc[1], Uc[2], U1[0], U1[1], U1[2], B, s),
-                     "rk1")))
-        return rc;
-    if ((rc = pll_channel_bc_vel(ch, U1[0], U1[1], U1[2], s))) return rc;
-    /* final boundary fill, forcing, correctVel (velocity part is the identity) */
-    if ((rc = pll_channel_bc_vel_adj(ch, L[0], L[1], L[2], s))) return rc;
-    if ((rc = pll_channel_force_vel_adj(ch, L[0], L[1], L[2], s))) return rc;
-    if ((rc = pll_channel_correct_vel_adj(ch, L[0], L[1], L[2], a->lamp, s))) return rc;
-    if ((rc = pll_channel_bc_p_adj(ch, a->lamp, s))) return rc;
-    if ((rc = pll_ppe_solve_adjoint(a->ppe, a->lamp, s))) return rc;
-    if ((rc = pll_channel_calc_rhs_adj(ch, a->lamp, L[0], L[1], L[2], s))) return rc;
-    if ((rc = pll_channel_bc_vel_adj(ch, L[0], L[1], L[2], s))) return rc;
-    /* RK2: u* = (u1 + dt (f(u1) + b) + u) / 2 */
-    if ((rc = launch(pll_launch_axpy3(g, 0.5 * g->dt, (const double *const *)L, Gr, s), "axpy")))
-        return rc;
     const double *U1c[3] = {U1[0], U1[1], U1[2]};
-    const double *Lc[3] = {L[0], L[1], L[2]};
-    if ((rc = launch(pll_launch_jtv(g, U1c, Lc, L1, 0.5 * g->dt, 0.5, 0.0, s), "rk2 adjoint")))
+    const double *B[3] = {fld(a, a->body, 0), fld(a, a->body, 1), fld(a, a->body, 2)};
+    const double h = 0.5 * g->dt;
+    double cb, ct;
+    int rc;
+    seed(a, &cb, &ct);
+    if ((rc = launch(pll_launch_rk1(g, Uc[0], Uc[1], Uc[2], U1[0], U1[1], U1[2], B, s), "rk1")) ||
+        (rc = launch(pll_launch_correct_adj_fold(g, Lc, a->lamp, fmask, a->tot, s),
+                     "correct_vel adjoint")) ||
+        (rc = pll_ppe_solve_adjoint(a->ppe, a->lamp, s)) ||
+        (rc = launch(pll_launch_rhs_adj_fold(g, a->lamp, L, fmask, a->tot, s),
+                     "calc_rhs adjoint")) ||
+        (rc = launch(pll_launch_jtv_fold(g, U1c, Lc, L1, NULL, h, 0.5, 0.0, NULL, 0.0, 0.0, 0.0,
+                                         0.0, NULL, s),
+                     "rk2 adjoint")))
         return rc;
-    if ((rc = pll_channel_bc_vel_adj(ch, L1[0], L1[1], L1[2], s))) return rc;
-    /* RK1: u1 = u + dt (f(u) + b) */
-    if ((rc = launch(pll_launch_axpy3(g, g->dt, (const double *const *)L1, Gr, s), "axpy")))
+    if (last) return launch(pll_launch_axpy3(g, g->dt, L1c, h, Lc, Gr, s), "gradient");
+    if ((rc = launch(pll_launch_jtv_fold(g, Uc, L1c, L, Lc, g->dt, 1.0, 0.5, Gr, g->dt, h, cb, ct,
+                                         a->jpart, s),
+                     "rk1 adjoint")))
         return rc;
-    const double *L1c[3] = {L1[0], L1[1], L1[2]};
-    return launch(pll_launch_jtv(g, Uc, L1c, L, g->dt, 1.0, 0.5, s), "rk1 adjoint");
+    return launch(pll_launch_sum3(pll_jtv_fold_blocks(g), a->jpart, a->tot,
+                                  1.0 / ((double)g->nx * g->ny), s),
+                  "forcing sums");
 }
 
 int pll_adjoint_backward(pll_adjoint *a, double *gu, double *gv, double *gw, void *stream)
@@ -243,12 +253,23 @@ int pll_adjoint_backward(pll_adjoint *a, double *gu, double *gv, double *gw, voi
     if (!a->have_forward) return pll_set_error(PLL_ESTATE, "pll_adjoint_forward not run");
     if (!gu || !gv || !gw) return pll_set_error(PLL_EINVAL, "NULL gradient field");
     hipStream_t s = (hipStream_t)stream;
-    int rc;
-    if ((rc = hipchk(hipMemsetAsync(a->grad, 0, 3 * a->fbytes, s), "clear")) ||
-        (rc = hipchk(hipMemsetAsync(a->lam, 0, 3 * a->fbytes, s), "clear")) ||
+    const pll_grid_dev *g = pll_channel_grid(a->ch);
+    double *const Gr[3] = {gu, gv, gw};
+    double *L[3] = {fld(a, a->lam, 0), fld(a, a->lam, 1), fld(a, a->lam, 2)};
+    int rc, forced[3], fmask = 0;
+    if ((rc = pll_channel_forcing(a->ch, forced, NULL))) return rc;
+    for (int d = 0; d < 3; d++) fmask |= forced[d] ? 1 << d : 0;
+    for (int d = 0; d < 3; d++)
+        if ((rc = hipchk(hipMemsetAsync(Gr[d], 0, a->fbytes, s), "clear"))) return rc;
+    if ((rc = hipchk(hipMemsetAsync(a->lam, 0, 3 * a->fbytes, s), "clear")) ||
         (rc = hipchk(hipMemsetAsync(a->lam1, 0, 3 * a->fbytes, s), "clear")))
         return rc;
-    if ((rc = seed(a, s))) return rc;  /* state after the last step */
+    /* state after the last step: J's reading of it, forcing transposed */
+    double cb, ct;
+    seed(a, &cb, &ct);
+    if ((rc = launch(pll_launch_wall_seed(g, L[0], cb, ct, s), "wall seed")) ||
+        (rc = pll_channel_force_vel_adj(a->ch, L[0], L[1], L[2], s)))
+        return rc;
     const size_t f3 = 3 * (a->fbytes / sizeof(double));
     for (int m = a->nck - 1; m >= 0; m--) {
         const int n0 = m * a->every;
@@ -263,16 +284,10 @@ int pll_adjoint_backward(pll_adjoint *a, double *gu, double *gv, double *gw, voi
             if ((rc = copy3(a, dst, Sf, s))) return rc;
             if ((rc = step_fwd(a, dst, s))) return rc;
         }
-        for (int n = n1 - 1; n >= n0; n--) {
-            if ((rc = step_adj(a, a->seg + (size_t)(n - n0) * f3, s))) return rc;
-            if (n >= 1 && (rc = seed(a, s))) return rc;  /* J reads the state n too */
-        }
+        for (int n = n1 - 1; n >= n0; n--)
+            if ((rc = step_adj(a, a->seg + (size_t)(n - n0) * f3, Gr,
+                               n == a->nsteps - 1 ? 0 : fmask, n == 0, s)))
+                return rc;
     }
-    double *G[3] = {gu, gv, gw};
-    for (int f = 0; f < 3; f++)
-        if ((rc = hipchk(hipMemcpyAsync(G[f], fld(a, a->grad, f), a->fbytes,
-                                        hipMemcpyDeviceToDevice, s),
-                         "copy of the gradient")))
-            return rc;
     return PLL_OK;
 }

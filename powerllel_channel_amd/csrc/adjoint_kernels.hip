@@ -81,6 +81,13 @@ __device__ __forceinline__ void set(double *b, unsigned o, double x)
     *reinterpret_cast<double *>(reinterpret_cast<char *>(b) + o) = x;
 }
 
+// periodic index in 1..n of any haloed index
+__device__ __forceinline__ int wrapn(int i, int n)
+{
+    const int r = (i - 1) % n;
+    return (r < 0 ? r + n : r) + 1;
+}
+
 struct JTiles {
     int ntx, nty, nkc, kc, xcd;
 };
@@ -145,8 +152,16 @@ __device__ __forceinline__ void jt_plane(const G &g, const double (*Q)[JNQ],
     a[2] = re * (dx * (Xm - X) + dy * (Ym - Y)) - 0.5 * cr * (X + Xm);
 }
 
-// o_F(c) = beta o_F(c) + a0 l_F(c) [c interior] + alpha (J_f(q)^T l)_F(c)
+// o_F(c) = beta x_F(c) + a0 l_F(c) [c interior] + alpha (J_f(q)^T l)_F(c)
 // over every cell c of the haloed arrays; l is read on the interior only.
+// FOLD: followed by the transposed boundary fill, on the interior alone.  The
+// fill copies periodically in x and y, so l and q wrap there; at the walls u
+// and v ghosts are 2 bc - the first or last plane, so what a ghost gathers
+// goes to that plane with a minus sign, and w's ghosts and wall row k = nz are
+// set to 0, so they pass nothing on.  q's own boundary values are formed from
+// its interior the same way (its fill need not be made).
+// GRAD: also gr += ga l + gb x, u's planes k = 1 and k = nz of o += cb and ct,
+// and the sums of o over the workgroup's cells into part (3 x workgroups).
 // A workgroup owns 64 x 4 columns and marches over a chunk of k with planes k
 // and k + 1 of q and l in LDS (tile plus one cell) and plane k + 2 on its way
 // into registers; what a z face adds to the plane above is carried there in
@@ -155,11 +170,19 @@ __device__ __forceinline__ void jt_plane(const G &g, const double (*Q)[JNQ],
 // 145 us, 3.1 TB/s; evaluating mom_rhs on dual numbers at the 13 outputs that
 // read a cell took 460 us.  Tiles of 64 x 8 and 64 x 12 (fewer workgroups per
 // CU) take 163 and 176 us, 64 x 8 at 16 waves (128 registers, spills) 255 us.
+// x may be o itself (each cell is read and written by the same lane).
+struct JGrad {
+    double *gu, *gv, *gw;
+    double ga, gb, cb, ct;
+    double *part;
+};
+
+template <bool FOLD, bool GRAD>
 __global__ void __launch_bounds__(JTX *JTY, 3)
 k_jtv(G g, JTiles t, const double *__restrict__ qu, const double *__restrict__ qv,
       const double *__restrict__ qw, const double *__restrict__ lu, const double *__restrict__ lv,
-      const double *__restrict__ lw, double *__restrict__ ou, double *__restrict__ ov,
-      double *__restrict__ ow, double alpha, double a0, double beta)
+      const double *__restrict__ lw, double *ou, double *ov, double *ow, const double *xu,
+      const double *xv, const double *xw, double alpha, double a0, double beta, JGrad J)
 {
     constexpr int NT = JTX * JTY, NR = (JNQ + NT - 1) / NT;
     __shared__ double tq[2][3][JNQ], tl[2][3][JNQ];
@@ -169,8 +192,9 @@ k_jtv(G g, JTiles t, const double *__restrict__ qu, const double *__restrict__ q
     lb /= t.ntx;
     const int ty = lb % t.nty, kc = lb / t.nty;
     const int tid = threadIdx.x, lx = tid & (JTX - 1), ly = tid / JTX;
-    const int i0 = tx * JTX, j0 = ty * JTY;  // haloed index of the tile's first cell
-    const int k0 = kc * t.kc, k1 = min(k0 + t.kc - 1, g.nz + 1);
+    constexpr int H = FOLD ? 1 : 0;  // first haloed index of the box
+    const int i0 = tx * JTX + H, j0 = ty * JTY + H;  // of the tile's first cell
+    const int k0 = kc * t.kc + H, k1 = min(k0 + t.kc - 1, g.nz + 1 - H);
     const int sy = (int)g.sy;
     unsigned off[NR];
     bool in[NR];
@@ -178,13 +202,15 @@ k_jtv(G g, JTiles t, const double *__restrict__ qu, const double *__restrict__ q
     for (int r = 0; r < NR; ++r) {
         const int q = min(tid + r * NT, JNQ - 1), row = q / JQX, col = q - row * JQX;
         const int i = i0 - 1 + col, j = j0 - 1 + row;
-        in[r] = i >= 1 && i <= g.nx && j >= 1 && j <= g.ny;
-        off[r] = 8u * (unsigned)(min(max(i, 0), g.nx + 1) + sy * min(max(j, 0), g.ny + 1));
+        in[r] = FOLD || (i >= 1 && i <= g.nx && j >= 1 && j <= g.ny);
+        const int ii = FOLD ? wrapn(i, g.nx) : min(max(i, 0), g.nx + 1);
+        const int jj = FOLD ? wrapn(j, g.ny) : min(max(j, 0), g.ny + 1);
+        off[r] = 8u * (unsigned)(ii + sy * jj);
     }
     double pq[3][NR], pl[3][NR];
-    bool lin = false;  // the plane fetched lies in the interior
+    int kpre = 0;  // the plane fetched
     auto fetch = [&](int kp) {
-        const long long e = g.sz * min(max(kp, 0), g.nz + 1);
+        const long long e = g.sz * min(max(kp, H), g.nz + 1 - H);
         // opaque offsets: no 64-bit lane address per array hoisted out of the loop
 #pragma unroll
         for (int r = 0; r < NR; ++r) asm volatile("" : "+v"(off[r]));
@@ -199,21 +225,30 @@ k_jtv(G g, JTiles t, const double *__restrict__ qu, const double *__restrict__ q
             pl[1][r] = at(m1, off[r]);
             pl[2][r] = at(m2, off[r]);
         }
-        lin = kp >= 1 && kp <= g.nz;
+        kpre = kp;
     };
     auto put = [&](int b) {
+        const bool wall = kpre < 1 || kpre > g.nz;
+        const double bcu = 0.0 - g.u_crf;
 #pragma unroll
-        for (int f = 0; f < 3; ++f)
-#pragma unroll
-            for (int r = 0; r < NR; ++r) {
-                const int q = min(tid + r * NT, JNQ - 1);
-                tq[b][f][q] = pq[f][r];
-                tl[b][f][q] = lin && in[r] ? pl[f][r] : 0.0;
+        for (int r = 0; r < NR; ++r) {
+            const int q = min(tid + r * NT, JNQ - 1);
+            double u = pq[0][r], v = pq[1][r], w = pq[2][r];
+            if (FOLD) {
+                u = wall ? 2.0 * bcu - u : u;
+                v = wall ? 2.0 * 0.0 - v : v;
+                w = wall || kpre == g.nz ? 0.0 : w;
             }
+            tq[b][0][q] = u;
+            tq[b][1][q] = v;
+            tq[b][2][q] = w;
+#pragma unroll
+            for (int f = 0; f < 3; ++f) tl[b][f][q] = !wall && in[r] ? pl[f][r] : 0.0;
+        }
     };
     const int c = (ly + 1) * JQX + lx + 1;
     const int i = i0 + lx, j = j0 + ly;
-    const bool own = i <= g.nx + 1 && j <= g.ny + 1;
+    const bool own = i <= g.nx + 1 - H && j <= g.ny + 1 - H;
     unsigned eo = 8u * (unsigned)(i + sy * j);
     double up[3] = {0.0, 0.0, 0.0};
     // plane k lives in slot (k - k0) & 1
@@ -226,7 +261,12 @@ k_jtv(G g, JTiles t, const double *__restrict__ qu, const double *__restrict__ q
     if (k0 > 0) {
         double lo[3] = {0.0, 0.0, 0.0};
         jt_face(g, jmet(g, k0 - 1), tq[1], tl[1], tq[0], tl[0], c, lo, up);
+        if (FOLD && k0 == 1) {  // the ghost plane's share goes to the first plane
+            up[0] -= lo[0];
+            up[1] -= lo[1];
+        }
     }
+    double sum[3] = {0.0, 0.0, 0.0};
     __syncthreads();
     put(1);
     __syncthreads();
@@ -239,13 +279,27 @@ k_jtv(G g, JTiles t, const double *__restrict__ qu, const double *__restrict__ q
         double a[3], nup[3];
         jt_plane(g, tq[b], tl[b], c, a);
         jt_face(g, jmet(g, k), tq[b], tl[b], tq[b ^ 1], tl[b ^ 1], c, a, nup);
+        if (FOLD && k == g.nz) {
+            a[0] -= nup[0];
+            a[1] -= nup[1];
+        }
         if (own) {
             const long long e = g.sz * k;
             double *const o[3] = {ou + e, ov + e, ow + e};
+            const double *const x[3] = {xu + e, xv + e, xw + e};
+            double *const gr[3] = {J.gu + e, J.gv + e, J.gw + e};
+            const double cw = k == 1 ? J.cb : (k == g.nz ? J.ct : 0.0);
 #pragma unroll
             for (int f = 0; f < 3; ++f) {
-                double r = alpha * (a[f] + up[f]) + a0 * tl[b][f][c];
-                if (beta != 0.0) r += beta * at(o[f], eo);
+                const double lc = tl[b][f][c];
+                const double xv = beta != 0.0 ? at(x[f], eo) : 0.0;
+                double r = alpha * (a[f] + up[f]) + a0 * lc + beta * xv;
+                if (FOLD && f == 2 && k == g.nz) r = 0.0;
+                if (GRAD) {
+                    if (f == 0) r += cw;
+                    set(gr[f], eo, at(gr[f], eo) + (J.ga * lc + J.gb * xv));
+                    sum[f] += r;
+                }
                 set(o[f], eo, r);
             }
         }
@@ -262,6 +316,19 @@ k_jtv(G g, JTiles t, const double *__restrict__ qu, const double *__restrict__ q
         plane(k + 1, std::integral_constant<int, 1>{});
     }
     if (k == k1) plane(k, std::integral_constant<int, 0>{});
+    if (GRAD) {
+        double *red = &tq[0][0][0];
+#pragma unroll
+        for (int f = 0; f < 3; ++f) red[f * NT + tid] = sum[f];
+        __syncthreads();
+        for (int h = NT / 2; h > 0; h >>= 1) {
+            if (tid < h)
+#pragma unroll
+                for (int f = 0; f < 3; ++f) red[f * NT + tid] += red[f * NT + tid + h];
+            __syncthreads();
+        }
+        if (tid < 3) J.part[(size_t)tid * gridDim.x + blockIdx.x] = red[tid * NT];
+    }
 }
 
 // o = J_f(q) dq on the interior (directional derivative of the momentum
@@ -426,6 +493,51 @@ __global__ void __launch_bounds__(256) k_rhs_adj(G g, const double *__restrict__
     lw[e] += wz;
 }
 
+// The same two transposes between transposed fills, on the interior alone: l
+// and the result are folded (periodic in x and y, no ghosts at the walls, w = 0
+// on its wall row), and the transposed forcing l -= dzflzi(k) tot of the
+// components in fmask is applied as l is read (tot: sum of l over the interior
+// / (nx ny)).  In the pressure gradient it cancels for u and v.
+#define PLL_CELL                                                   \
+    const int i = blockIdx.x * blockDim.x + threadIdx.x + 1;       \
+    const int j = blockIdx.y * blockDim.y + threadIdx.y + 1;       \
+    const int k = blockIdx.z + 1;                                  \
+    if (i > g.nx || j > g.ny) return;                              \
+    const long long sy = g.sy, sz = g.sz, e = i + sy * j + sz * k;
+
+__global__ void __launch_bounds__(256) k_correct_adj_fold(G g, const double *__restrict__ lu,
+                                                          const double *__restrict__ lv,
+                                                          const double *__restrict__ lw,
+                                                          double *__restrict__ lp, double dtdxi,
+                                                          double dtdyi, int fmask,
+                                                          const double *__restrict__ tot)
+{
+    PLL_CELL
+    const double sw = (fmask & 4) ? tot[2] : 0.0;
+    const double um = lu[i == 1 ? e - 1 + g.nx : e - 1], vm = lv[j == 1 ? e + sy * (g.ny - 1) : e - sy];
+    const double wt = k < g.nz ? g.dzc_inv[k] * (lw[e] - g.dzflzi[k] * sw) : 0.0;
+    const double wb = k > 1 ? g.dzc_inv[k - 1] * (lw[e - sz] - g.dzflzi[k - 1] * sw) : 0.0;
+    lp[e] = dtdxi * (lu[e] - um) + dtdyi * (lv[e] - vm) + g.dt * (wt - wb);
+}
+
+__global__ void __launch_bounds__(256) k_rhs_adj_fold(G g, const double *__restrict__ lr,
+                                                      double *__restrict__ lu,
+                                                      double *__restrict__ lv,
+                                                      double *__restrict__ lw, double dti,
+                                                      double dtidxi, double dtidyi, int fmask,
+                                                      const double *__restrict__ tot)
+{
+    PLL_CELL
+    const double wk = g.dzflzi[k];
+    const double rc = lr[e], rx = lr[i == g.nx ? e + 1 - g.nx : e + 1];
+    const double ry = lr[j == g.ny ? e - sy * (g.ny - 1) : e + sy], rz = k < g.nz ? lr[e + sz] : 0.0;
+    const double tu = (fmask & 1) ? wk * tot[0] : 0.0, tv = (fmask & 2) ? wk * tot[1] : 0.0,
+                 tw = (fmask & 4) ? wk * tot[2] : 0.0;
+    lu[e] = (lu[e] - tu) + dtidxi * (rc - rx);
+    lv[e] = (lv[e] - tv) + dtidyi * (rc - ry);
+    lw[e] = k == g.nz ? 0.0 : (lw[e] - tw) + dti * (g.dzf_inv[k] * rc - g.dzf_inv[k + 1] * rz);
+}
+
 // ------------------------------------------------------------ forcing
 // forceVel: q += vel_force - sum_c q_c dzflzi(k_c) / (nx ny).  Transpose:
 // l(c) -= dzflzi(k_c) / (nx ny) * sum_interior l.  Pass 1: per-(j,k)-row
@@ -447,11 +559,13 @@ __global__ void __launch_bounds__(256) k_rowsum(G g, const double *__restrict__ 
     if (threadIdx.x == 0) part[blockIdx.x] = sh[0];
 }
 
+// one workgroup per sum: out[b] = scale * sum of part[b n .. b n + n)
 __global__ void __launch_bounds__(1024) k_sum(int n, const double *__restrict__ part,
                                               double *__restrict__ out, double scale)
 {
     __shared__ double sh[1024];
     double s = 0.0;
+    part += (size_t)blockIdx.x * n;
     for (int t = threadIdx.x; t < n; t += blockDim.x) s += part[t];
     sh[threadIdx.x] = s;
     __syncthreads();
@@ -459,7 +573,7 @@ __global__ void __launch_bounds__(1024) k_sum(int n, const double *__restrict__ 
         if ((int)threadIdx.x < h) sh[threadIdx.x] += sh[threadIdx.x + h];
         __syncthreads();
     }
-    if (threadIdx.x == 0) out[0] = sh[0] * scale;
+    if (threadIdx.x == 0) out[blockIdx.x] = sh[0] * scale;
 }
 
 __global__ void __launch_bounds__(256) k_force_adj(G g, double *__restrict__ q,
@@ -511,18 +625,17 @@ __global__ void __launch_bounds__(256) k_wall_seed(G g, double *__restrict__ lu,
     lu[i + g.sy * j + g.sz * k] += (w == 0 ? c_bot : c_top);
 }
 
-// y += a x over every cell of the haloed arrays (three fields).
-__global__ void __launch_bounds__(256) k_axpy3(long long n, double a, const double *__restrict__ x0,
-                                               const double *__restrict__ x1,
-                                               const double *__restrict__ x2,
-                                               double *__restrict__ y0, double *__restrict__ y1,
-                                               double *__restrict__ y2)
+// y += a x + b z over every cell of the haloed arrays (three fields).
+struct Axpy3 {
+    const double *x[3], *z[3];
+    double *y[3];
+};
+__global__ void __launch_bounds__(256) k_axpy3(long long n, double a, double b, Axpy3 v)
 {
     const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= n) return;
-    y0[t] += a * x0[t];
-    y1[t] += a * x1[t];
-    y2[t] += a * x2[t];
+#pragma unroll
+    for (int f = 0; f < 3; ++f) v.y[f][t] += a * v.x[f][t] + b * v.z[f][t];
 }
 
 inline int ok() { return hipGetLastError() == hipSuccess ? 0 : -3; }
@@ -554,10 +667,41 @@ extern "C" int pll_launch_jtv(const pll_grid_dev *gd, const double *const q[3],
                               double a0, double beta, hipStream_t s)
 {
     const G g = make_g(gd);
-    if (g.sz > 0x7fffffffLL) return -1;
+    if (g.sz > 0x1fffffffLL) return -1;
     const JTiles t = jt_tiles(g.nx + 2, g.ny + 2, g.nz + 2, g.kc);
-    hipLaunchKernelGGL(k_jtv, dim3((unsigned)(t.ntx * t.nty * t.nkc)), dim3(JTX * JTY), 0, s, g, t,
-                       q[0], q[1], q[2], l[0], l[1], l[2], o[0], o[1], o[2], alpha, a0, beta);
+    hipLaunchKernelGGL((k_jtv<false, false>), dim3((unsigned)(t.ntx * t.nty * t.nkc)),
+                       dim3(JTX * JTY), 0, s, g, t, q[0], q[1], q[2], l[0], l[1], l[2], o[0], o[1],
+                       o[2], o[0], o[1], o[2], alpha, a0, beta, JGrad{});
+    return ok();
+}
+
+extern "C" int pll_jtv_fold_blocks(const pll_grid_dev *gd)
+{
+    const G g = make_g(gd);
+    const JTiles t = jt_tiles(g.nx, g.ny, g.nz, g.kc);
+    return t.ntx * t.nty * t.nkc;
+}
+
+extern "C" int pll_launch_jtv_fold(const pll_grid_dev *gd, const double *const q[3],
+                                   const double *const l[3], double *const o[3],
+                                   const double *const x[3], double alpha, double a0, double beta,
+                                   double *const gr[3], double ga, double gb, double cb, double ct,
+                                   double *part, hipStream_t s)
+{
+    const G g = make_g(gd);
+    if (g.sz > 0x1fffffffLL) return -1;
+    const JTiles t = jt_tiles(g.nx, g.ny, g.nz, g.kc);
+    const dim3 grid((unsigned)(t.ntx * t.nty * t.nkc)), blk(JTX * JTY);
+    const double *const *y = x ? x : l;
+    if (gr) {
+        const JGrad J{gr[0], gr[1], gr[2], ga, gb, cb, ct, part};
+        hipLaunchKernelGGL((k_jtv<true, true>), grid, blk, 0, s, g, t, q[0], q[1], q[2], l[0], l[1],
+                           l[2], o[0], o[1], o[2], y[0], y[1], y[2], alpha, a0, x ? beta : 0.0, J);
+    } else {
+        hipLaunchKernelGGL((k_jtv<true, false>), grid, blk, 0, s, g, t, q[0], q[1], q[2], l[0],
+                           l[1], l[2], o[0], o[1], o[2], y[0], y[1], y[2], alpha, a0,
+                           x ? beta : 0.0, JGrad{});
+    }
     return ok();
 }
 
@@ -631,9 +775,7 @@ extern "C" int pll_launch_wall_sum(const pll_grid_dev *gd, const double *u, doub
     const G g = make_g(gd);
     hipLaunchKernelGGL(k_wall_rows, dim3(2 * g.ny), dim3(256), 0, s, g, u, part);
     if (ok()) return -3;
-    hipLaunchKernelGGL(k_sum, dim3(1), dim3(1024), 0, s, g.ny, part, out, 1.0);
-    if (ok()) return -3;
-    hipLaunchKernelGGL(k_sum, dim3(1), dim3(1024), 0, s, g.ny, part + g.ny, out + 1, 1.0);
+    hipLaunchKernelGGL(k_sum, dim3(2), dim3(1024), 0, s, g.ny, part, out, 1.0);
     return ok();
 }
 
@@ -647,11 +789,40 @@ extern "C" int pll_launch_wall_seed(const pll_grid_dev *gd, double *lu, double c
 }
 
 extern "C" int pll_launch_axpy3(const pll_grid_dev *gd, double a, const double *const x[3],
-                                double *const y[3], hipStream_t s)
+                                double b, const double *const z[3], double *const y[3],
+                                hipStream_t s)
 {
     const G g = make_g(gd);
     const long long n = ncell(g);
-    hipLaunchKernelGGL(k_axpy3, dim3(nblk(n)), dim3(256), 0, s, n, a, x[0], x[1], x[2], y[0], y[1],
-                       y[2]);
+    const Axpy3 v{{x[0], x[1], x[2]}, {z[0], z[1], z[2]}, {y[0], y[1], y[2]}};
+    hipLaunchKernelGGL(k_axpy3, dim3(nblk(n)), dim3(256), 0, s, n, a, b, v);
+    return ok();
+}
+
+extern "C" int pll_launch_correct_adj_fold(const pll_grid_dev *gd, const double *const l[3],
+                                           double *lp, int fmask, const double *tot, hipStream_t s)
+{
+    const G g = make_g(gd);
+    hipLaunchKernelGGL(k_correct_adj_fold, dim3((g.nx + 63) / 64, (g.ny + 3) / 4, g.nz),
+                       dim3(64, 4, 1), 0, s, g, l[0], l[1], l[2], lp, g.dt * g.dx_inv,
+                       g.dt * g.dy_inv, fmask, tot);
+    return ok();
+}
+
+extern "C" int pll_launch_rhs_adj_fold(const pll_grid_dev *gd, const double *lr,
+                                       double *const l[3], int fmask, const double *tot,
+                                       hipStream_t s)
+{
+    const G g = make_g(gd);
+    const double dti = 1.0 / g.dt;
+    hipLaunchKernelGGL(k_rhs_adj_fold, dim3((g.nx + 63) / 64, (g.ny + 3) / 4, g.nz),
+                       dim3(64, 4, 1), 0, s, g, lr, l[0], l[1], l[2], dti, dti * g.dx_inv,
+                       dti * g.dy_inv, fmask, tot);
+    return ok();
+}
+
+extern "C" int pll_launch_sum3(int n, const double *part, double *out, double scale, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_sum, dim3(3), dim3(1024), 0, s, n, part, out, scale);
     return ok();
 }

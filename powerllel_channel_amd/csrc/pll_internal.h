@@ -263,9 +263,29 @@ int pll_launch_wall_sum(const pll_grid_dev *g, const double *u, double *part, do
 /* lu += c_bot on the plane k = 1 and c_top on k = nz (interior) */
 int pll_launch_wall_seed(const pll_grid_dev *g, double *lu, double c_bot, double c_top,
                          hipStream_t s);
-/* y += a x over every cell, three fields */
-int pll_launch_axpy3(const pll_grid_dev *g, double a, const double *const x[3],
-                     double *const y[3], hipStream_t s);
+/* y += a x + b z over every cell, three fields */
+int pll_launch_axpy3(const pll_grid_dev *g, double a, const double *const x[3], double b,
+                     const double *const z[3], double *const y[3], hipStream_t s);
+/* The pieces of a reversed step between transposed boundary fills: every
+ * adjoint field is folded (ghosts not read or written, w = 0 on its wall row).
+ * o = beta x + a0 l + alpha J_f(q)^T l folded, x NULL (no beta term) or three
+ * fields, o themselves included; q's boundary values are formed from its
+ * interior.  gr non-NULL: also gr += ga l + gb x, o_u += cb on the plane k = 1
+ * and ct on k = nz, and the sums of o's fields over each workgroup into part
+ * (three times pll_jtv_fold_blocks). */
+int pll_launch_jtv_fold(const pll_grid_dev *g, const double *const q[3], const double *const l[3],
+                        double *const o[3], const double *const x[3], double alpha, double a0,
+                        double beta, double *const gr[3], double ga, double gb, double cb,
+                        double ct, double *part, hipStream_t s);
+int pll_jtv_fold_blocks(const pll_grid_dev *g);
+/* tot: device, 3 sums of l over the interior / (nx ny); the components in
+ * fmask take the transposed forcing l -= dzflzi(k) tot as they are read */
+int pll_launch_correct_adj_fold(const pll_grid_dev *g, const double *const l[3], double *lp,
+                                int fmask, const double *tot, hipStream_t s);
+int pll_launch_rhs_adj_fold(const pll_grid_dev *g, const double *lr, double *const l[3],
+                            int fmask, const double *tot, hipStream_t s);
+/* out[d] = scale * sum of part[d n .. d n + n), d = 0, 1, 2 */
+int pll_launch_sum3(int n, const double *part, double *out, double scale, hipStream_t s);
 
 /* Host-layer calls between ppe.c and channel.c (pll_ppe from powerllel.h). */
 struct pll_ppe;

@@ -105,3 +105,74 @@ def test_rk_vjp_transposes_jvp(cuda, shape):
         want = 0.25 * b - 0.5 * y
         want[inner] += 1.5 * l[inner]
         assert float((a - want).abs().max()) <= 1e-14 * float(b.abs().max() + y.abs().max() + 2.0)
+
+
+@pytest.mark.parametrize("shape,forced,every", [
+    ((66, 18, 17), (True, False, False), 1), ((12, 10, 8), (True, True, False), 2),
+    ((64, 4, 37), (False, False, True), 3), ((130, 20, 6), (False, False, False), 2)])
+def test_window_gradient_vs_pieces(cuda, shape, forced, every):
+    """The window's reversed steps (transposed fills, forcing and gradient
+    fused into the passes around them) against the public transposes applied
+    one after the other: 3 steps, 1e-11 of the largest gradient value (the
+    pieces agree with the forward ones to 1e-12)."""
+    import torch
+    from powerllel_channel_amd import Channel, PoissonSolver
+    from powerllel_channel_amd.adjoint import WallShearWindow
+    from powerllel_channel_amd.mesh import Grid
+    nx, ny, nz = shape
+    print(f"[window vs pieces] {shape} forced={forced} every={every}", flush=True)
+    nu, dt, n = 1e-2, 1e-3, 3
+    g = Grid(nx, ny, nz, 0.1 * nx, 0.1 * ny, 2.0, 2.0)
+    ch = Channel(nx, ny, nz, g.lx, g.ly, g.lz, g.dzf, nu, dt, u_crf=0.2, is_forced=forced,
+                 vel_force=(1.0, 0.1, 0.0))
+    s = PoissonSolver(nx, ny, nz, g.dx, g.dy, g.dzf)
+    gen = torch.Generator().manual_seed(7)
+    U, b = [[0.3 * torch.randn(g.shape, generator=gen, dtype=torch.float64).to(cuda)
+             for _ in range(3)] for _ in range(2)]
+    ch.bc_vel(*U)
+    win = WallShearWindow(ch, s, n, every)
+    for _ in range(2):  # a second pass on the same window
+        win.forward(*U, *b)
+        got = [torch.full_like(U[0], 9.0) for _ in range(3)]
+        win.backward(*got)
+    again = [torch.zeros_like(U[0]) for _ in range(3)]
+    win.backward(*again)  # and a second backward of one forward
+
+    def zeros(m):
+        return [torch.zeros_like(U[0]) for _ in range(m)]
+    states, u = [], [t.clone() for t in U]
+    for _ in range(n):
+        states.append([t.clone() for t in u])
+        ch.step_body(s, *u, *zeros(4), *b)
+    inner = (slice(1, -1),) * 3
+    c = nu / (n * nx * ny)
+
+    def seed(lam):
+        lam[0][1, 1:-1, 1:-1] += c / g.dzf[1]
+        lam[0][nz, 1:-1, 1:-1] += c / g.dzf[nz]
+    lam, grad = zeros(3), zeros(3)
+    seed(lam)
+    for m in range(n - 1, -1, -1):
+        u1, (lp,), l1 = zeros(3), zeros(1), zeros(3)
+        ch.rk1(*states[m], *u1)
+        for t, f in zip(u1, b):
+            t[inner] += dt * f[inner]
+        ch.bc_vel(*u1)
+        ch.bc_vel_adj(*lam)
+        ch.force_vel_adj(*lam)
+        ch.correct_vel_adj(*lam, lp)
+        ch.bc_p_adj(lp)
+        s.solve_adjoint(lp)
+        ch.calc_rhs_adj(lp, *lam)
+        ch.bc_vel_adj(*lam)
+        ch.rk_vjp(u1, lam, l1, 0.5 * dt, 0.5, 0.0)
+        ch.bc_vel_adj(*l1)
+        for q, a, d in zip(grad, lam, l1):
+            q += 0.5 * dt * a + dt * d
+        ch.rk_vjp(states[m], l1, lam, dt, 1.0, 0.5)
+        if m:
+            seed(lam)
+    top = max(float(q.abs().max()) for q in grad)
+    for q, w, w2 in zip(got, grad, again):
+        assert float((q - w).abs().max()) <= 1e-11 * top
+        assert torch.equal(q, w2)
