@@ -8,9 +8,10 @@
  * RK stages of every step (pll_channel_step_body).
  *
  * Forward: the steps run with checkpoints of (u,v,w) every `ckpt_every`
- * steps.  Backward: per segment, the states of the segment are recomputed
- * from its checkpoint, then the steps are reversed; each reversed step
- * recomputes its RK1 stage (stage recomputation).  One reversed step is the
+ * steps and leave the last segment's states in place.  Backward: per segment,
+ * the states of the segment are recomputed from its checkpoint, then the steps
+ * are reversed; each reversed step recomputes its RK1 stage (stage
+ * recomputation).  One reversed step is the
  * transpose of the forward step's linearisation, in reverse order:
  *   boundary fill, forcing, correctVel, updateBoundP, PPE (transposed solve),
  *   calcRHS, boundary fill, RK2 (Jacobian at u1), boundary fill, RK1
@@ -29,7 +30,7 @@ struct pll_adjoint {
     int nsteps, every, nck;
     size_t fbytes;           /* bytes of one haloed field */
     double *ck;              /* nck checkpoints x 3 fields */
-    double *seg;             /* every states x 3 fields */
+    double *seg;             /* every states x 3 fields: see state() */
     double *u1, *p;          /* 3 fields, 1 field */
     double *lam, *lam1, *lamp, *body; /* 3, 3, 1, 3 fields */
     double *jpart, *tot;     /* device: partial sums of lam, the 3 sums */
@@ -37,6 +38,7 @@ struct pll_adjoint {
     double *part;            /* device: partials for the wall sums */
     double *hsum;            /* host: 2 nsteps */
     int have_forward;
+    int held;                /* segment whose states are in seg (-1: none) */
     size_t dev_bytes;
 };
 
@@ -139,12 +141,25 @@ static int copy3(const pll_adjoint *a, double *dst, const double *const src[3], 
     return PLL_OK;
 }
 
-static int step_fwd(pll_adjoint *a, double *U, hipStream_t s)
+/* Where state n of the window lives: the states at multiples of `every` are
+ * the checkpoints (but the window's last state), the others go to slot
+ * n mod every of seg, which holds one segment at a time. */
+static double *state(const pll_adjoint *a, int n)
 {
+    const size_t f3 = 3 * (a->fbytes / sizeof(double));
+    return n % a->every == 0 && n < a->nsteps ? a->ck + (size_t)(n / a->every) * f3
+                                              : a->seg + (size_t)(n % a->every) * f3;
+}
+
+/* state n -> state n + 1; the ghosts of state 0 are the caller's */
+static int step_fwd(pll_adjoint *a, int n, hipStream_t s)
+{
+    double *S = state(a, n), *D = state(a, n + 1);
+    const double *src[3] = {fld(a, S, 0), fld(a, S, 1), fld(a, S, 2)};
+    double *dst[3] = {fld(a, D, 0), fld(a, D, 1), fld(a, D, 2)};
+    double *tmp[3] = {fld(a, a->u1, 0), fld(a, a->u1, 1), fld(a, a->u1, 2)};
     const double *body[3] = {fld(a, a->body, 0), fld(a, a->body, 1), fld(a, a->body, 2)};
-    return pll_channel_step_body_internal(a->ch, a->ppe, fld(a, U, 0), fld(a, U, 1),
-                                          fld(a, U, 2), fld(a, a->u1, 0), fld(a, a->u1, 1),
-                                          fld(a, a->u1, 2), a->p, body, s);
+    return pll_channel_step_from(a->ch, a->ppe, src, dst, tmp, a->p, body, n > 0, s);
 }
 
 int pll_adjoint_forward(pll_adjoint *a, const double *u0, const double *v0, const double *w0,
@@ -160,21 +175,14 @@ int pll_adjoint_forward(pll_adjoint *a, const double *u0, const double *v0, cons
     int rc;
     if ((rc = copy3(a, a->body, B, s))) return rc;
     if ((rc = copy3(a, a->ck, U0, s))) return rc;
-    /* the running state lives in seg[0] */
-    double *S = a->seg;
-    const double *C0[3] = {fld(a, a->ck, 0), fld(a, a->ck, 1), fld(a, a->ck, 2)};
-    if ((rc = copy3(a, S, C0, s))) return rc;
+    a->held = -1;
     for (int n = 0; n < a->nsteps; n++) {
-        if ((rc = step_fwd(a, S, s))) return rc;
-        if ((rc = launch(pll_launch_wall_sum(g, fld(a, S, 0), a->part, a->wsum + 2 * n, s),
+        if ((rc = step_fwd(a, n, s))) return rc;
+        if ((rc = launch(pll_launch_wall_sum(g, state(a, n + 1), a->part, a->wsum + 2 * n, s),
                          "wall shear")))
             return rc;
-        if ((n + 1) % a->every == 0 && (n + 1) < a->nsteps) {
-            const double *Sf[3] = {fld(a, S, 0), fld(a, S, 1), fld(a, S, 2)};
-            if ((rc = copy3(a, a->ck + (size_t)((n + 1) / a->every) * 3 * (a->fbytes / 8), Sf, s)))
-                return rc;
-        }
     }
+    a->held = a->nck - 1;
     if ((rc = hipchk(hipMemcpyAsync(a->hsum, a->wsum, sizeof(double) * 2 * (size_t)a->nsteps,
                                     hipMemcpyDeviceToHost, s),
                      "copy of wall sums")))
@@ -270,22 +278,20 @@ int pll_adjoint_backward(pll_adjoint *a, double *gu, double *gv, double *gw, voi
     if ((rc = launch(pll_launch_wall_seed(g, L[0], cb, ct, s), "wall seed")) ||
         (rc = pll_channel_force_vel_adj(a->ch, L[0], L[1], L[2], s)))
         return rc;
-    const size_t f3 = 3 * (a->fbytes / sizeof(double));
     for (int m = a->nck - 1; m >= 0; m--) {
         const int n0 = m * a->every;
         const int n1 = n0 + a->every < a->nsteps ? n0 + a->every : a->nsteps;
-        /* states n0 .. n1-1 of the segment into seg[0 .. n1-n0) */
-        const double *C[3] = {a->ck + (size_t)m * f3, a->ck + (size_t)m * f3 + f3 / 3,
-                              a->ck + (size_t)m * f3 + 2 * (f3 / 3)};
-        if ((rc = copy3(a, a->seg, C, s))) return rc;
-        for (int n = n0; n < n1 - 1; n++) {
-            double *src = a->seg + (size_t)(n - n0) * f3, *dst = src + f3;
-            const double *Sf[3] = {src, src + f3 / 3, src + 2 * (f3 / 3)};
-            if ((rc = copy3(a, dst, Sf, s))) return rc;
-            if ((rc = step_fwd(a, dst, s))) return rc;
+        /* the segment's states after its checkpoint, unless seg holds them
+         * (the last segment's after a forward, the first one's after a
+         * backward) */
+        if (a->held != m) {
+            a->held = -1;
+            for (int n = n0; n < n1 - 1; n++)
+                if ((rc = step_fwd(a, n, s))) return rc;
+            a->held = m;
         }
         for (int n = n1 - 1; n >= n0; n--)
-            if ((rc = step_adj(a, a->seg + (size_t)(n - n0) * f3, Gr,
+            if ((rc = step_adj(a, state(a, n), Gr,
                                n == a->nsteps - 1 ? 0 : fmask, n == 0, s)))
                 return rc;
     }

@@ -364,6 +364,30 @@ int pll_channel_step(pll_channel *c, pll_ppe *ppe, double *u, double *v, double 
     return step_impl(c, ppe, u, v, w, u1, v1, w1, p, NULL, stream);
 }
 
+/* Mean_h of the RK2 output from its partial sums, into scal[4], scal[5] */
+static int forcing_means(pll_channel *c, int fmask, hipStream_t s)
+{
+    const int nb = pll_rk_blocks(&c->g);
+    for (int d = 0; d < 2; d++)
+        if ((fmask >> d) & 1) {
+            const int rc = kl(pll_launch_mean_final(nb, c->part + (size_t)d * nb, c->scal + 4 + d,
+                                                    c->g.nx, c->g.ny, s),
+                              "mean final");
+            if (rc) return rc;
+        }
+    return PLL_OK;
+}
+
+/* the FP64 solve with calcRHS of a velocity whose boundary fill is not made */
+static int solve_unfilled(pll_channel *c, pll_ppe *ppe, const double *const q[3], double *p,
+                          hipStream_t s)
+{
+    const double dti = 1.0 / c->g.dt;
+    const pll_div_src d = {q[0], q[1], q[2], c->g.dzf_inv, dti, dti * c->g.dx_inv,
+                           dti * c->g.dy_inv, 1};
+    return pll_ppe_solve_div(ppe, &d, p, s);
+}
+
 /* m steps whose projections are carried into the next step.  Step 0 takes
  * the caller's state (whatever its ghost cells hold) through RK1 and RK2 in
  * place.  Every later step reads the previous step's RK2 output X, neither
@@ -382,8 +406,6 @@ static int run_chain(pll_channel *c, pll_ppe *ppe, int m, double *u, double *v, 
     double *const *X = A;
     const double *mean = fmask ? c->scal + 4 : NULL;
     double *part = fmask ? c->part : NULL;
-    const double dti = 1.0 / c->g.dt;
-    const int nb = pll_rk_blocks(&c->g);
     int rc;
     for (int i = 0; i < m; i++) {
         if (i == 0) {
@@ -400,15 +422,8 @@ static int run_chain(pll_channel *c, pll_ppe *ppe, int m, double *u, double *v, 
                 return rc;
             X = Y;
         }
-        for (int d = 0; d < 2; d++)
-            if ((fmask >> d) & 1)
-                if ((rc = kl(pll_launch_mean_final(nb, c->part + (size_t)d * nb, c->scal + 4 + d,
-                                                   c->g.nx, c->g.ny, s),
-                             "mean final")))
-                    return rc;
-        const pll_div_src q = {X[0], X[1], X[2], c->g.dzf_inv, dti, dti * c->g.dx_inv,
-                               dti * c->g.dy_inv, 1};
-        if ((rc = pll_ppe_solve_div(ppe, &q, p, s))) return rc;
+        const double *q[3] = {X[0], X[1], X[2]};
+        if ((rc = forcing_means(c, fmask, s)) || (rc = solve_unfilled(c, ppe, q, p, s))) return rc;
     }
     const double *q[3] = {X[0], X[1], X[2]};
     if ((rc = kl(pll_launch_correct_vel(&c->g, p, q, u, v, w, fmask, c->vel_force[0],
@@ -443,11 +458,36 @@ int pll_channel_run(pll_channel *c, pll_ppe *ppe, int nsteps, double *u, double 
     return run_chain(c, ppe, nsteps, u, v, w, u1, v1, w1, p, fmask, s);
 }
 
-int pll_channel_step_body_internal(pll_channel *c, pll_ppe *ppe, double *u, double *v,
-                                   double *w, double *u1, double *v1, double *w1, double *p,
-                                   const double *const *body, void *stream)
+/* A step with a body force from src to dst (other arrays, like the work space
+ * tmp; dst ends filled).  With filled, src's boundary fill has been made by this
+ * library, and RK1 and RK2 are one pass from src to tmp, corrected into dst:
+ * the roundings of step_impl.  Otherwise (a caller's ghost cells, a forced w,
+ * the refined solve) src is copied to dst and stepped in place. */
+int pll_channel_step_from(pll_channel *c, pll_ppe *ppe, const double *const src[3],
+                          double *const dst[3], double *const tmp[3], double *p,
+                          const double *const *body, int filled, void *stream)
 {
-    return step_impl(c, ppe, u, v, w, u1, v1, w1, p, body, stream);
+    CHK_C(c);
+    hipStream_t s = (hipStream_t)stream;
+    int rc;
+    if (!filled || c->is_forced[2] || pll_ppe_refinement(ppe) >= 0) {
+        const size_t bytes = sizeof(double) * (size_t)(c->g.nx + 2) * (c->g.ny + 2) * (c->g.nz + 2);
+        for (int f = 0; f < 3; f++)
+            HIPCHK(hipMemcpyAsync(dst[f], src[f], bytes, hipMemcpyDeviceToDevice, s));
+        return step_impl(c, ppe, dst[0], dst[1], dst[2], tmp[0], tmp[1], tmp[2], p, body, stream);
+    }
+    const int fmask = (c->is_forced[0] ? 1 : 0) | (c->is_forced[1] ? 2 : 0);
+    const double *mean = fmask ? c->scal + 4 : NULL;
+    const double *q[3] = {tmp[0], tmp[1], tmp[2]};
+    if ((rc = kl(pll_launch_rk12(&c->g, src, tmp, NULL, fmask ? c->part : NULL, fmask, 0.0, 0.0,
+                                 NULL, body, s),
+                 "rk1 + rk2")) ||
+        (rc = forcing_means(c, fmask, s)) || (rc = solve_unfilled(c, ppe, q, p, s)) ||
+        (rc = kl(pll_launch_correct_vel(&c->g, p, q, dst[0], dst[1], dst[2], fmask,
+                                        c->vel_force[0], c->vel_force[1], mean, s),
+                 "correct_vel")))
+        return rc;
+    return pll_channel_bc_vel(c, dst[0], dst[1], dst[2], stream);
 }
 
 int pll_channel_step_body(pll_channel *c, pll_ppe *ppe, double *u, double *v, double *w,

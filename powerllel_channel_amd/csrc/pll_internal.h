@@ -298,13 +298,16 @@ int pll_ppe_solve_div(struct pll_ppe *h, const pll_div_src *q, double *d_var, vo
 int pll_ppe_refinement(const struct pll_ppe *h);
 struct pll_channel;
 const pll_grid_dev *pll_channel_grid(const struct pll_channel *c);
+int pll_set_error(int code, const char *fmt, ...);
 int pll_channel_forcing(const struct pll_channel *c, int is_forced[3], double vel_force[3]);
 const double *pll_channel_dzf_host(const struct pll_channel *c);
 /* averaged wall shear from the two plane sums of u */
 double pll_wall_shear_from_sums(const struct pll_channel *c, const double sums[2]);
-int pll_channel_step_body_internal(struct pll_channel *c, struct pll_ppe *ppe, double *u,
-                                   double *v, double *w, double *u1, double *v1, double *w1,
-                                   double *p, const double *const *body, void *stream);
+/* one step with a body force from src to dst (work space tmp; three different
+ * sets); filled: src's boundary fill has been made */
+int pll_channel_step_from(struct pll_channel *c, struct pll_ppe *ppe, const double *const src[3],
+                          double *const dst[3], double *const tmp[3], double *p,
+                          const double *const *body, int filled, void *stream);
 
 #ifdef __cplusplus
 }
