@@ -64,6 +64,9 @@ typedef struct {
         int h64;               /* FP64 storage: the same, at S = 16 only */
         int qx32;              /* qx for those tiles */
         const int *order32;    /* [nx/(2S) ny] their launch order */
+        int rag;               /* tiles of S columns of the plane's nx ny, P M >= nz
+                                  rows; order: ceil(nx ny / S) entries, exact tiles
+                                  marked (qx, iyx, h32, h64, order32 unused) */
     } tp;
     /* refined form: the lowest modes (kx in {0,1}, ky in {0,1,ny-1}) of each
      * FP32 solve in FP64 (low_on = 0: off).  low_rx [ny nz][2] the x sums of
@@ -157,6 +160,7 @@ void pll_copy_pool_destroy(pll_copy_pool *p);
 int pll_launch_xbwd_fill(const pll_ppe_dev *d, const void *W, double *p, hipStream_t s);
 /* 1 if the partitioned z solve is instantiated for M rows per lane. */
 int pll_trid_part_supported(int M);
+int pll_trid_rag_exact(void); /* the mark of an exact tile in a ragged tile list */
 /* 1 if a kernel instantiation exists for E (elements per thread). */
 int pll_fft_supported_E(int E);
 /* largest workgroup the E instantiation is compiled for (FP64 kernels;

@@ -339,6 +339,54 @@ static int choose_part(int nx, int nz, int *M, int *P, int *S)
     return 0;
 }
 
+/* Ragged layout of the partitioned z solve, for any nx and nz: tiles of S
+ * consecutive columns of the plane's nx ny, P lanes of M rows with P M >= nz.
+ * P = 16 lanes (one DPP row per column) where its padding is at most 16 rows
+ * over the smallest; else the least padding.  Returns 0 for nz > 1024. */
+static int choose_rag(int nz, int *M, int *P, int *S)
+{
+    static const int Ps[] = {16, 8, 4, 2, 32, 64};
+    int best = 0;
+    for (size_t i = 0; i < sizeof Ps / sizeof Ps[0]; i++) {
+        const int p = Ps[i];
+        int m = (nz + p - 1) / p;
+        m = m < 4 ? 4 : m + m % 2;
+        if (m > 16 || (best && m * p >= best - (*P == 16 ? 16 : 0))) continue;
+        best = m * p;
+        *M = m;
+        *P = p;
+        *S = p <= 16 ? 32 : 512 / p;
+    }
+    return best > 0;
+}
+
+/* Launch order of the ragged tiles: those with a column of the exact path
+ * (q < qx and iy < iyx) first and marked, then as tile_order. */
+static int *rag_order(int nx, int ny, int S, int qx, int iyx)
+{
+    const int ncol = nx * ny, nt = (ncol + S - 1) / S, mark = pll_trid_rag_exact();
+    char *ex = (char *)calloc((size_t)nt, 1);
+    int *list = (int *)malloc(sizeof(int) * (size_t)nt);
+    int *order = (int *)malloc(sizeof(int) * (size_t)nt);
+    if (ex && list && order) {
+        for (int my = 0; my < ny; my++)
+            if ((my <= ny - my ? my : ny - my) < iyx)
+                for (int q = 0; q < nx && q < qx; q++) ex[(my * nx + q) / S] = 1;
+        int n = 0;
+        for (int pass = 0; pass < 2; pass++)
+            for (int t = 0; t < nt; t++)
+                if (ex[t] == (pass == 0)) list[n++] = ex[t] ? t | mark : t;
+        for (int b = 0; b < nt; b++)
+            order[b] = nt % 8 == 0 ? list[(b % 8) * (nt / 8) + b / 8] : list[b];
+    } else {
+        free(order);
+        order = NULL;
+    }
+    free(ex);
+    free(list);
+    return order;
+}
+
 /* Launch order of the z-solve tiles (SW columns each, nx/SW per y row): tiles
  * with exact-path columns (q0 < qx, iy < iyx) first; workgroup b runs tile
  * order[b].  Workgroups reach the 8 XCDs round-robin, so each XCD is handed a
@@ -492,9 +540,23 @@ int pll_ppe_create(pll_ppe **out, int nx, int ny, int nz, double dx, double dy,
     h->d.bz = (const double *)h->bz;
     h->d.dz = (const double *)h->bz + nz;
     {
-        int M, P, S;
-        if (!getenv("PLL_TRID_STREAMING") && choose_part(nx, nz, &M, &P, &S)) {
-            const int ntx = nx / S, ntiles = ntx * ny;
+        int M, P, S, rM, rP = 0, rS;
+        int part = choose_part(nx, nz, &M, &P, &S);
+        /* Ragged tiles where the regular layout does not exist, or has 4 columns
+         * (32-byte row segments): 500x250x128 498 -> 442 us per solve, 100x100x64
+         * 43 -> 40.  With 8 columns and more the regular one is faster:
+         * 360x128x128 159 us (ragged 166), 400x256x128 242 (257).
+         * PLL_TRID_RAG (tuning): 0 never, 1 always */
+        const char *pr = getenv("PLL_TRID_RAG");
+        int rag = choose_rag(nz, &rM, &rP, &rS) && (pr ? atoi(pr) != 0 : !part || S < 8);
+        if (rag) {
+            M = rM;
+            P = rP;
+            S = rS;
+            part = 1;
+        }
+        if (!getenv("PLL_TRID_STREAMING") && part) {
+            const int ntx = nx / S, ntiles = rag ? (nx * ny + S - 1) / S : ntx * ny;
             /* exact-path thresholds: |lambda| < tau * max|bz| */
             double bmax = 0.0;
             for (int k = 0; k < nz; k++) bmax = fabs(bz[k]) > bmax ? fabs(bz[k]) : bmax;
@@ -506,7 +568,7 @@ int pll_ppe_create(pll_ppe **out, int nx, int ny, int nz, double dx, double dy,
             int qx = iyx > 0 ? 2 * (ixmax + 1) : 0;
             const int qx0 = qx;
             qx = ((qx0 + S - 1) / S) * S;
-            int *order = tile_order(nx, ny, S, qx, iyx);
+            int *order = rag ? rag_order(nx, ny, S, qx0, iyx) : tile_order(nx, ny, S, qx, iyx);
             if (!order) {
                 rc = pll_set_error(PLL_ENOMEM, "host allocation failed");
                 goto fail;
@@ -514,7 +576,7 @@ int pll_ppe_create(pll_ppe **out, int nx, int ny, int nz, double dx, double dy,
             /* FP32 storage: tiles of 2 S columns (256-byte row segments at
              * S = 32), if their LDS fits (PLL_TRID32_H=1: S columns) */
             const char *ph = getenv("PLL_TRID32_H");
-            const int h32 = (S >= 16 && nx % (2 * S) == 0 &&
+            const int h32 = (!rag && S >= 16 && nx % (2 * S) == 0 &&
                              (size_t)nz * 2 * S * 8 + (size_t)nz * 24 + (size_t)P * 8 <= 163840 &&
                              !(ph && atoi(ph) == 1)) ? 2 : 1;
             const int qx32 = ((qx0 + 2 * S - 1) / (2 * S)) * (2 * S);
@@ -568,6 +630,7 @@ int pll_ppe_create(pll_ppe **out, int nx, int ny, int nz, double dx, double dy,
             }
             free(order);
             free(lxh);
+            h->d.tp.rag = rag;
             h->d.tp.M = M;
             h->d.tp.P = P;
             h->d.tp.S = S;

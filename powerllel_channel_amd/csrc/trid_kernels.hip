@@ -119,7 +119,11 @@ struct PArgs {
     const int *order;
     int L, nx, ny, nz, P, lP, S, ntx, ntiles, pin_gauge;  // P = 1 << lP
     int qx, iyx;  // exact path for tiles with q0 < qx and iy < iyx
+    int ncol;     // RAG: columns nx ny
 };
+
+// RAG tile lists: this bit of an entry marks an exact-path tile
+constexpr int RAG_EXACT = 1 << 30;
 
 // 1/x from the hardware reciprocal plus two Newton steps (full double
 // precision, not necessarily correctly rounded); x is a nonzero pivot.
@@ -199,7 +203,15 @@ __device__ __forceinline__ int lam_ix(int q, int my, int L, int ny)
 // wide in memory (256-byte row segments where S floats make only 128), and
 // the S P threads solve the groups one after the other; g.ntx counts tiles of
 // SW columns.
-template <int M, int S, typename St, bool DPP16, int H = 1>
+// RAG: any nx and nz.  The columns of a plane are contiguous in memory, so a
+// tile is S consecutive ones of the nx ny whichever y rows they belong to
+// (the last tile may be cut), and the P M rows that the lanes hold may exceed
+// nz: the rows above are empty equations (a = c = 0, d = 0, and the wall's
+// c_{nz-1} = 0 keeps row nz - 1 from them), neither loaded nor stored.  One
+// read and one write of the array where the streaming recurrence below makes
+// two of each and reads the pivots, with one serial chain per thread; z solve
+// at 360x200x150 177 -> 52 us, solve at 128x128x240 274 -> 79 us.
+template <int M, int S, typename St, bool DPP16, int H = 1, bool RAG = false>
 __global__ void __launch_bounds__(512) k_trid_part(St *__restrict__ Wr,
                                                    const int *__restrict__ order, PArgs g)
 {
@@ -217,30 +229,55 @@ __global__ void __launch_bounds__(512) k_trid_part(St *__restrict__ Wr,
     // CS = 3M + 1 puts the P lanes of a column in distinct banks, and a lane's
     // reads are at fixed offsets from one address.
     constexpr int CS = 3 * M + 1;
-    double *cf = tl + (size_t)nz * SW;
+    static_assert(!RAG || H == 1, "ragged tiles are one column group wide");
+    const int nrow = RAG ? P * M : nz;
+    double *cf = tl + (size_t)nrow * SW;
 
-    for (int k = tid; k < nz; k += nthr) {
+    for (int k = tid; k < nrow; k += nthr) {
         const int o = (k / M) * CS + 3 * (k % M);
-        cf[o] = g.a[k];
-        cf[o + 1] = g.c[k];
-        cf[o + 2] = g.bz[k];
+        const bool in = !RAG || k < nz;
+        cf[o] = in ? g.a[k] : 0.0;
+        cf[o + 1] = in ? g.c[k] : 0.0;
+        cf[o + 2] = in ? g.bz[k] : -1.0;  // eigenvalues are <= 0
     }
     // element j of this thread: column st, row kt + j P/H (nthr = SW P/H),
     // at tile_base + toff + j jstride
     const int lPH = lP - (H == 2), st = tid & (SW - 1), kt = tid >> LSW;
     const long long toff = st + kt * plane, jstride = (long long)(P / H) * plane;
+    // RAG: this thread's rows kt + j P below nz are j < nj
+    const int nj = RAG ? (nz - kt + P - 1) >> lP : 0;
     St pre[H * M];
     auto fetch = [&](int tile) {
-        const St *__restrict__ src =
-            Wr + (long long)(tile / g.ntx) * g.nx + (tile % g.ntx) * SW + toff;
+        if constexpr (RAG) {
+            // lanes and rows outside read the last ones inside again
+            const int f = min((tile & ~RAG_EXACT) * SW + st, g.ncol - 1);
+            const St *__restrict__ src = Wr + f + (nj > 0 ? kt : nz - 1) * plane;
+            const long long last = nj > 0 ? (nj - 1) * jstride : 0;
 #pragma unroll
-        for (int j = 0; j < H * M; ++j) pre[j] = src[j * jstride];
+            for (int j = 0; j < M; ++j) pre[j] = src[j < nj ? j * jstride : last];
+        } else {
+            const St *__restrict__ src =
+                Wr + (long long)(tile / g.ntx) * g.nx + (tile % g.ntx) * SW + toff;
+#pragma unroll
+            for (int j = 0; j < H * M; ++j) pre[j] = src[j * jstride];
+        }
     };
     const int s = tid >> lP, p = tid & (P - 1);
     // eigenvalues of this thread's column in each group of a tile, loaded
     // with the tile's values (so one wait covers both)
     double lams[H];
+    int ixs = 0, iys = 0, nixs = 0, niys = 0;  // RAG: its eigenvalue indices, now and next
+    bool zero = false, nzero = false;          // RAG: its column is the (0, 0) mode
     auto load_lams = [&](int tile) {
+        if constexpr (RAG) {
+            const int f = min((tile & ~RAG_EXACT) * SW + s, g.ncol - 1);
+            const int my = f / g.nx, q = f - my * g.nx;
+            nixs = lam_ix(q, my, g.L, g.ny);
+            niys = my <= g.ny - my ? my : g.ny - my;
+            nzero = f == 0;
+            lams[0] = g.lamx[nixs] + g.lamy[niys];
+            return;
+        }
         const int my = tile / g.ntx, qt0 = (tile % g.ntx) * SW;
         const int iy = my <= g.ny - my ? my : g.ny - my;
 #pragma unroll
@@ -262,12 +299,18 @@ __global__ void __launch_bounds__(512) k_trid_part(St *__restrict__ Wr,
     for (int t = blockIdx.x; t < g.ntiles; t += gridDim.x) {
     const int tn = t + (int)gridDim.x;
     const int tile_next = order[tn < g.ntiles ? tn : t];
-    const int my = tile / g.ntx, qt0 = (tile % g.ntx) * SW;
+    const int my = RAG ? 0 : tile / g.ntx, qt0 = RAG ? 0 : (tile % g.ntx) * SW;
     St *__restrict__ base = Wr + (long long)my * g.nx + qt0;
     const int iy = my <= g.ny - my ? my : g.ny - my;
     __syncthreads();  // the previous tile's results have been read from LDS
 #pragma unroll
-    for (int j = 0; j < H * M; ++j) tl[swz(kt + (j << lPH), st, S, SW, M)] = (double)pre[j];
+    for (int j = 0; j < H * M; ++j)
+        tl[swz(kt + (j << lPH), st, S, SW, M)] = !RAG || j < nj ? (double)pre[j] : 0.0;
+    if (RAG) {
+        ixs = nixs;
+        iys = niys;
+        zero = nzero;
+    }
     __syncthreads();
     double lamc[H];
 #pragma unroll
@@ -279,7 +322,7 @@ __global__ void __launch_bounds__(512) k_trid_part(St *__restrict__ Wr,
     for (int h = 0; h < H; ++h) {
     const int q = qt0 + h * S + s;
     const double lam = (H == 1 || h == 0) ? lamc[0] : lamc[H - 1];
-    if (qt0 < g.qx && iy < g.iyx) {
+    if (RAG ? (tile & RAG_EXACT) != 0 : (qt0 < g.qx && iy < g.iyx)) {
         // The reference's recurrences with the stored pivots (low modes, where
         // the block elimination below loses accuracy):
         //   forward  y_k = d_k - m_k y_{k-1},  m_k = a_k / piv_{k-1},
@@ -293,17 +336,25 @@ __global__ void __launch_bounds__(512) k_trid_part(St *__restrict__ Wr,
         const int lane = tid & 63;
         const long long pst = (long long)(g.L + 1) * (g.ny / 2 + 1);
         const double *__restrict__ pc =
-            g.piv + (long long)iy * (g.L + 1) + lam_ix(q, my, g.L, g.ny);
+            RAG ? g.piv + (long long)iys * (g.L + 1) + ixs
+                : g.piv + (long long)iy * (g.L + 1) + lam_ix(q, my, g.L, g.ny);
         const double *__restrict__ cl = cf + p * CS;
         // the lane's rows stay in its LDS slots (registers hold the pivots)
         double pv[M];
 #pragma unroll
-        for (int i = 0; i < M; ++i) pv[i] = pc[(long long)(k0 + i) * pst];
+        for (int i = 0; i < M; ++i)
+            pv[i] = !RAG || k0 + i < nz ? pc[(long long)(k0 + i) * pst] : 1.0;
+        // the lane's row nz - 1, if it has it
+        const int it = RAG ? nz - 1 - k0 : (p == P - 1 ? M - 1 : -1);
+        double ytop = 0.0, ptop = 1.0;
         const double pleft = shfl(pv[M - 1], p > 0 ? lane - 1 : lane);  // pivot of row k0-1
+        // row i has a row below it (the one above row nz - 1, RAG only, must not
+        // be divided into by that row's pivot, which may be zero)
+        auto has = [&](int i) { return k0 + i > 0 && (!RAG || k0 + i < nz); };
         double al = 0.0, be = 1.0;  // lane map: y(last row) = al + be * y(row k0-1)
 #pragma unroll
         for (int i = 0; i < M; ++i) {
-            const double m = (k0 + i > 0) ? cl[3 * i] / (i ? pv[i - 1] : pleft) : 0.0;
+            const double m = has(i) ? cl[3 * i] / (i ? pv[i - 1] : pleft) : 0.0;
             al = tl[pb + i * SW] - m * al;
             be = -m * be;
         }
@@ -319,20 +370,27 @@ __global__ void __launch_bounds__(512) k_trid_part(St *__restrict__ Wr,
         if (p == 0) prev = 0.0;
 #pragma unroll
         for (int i = 0; i < M; ++i) {
-            const double m = (k0 + i > 0) ? cl[3 * i] / (i ? pv[i - 1] : pleft) : 0.0;
+            const double m = has(i) ? cl[3 * i] / (i ? pv[i - 1] : pleft) : 0.0;
             const double yi = tl[pb + i * SW] - m * prev;
             tl[pb + i * SW] = yi;
             prev = yi;
+            if (RAG && i == it) {
+                ytop = yi;
+                ptop = pv[i];
+            }
         }
         // top row: pinned gauge, y / piv, or 0 for an exactly zero pivot
         const bool top = p == P - 1;
-        const bool pin = g.pin_gauge && my == 0 && q == 0;
-        const double bl = pv[M - 1];
-        const double xtop = pin ? 0.0 : (bl != 0.0 ? prev / bl : 0.0);
+        const bool pin = g.pin_gauge && (RAG ? zero : my == 0 && q == 0);
+        if (!RAG) {
+            ytop = prev;
+            ptop = pv[M - 1];
+        }
+        const double xtop = pin ? 0.0 : (ptop != 0.0 ? ytop / ptop : 0.0);
         double ga = 0.0, de = 1.0;  // lane map: x(row k0) = ga + de * x(row k0+M)
 #pragma unroll
         for (int i = M - 1; i >= 0; --i) {
-            if (top && i == M - 1) {
+            if (RAG ? i == it : top && i == M - 1) {
                 ga = xtop;
                 de = 0.0;
             } else {
@@ -353,7 +411,7 @@ __global__ void __launch_bounds__(512) k_trid_part(St *__restrict__ Wr,
 #pragma unroll
         for (int i = M - 1; i >= 0; --i) {
             const double x =
-                (top && i == M - 1) ? xtop : (tl[pb + i * SW] - cl[3 * i + 1] * next) / pv[i];
+                (RAG ? i == it : top && i == M - 1) ? xtop : (tl[pb + i * SW] - cl[3 * i + 1] * next) / pv[i];
             tl[pb + i * SW] = x;
             next = x;
         }
@@ -402,7 +460,8 @@ __global__ void __launch_bounds__(512) k_trid_part(St *__restrict__ Wr,
         // 2. reduced system: equation 2p = block's first row (F), 2p+1 = last (L)
         double fa = ap[0], fg = cp[0], fd = d[0];
         double la = ap[M - 1], lg = cp[M - 1], ld = d[M - 1];
-        if (g.pin_gauge && my == 0 && q == 0 && p == P - 1) {
+        // (RAG: the (0,0) mode is always in an exact-path tile)
+        if (!RAG && g.pin_gauge && my == 0 && q == 0 && p == P - 1) {
             la = 0.0; lg = 0.0; ld = 0.0;  // top value of the (0,0) mode = 0
             fg = 0.0;
         }
@@ -475,9 +534,20 @@ __global__ void __launch_bounds__(512) k_trid_part(St *__restrict__ Wr,
     }
     }  // h
     __syncthreads();
-    St *__restrict__ dst = base + toff;
+    if constexpr (RAG) {
+        const int f = (tile & ~RAG_EXACT) * SW + st;
+        if (f < g.ncol) {
+            St *__restrict__ dst = Wr + f + kt * plane;
 #pragma unroll
-    for (int j = 0; j < H * M; ++j) dst[j * jstride] = (St)tl[swz(kt + (j << lPH), st, S, SW, M)];
+            for (int j = 0; j < M; ++j)
+                if (j < nj) dst[j * jstride] = (St)tl[swz(kt + (j << lPH), st, S, SW, M)];
+        }
+    } else {
+        St *__restrict__ dst = base + toff;
+#pragma unroll
+        for (int j = 0; j < H * M; ++j)
+            dst[j * jstride] = (St)tl[swz(kt + (j << lPH), st, S, SW, M)];
+    }
     tile = tile_next;
     }
 }
@@ -507,10 +577,74 @@ unsigned persistent_grid(const void *fn, int threads, size_t shm, int ntiles)
     return (unsigned)(n < ntiles ? n : ntiles);
 }
 
+// FP64 storage only.  FP32 storage on such grids keeps the streaming solve: with
+// ragged tiles the error left after one refinement sweep is 13 +- 5% larger
+// (150 right-hand sides on six grids; 515 for 773 us at 360x200x150).
+int launch_rag(const pll_ppe_dev *d, void *W, hipStream_t s)
+{
+    using St = double;
+    PArgs g;
+    g.a = d->a;
+    g.c = d->c;
+    g.bz = d->tp.bz;
+    g.lamx = d->tp.lamx;
+    g.lamy = d->tp.lamy;
+    g.piv = d->piv;
+    g.order = d->tp.order;
+    g.L = d->L;
+    g.nx = d->nx;
+    g.ny = d->ny;
+    g.nz = d->nz;
+    g.P = d->tp.P;
+    g.lP = 0;
+    while ((1 << g.lP) < g.P) g.lP++;
+    g.S = d->tp.S;
+    g.ncol = d->nx * d->ny;
+    g.ntx = 1;
+    g.ntiles = (g.ncol + g.S - 1) / g.S;
+    g.pin_gauge = d->pin_gauge;
+    g.qx = g.iyx = 0;
+    const int M = d->tp.M, threads = g.S * g.P;
+    const size_t shm = sizeof(double) * ((size_t)M * g.P * g.S + (3 * (size_t)M + 1) * g.P);
+    if ((1 << g.lP) != g.P || M * g.P < d->nz || threads > 512 || shm > 163840 || !g.order) return -1;
+#define PLL_RAG_L(M_, S_, D_)                                                                      \
+    do {                                                                                           \
+        const void *fn = (const void *)k_trid_part<M_, S_, St, D_, 1, true>;                       \
+        if (shm > 65536 && hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize,     \
+                                               (int)shm) != hipSuccess)                            \
+            return -3;                                                                             \
+        hipLaunchKernelGGL((k_trid_part<M_, S_, St, D_, 1, true>),                                 \
+                           dim3(persistent_grid(fn, threads, shm, g.ntiles)), dim3(threads), shm,  \
+                           s, (St *)W, g.order, g);                                                \
+    } while (0)
+#define PLL_RAG(M_)                                                                                \
+    case M_:                                                                                       \
+        if (g.P == 16 && g.S == 32) PLL_RAG_L(M_, 32, true);                                       \
+        else if (g.S == 32) PLL_RAG_L(M_, 32, false);                                              \
+        else if (g.S == 16) PLL_RAG_L(M_, 16, false);                                              \
+        else if (g.S == 8) PLL_RAG_L(M_, 8, false);                                                \
+        else return -5;                                                                            \
+        break;
+    switch (M) {
+        PLL_RAG(4)
+        PLL_RAG(6)
+        PLL_RAG(8)
+        PLL_RAG(10)
+        PLL_RAG(12)
+        PLL_RAG(14)
+        PLL_RAG(16)
+        default: return -5;
+    }
+#undef PLL_RAG
+#undef PLL_RAG_L
+    return hipGetLastError() == hipSuccess ? 0 : -3;
+}
+
 template <typename St, typename C>
 int launch_trid(const pll_ppe_dev *d, void *W, hipStream_t s)
 {
-    if (d->tp.P > 0) {
+    if (d->tp.rag && sizeof(St) == sizeof(double)) return launch_rag(d, W, s);
+    if (d->tp.P > 0 && !d->tp.rag) {
         // FP32 storage with wide tiles: H = 2 groups of S columns per tile
         const int H = ((sizeof(St) == sizeof(float) ? d->tp.h32 : d->tp.h64) == 2) ? 2 : 1;
         // H = 2: FP32 storage at S = 16 and 32, FP64 storage at S = 16 only (FP64
@@ -608,6 +742,8 @@ int launch_trid(const pll_ppe_dev *d, void *W, hipStream_t s)
 }
 
 }  // namespace
+
+extern "C" int pll_trid_rag_exact(void) { return RAG_EXACT; }
 
 extern "C" int pll_trid_part_supported(int M) { return M == 4 || M == 8 || M == 12 || M == 16; }
 

@@ -176,3 +176,51 @@ def test_window_gradient_vs_pieces(cuda, shape, forced, every):
     for q, w, w2 in zip(got, grad, again):
         assert float((q - w).abs().max()) <= 1e-11 * top
         assert torch.equal(q, w2)
+
+
+# z solve on ragged tiles: every rows-per-lane count with full and short last
+# lanes, 2 to 64 lanes per column, plane sizes that are no multiple of a tile
+# (nx ny = 24, 98 x 42, ...), tiles spanning several y rows
+@pytest.mark.parametrize("shape,bc", [
+    ((4, 6, 2), "NN"), ((8, 6, 9), "NN"), ((10, 14, 13), "ND"), ((24, 16, 50), "NN"),
+    ((98, 42, 33), "NN"), ((36, 20, 65), "DD"), ((40, 12, 81), "NN"), ((20, 10, 127), "NN"),
+    ((28, 18, 150), "NN"), ((360, 20, 180), "NN"), ((12, 30, 200), "ND"), ((60, 8, 250), "NN"),
+    ((20, 12, 255), "NN"), ((24, 10, 257), "NN"), ((12, 14, 400), "NN"), ((8, 6, 512), "NN"),
+    ((16, 6, 700), "NN"), ((64, 10, 1024), "NN")])
+def test_ragged_z_solve(orc, cuda, shape, bc, monkeypatch):
+    """The partitioned solve on ragged tiles against the oracle (1e-12, the
+    solve's tolerance), its transpose against the streaming recurrence (1e-12);
+    the refined form keeps the streaming solve on such grids (bit-identical)."""
+    import torch
+    from powerllel_channel_amd import PoissonSolver
+    from powerllel_channel_amd.mesh import Grid
+    nx, ny, nz = shape
+    print(f"[ragged z solve] {shape} {bc}", flush=True)
+    g = Grid(nx, ny, nz, 6.0, 3.0, 2.0, 3.0 if nz < 300 else 2.0)
+    rng = np.random.default_rng(11)
+    f = rng.standard_normal(g.shape)
+    wz = g.dzf[1:-1]
+    inner = (slice(1, -1),) * 3
+    f[inner] -= (f[inner].sum(axis=(1, 2)) * wz).sum() / (wz.sum() * nx * ny)
+
+    def solver():
+        return PoissonSolver(nx, ny, nz, g.dx, g.dy, g.dzf, bctype_z=bc)
+    monkeypatch.setenv("PLL_TRID_RAG", "1")
+    rag = solver()
+    monkeypatch.delenv("PLL_TRID_RAG")
+    monkeypatch.setenv("PLL_TRID_STREAMING", "1")
+    streaming = solver()
+    monkeypatch.delenv("PLL_TRID_STREAMING")
+    ref = f.copy()
+    orc.OraclePPE(nx, ny, nz, g.dx, g.dy, g.dzf, bc=("PP", "PP", bc), pin_gauge=True).solve(ref)
+    p, q = _dev(torch, cuda, f, f)
+    rag.solve(p)
+    assert np.abs(p.cpu().numpy() - ref)[inner].max() <= 1e-12 * np.abs(ref[inner]).max()
+    for solve, tol in (("solve_adjoint", 1e-12), ("solve_refined", 0.0)):
+        arg = (1,) if solve == "solve_refined" else ()
+        p, q = _dev(torch, cuda, f, f)
+        getattr(rag, solve)(p, *arg)
+        getattr(streaming, solve)(q, *arg)
+        a, b = p[inner], q[inner]
+        assert float((a - b).abs().max()) <= tol * float(b.abs().max()), solve
+        assert torch.equal(p[0], torch.from_numpy(f[0]).to(cuda))
