@@ -55,9 +55,9 @@ struct Proj {
 struct Tiles {
     int ntx, nty, nkc, kc;
     int xcd;
-    // Mean_h partials are those of the RK2 kernel: one per 64 x 4 x kc tile,
-    // at that kernel's workgroup index
-    int nty4, xcd4;
+    // Mean_h partials are those of the RK2 kernel: one per 64 x 4 x kc4 tile
+    // (kc a multiple of kc4), at that kernel's workgroup index
+    int nty4, nkc4, kc4, xcd4;
 };
 
 // Fluxes through the upper z face of a cell, carried from plane k to plane
@@ -185,7 +185,8 @@ __device__ __forceinline__ ZFlux rhs_tile(const G &g, const ZMet &z, const doubl
 // at 128 registers for 16 waves, which spills.
 constexpr int TY = 12;
 
-template <bool PROJ, bool MEAN, bool BODY = !PROJ>
+// SUB: the chunk holds several of the partials' chunks (kc > kc4).
+template <bool PROJ, bool MEAN, bool SUB, bool BODY = !PROJ>
 __global__ void __launch_bounds__(64 * TY, 3)
 k_rk12(G g, Tiles t, const double *__restrict__ qu, const double *__restrict__ qv,
        const double *__restrict__ qw, double *__restrict__ ou, double *__restrict__ ov,
@@ -322,6 +323,31 @@ k_rk12(G g, Tiles t, const double *__restrict__ qu, const double *__restrict__ q
     double oldu = 0.0, oldv = 0.0, oldw = 0.0;
     if (MEAN) red[tid] = red[NT + tid] = 0.0;
 
+    const bool own = i0 + lx + 1 <= g.nx && j0 + ly + 1 <= g.ny;
+    // the partials of a chunk of kc4 planes that ends with plane k, in the order
+    // of the RK2 kernel's reduction
+    auto emit = [&](int k) {
+        if (!own) red[tid] = red[NT + tid] = 0.0;
+        __syncthreads();
+        const int q = tid & 255, base = tid - q;
+        for (int h = 128; h > 0; h >>= 1) {
+            if (q < h) {
+                red[base + q] += red[base + q + h];
+                red[NT + base + q] += red[NT + base + q + h];
+            }
+            __syncthreads();
+        }
+        const int ty4 = ty * (TY / 4) + (tid >> 8);
+        if (q == 0 && ty4 < t.nty4) {
+            const int nb = t.ntx * t.nty4 * t.nkc4;
+            int b4 = ((k - 1) / t.kc4 * t.nty4 + ty4) * t.ntx + tx;
+            if (t.xcd4) b4 = (b4 % (nb >> 3)) * 8 + b4 / (nb >> 3);
+            mpart[b4] = (fmask & 1) ? red[base] : 0.0;
+            mpart[nb + b4] = (fmask & 2) ? red[NT + base] : 0.0;
+        }
+        if (SUB) red[tid] = red[NT + tid] = 0.0;
+    };
+
     // RK1 stage of plane kb (slot PAR) into LDS; MODE 2: then RK2 of plane kb - 1,
     // 1: its lower z fluxes, 0: neither; 3: as 2 with kb the wall's ghost plane
     // nz + 1.  Loads of plane kb + 2 throughout.
@@ -427,6 +453,7 @@ k_rk12(G g, Tiles t, const double *__restrict__ qu, const double *__restrict__ q
         oldw = now;
         put(kb + 2, a);
         __syncthreads();
+        if (SUB && mode >= 2 && ((kb - 1) % t.kc4 == 0 || kb - 1 == nz)) emit(kb - 1);
     };
     using I0 = std::integral_constant<int, 0>;
     using I1 = std::integral_constant<int, 1>;
@@ -451,29 +478,7 @@ k_rk12(G g, Tiles t, const double *__restrict__ qu, const double *__restrict__ q
         else
             iter(kb, I3{}, I0{});
     }
-
-    if (MEAN) {
-        // per 64 x 4 tile, in the order of the RK2 kernel's reduction
-        const bool own = i0 + lx + 1 <= g.nx && j0 + ly + 1 <= g.ny;
-        if (!own) red[tid] = red[NT + tid] = 0.0;
-        __syncthreads();
-        const int q = tid & 255, base = tid - q;
-        for (int h = 128; h > 0; h >>= 1) {
-            if (q < h) {
-                red[base + q] += red[base + q + h];
-                red[NT + base + q] += red[NT + base + q + h];
-            }
-            __syncthreads();
-        }
-        const int ty4 = ty * (TY / 4) + (tid >> 8);
-        if (q == 0 && ty4 < t.nty4) {
-            const int nb = t.ntx * t.nty4 * t.nkc;
-            int b4 = (kc * t.nty4 + ty4) * t.ntx + tx;
-            if (t.xcd4) b4 = (b4 % (nb >> 3)) * 8 + b4 / (nb >> 3);
-            mpart[b4] = (fmask & 1) ? red[base] : 0.0;
-            mpart[nb + b4] = (fmask & 2) ? red[NT + base] : 0.0;
-        }
-    }
+    if (MEAN && !SUB) emit(k1);
 }
 
 inline int ok() { return hipGetLastError() == hipSuccess ? 0 : -3; }
@@ -491,23 +496,41 @@ extern "C" int pll_launch_rk12(const pll_grid_dev *gd, const double *const q[3],
     Tiles t;
     t.ntx = rk[0];
     t.nty4 = rk[1];
-    t.nkc = rk[2];
-    t.kc = rk[3];
+    t.nkc4 = rk[2];
+    t.kc4 = rk[3];
     t.xcd4 = rk[4];
     t.nty = (g.ny + TY - 1) / TY;
-    const long long nb = (long long)t.ntx * t.nty * t.nkc;
+    // Planes per workgroup: kc4, or the multiple of it with the least rounds of
+    // the 256 CUs (one workgroup each) times planes per round, a chunk costing
+    // three planes more than it has (the RK1 stage below and above it, two
+    // planes of loads before the first), if that saves a tenth: small grids,
+    // whose RK2 chunks are a few planes.  Per step of a run, kc4 planes against
+    // this: 240x140x90 (4, 20 planes) 275 -> 244 us, 96x96x96 (2, 6) 126 -> 109,
+    // 64x64x64 (1, 2) 65 -> 58.  SUB's partial sums inside the loop spill, so
+    // smaller gains are none (192x192x128, 384x384x192: 2 to 4% slower).
+    const long long cols = (long long)t.ntx * t.nty;
+    auto cost = [&](int kc) { return (cols * ((g.nz + kc - 1) / kc) + 255) / 256 * (kc + 3); };
+    const bool m = mpart && fmask;
+    t.kc = t.kc4;
+    for (int kc = 2 * t.kc4; kc < g.nz + t.kc4; kc += t.kc4)
+        if (cost(kc) < cost(t.kc)) t.kc = kc;
+    if (10 * cost(t.kc) > 9 * cost(t.kc4)) t.kc = t.kc4;
+    const bool sub = m && t.kc > t.kc4;
+    t.nkc = (g.nz + t.kc - 1) / t.kc;
+    const long long nb = cols * t.nkc;
     if (nb > 0x7fffffffLL || g.sz > 0x1fffffffLL || (p != nullptr) == (body != nullptr)) return -1;
     t.xcd = nb % 8 == 0;
     const Body fb = body ? Body{body[0], body[1], body[2]} : Body{nullptr, nullptr, nullptr};
     const Proj pr{p, g.dt * g.dx_inv, g.dt * g.dy_inv, (p && mean) ? fmask : 0, vfu, vfv, mean};
-    const bool m = mpart && fmask;
-#define PLL_RK12(P_, M_)                                                                       \
-    hipLaunchKernelGGL((k_rk12<P_, M_>), dim3((unsigned)nb), dim3(64 * TY), 0, s, g, t, q[0],  \
+#define PLL_RK12(P_, M_, S_)                                                                      \
+    hipLaunchKernelGGL((k_rk12<P_, M_, S_>), dim3((unsigned)nb), dim3(64 * TY), 0, s, g, t, q[0], \
                        q[1], q[2], o[0], o[1], o[2], mpart, m ? fmask : 0, fb, pr)
-    if (p && m) PLL_RK12(true, true);
-    else if (p) PLL_RK12(true, false);
-    else if (m) PLL_RK12(false, true);
-    else PLL_RK12(false, false);
+    if (p && sub) PLL_RK12(true, true, true);
+    else if (p && m) PLL_RK12(true, true, false);
+    else if (p) PLL_RK12(true, false, false);
+    else if (sub) PLL_RK12(false, true, true);
+    else if (m) PLL_RK12(false, true, false);
+    else PLL_RK12(false, false, false);
 #undef PLL_RK12
     return ok();
 }
