@@ -25,6 +25,7 @@ ARCH = "gfx950"
 
 HIP_SOURCES = {
     # one rounding per transform whatever the I/O policy: no automatic contraction
+    # (four objects of the one file, see FFT_UNITS)
     "fft_kernels.hip": ["-ffp-contract=off"],
     "trid_kernels.hip": [],
     "resid_kernels.hip": [],
@@ -36,6 +37,8 @@ HIP_SOURCES = {
     # allocation-free calcMaxDiv: its static device scratch array and launcher
     "noalloc.hip": [],
 }
+# fft_kernels.hip compiles in parts (its launchers instantiate some 500 kernels)
+FFT_UNITS = 4
 C_SOURCES = ["ppe.c", "channel.c", "adjoint.c", "hostcopy.c"]
 
 HIPFLAGS = [
@@ -89,14 +92,17 @@ def build(verbose: bool = False) -> str:
     jobs = []
     objs = []
     for src, extra in HIP_SOURCES.items():
-        obj = os.path.join(BUILD, src.replace(".hip", ".o"))
-        objs.append(obj)
-        jobs.append([hipcc, *HIPFLAGS, *extra, "-c", os.path.join(CSRC, src), "-o", obj])
+        units = range(1, FFT_UNITS + 1) if src == "fft_kernels.hip" else [0]
+        for u in units:
+            obj = os.path.join(BUILD, src.replace(".hip", f"{u or ''}.o"))
+            objs.append(obj)
+            jobs.append([hipcc, *HIPFLAGS, *extra, *([f"-DPLL_FFT_UNIT={u}"] if u else []), "-c",
+                         os.path.join(CSRC, src), "-o", obj])
     for src in C_SOURCES:
         obj = os.path.join(BUILD, src.replace(".c", ".o"))
         objs.append(obj)
         jobs.append(["gcc", *CFLAGS, "-c", os.path.join(CSRC, src), "-o", obj])
-    with ThreadPoolExecutor(max_workers=min(4, len(jobs))) as ex:
+    with ThreadPoolExecutor(max_workers=min(6, len(jobs))) as ex:
         outs = list(ex.map(_run, jobs))
     if verbose:
         for o in outs:

@@ -254,13 +254,19 @@ struct Dft<11, DIR> : DftOdd<11, DIR> {};
 template <int DIR>
 struct Dft<13, DIR> : DftOdd<13, DIR> {};
 
+// b mod Ns, mag = ceil(2^32 / Ns) (for Ns = 1, where that is 2^32, 0: mag wraps)
+__device__ __forceinline__ int mod_ns(int b, int Ns, unsigned mag)
+{
+    return Ns == 1 ? 0 : b - (int)__umulhi((unsigned)b, mag) * Ns;
+}
+
 // One Stockham radix-R stage.  Thread t holds elements t + e*T (e < E).
 // Butterfly b = t + q*T (q < E/R) takes elements b + r*L/R = slot q + r*E/R,
 // twiddles them by w^(r*k) (k = b mod Ns, w = exp(DIR 2 pi i/(Ns R))) and
 // writes output r to position (b - k)*R + k + r*Ns.  In the last stage that
 // position is element t + (q + r*E/R)*T, i.e. the same register slot.
 template <int R, int E, int DIR, typename V>
-__device__ __forceinline__ void stage(V (&v)[E], int t, int T, int Ns, int twstep,
+__device__ __forceinline__ void stage(V (&v)[E], int t, int T, int Ns, unsigned mag, int twstep,
                                       const V *__restrict__ tw, V *lds, bool last)
 {
     if constexpr (E % R == 0) {
@@ -268,7 +274,7 @@ __device__ __forceinline__ void stage(V (&v)[E], int t, int T, int Ns, int twste
 #pragma unroll
         for (int q = 0; q < Q; ++q) {
             const int b = t + q * T;
-            const int k = b % Ns;
+            const int k = mod_ns(b, Ns, mag);
             V x[R];
 #pragma unroll
             for (int r = 0; r < R; ++r) x[r] = v[q + r * Q];
@@ -298,7 +304,7 @@ __device__ __forceinline__ void stage(V (&v)[E], int t, int T, int Ns, int twste
 // ceil(E/R) of them), reads their R inputs each, and after a barrier writes
 // the outputs back to LDS at the Stockham positions.
 template <int R, int E, int DIR, typename V>
-__device__ __forceinline__ void stage_lds(int t, int T, int L, int Ns, int twstep,
+__device__ __forceinline__ void stage_lds(int t, int T, int L, int Ns, unsigned mag, int twstep,
                                           const V *__restrict__ tw, V *lds)
 {
     constexpr int QM = (E + R - 1) / R;
@@ -308,7 +314,7 @@ __device__ __forceinline__ void stage_lds(int t, int T, int L, int Ns, int twste
     for (int q = 0; q < QM; ++q) {
         const int b = t + q * T;
         if (b < nb) {
-            const int k = b % Ns;
+            const int k = mod_ns(b, Ns, mag);
 #pragma unroll
             for (int r = 0; r < R; ++r) x[q][r] = lds[b + r * nb];
             if (Ns > 1) {
@@ -327,7 +333,7 @@ __device__ __forceinline__ void stage_lds(int t, int T, int L, int Ns, int twste
     for (int q = 0; q < QM; ++q) {
         const int b = t + q * T;
         if (b < nb) {
-            const int k = b % Ns;
+            const int k = mod_ns(b, Ns, mag);
             const int base = (b - k) * R + k;
 #pragma unroll
             for (int r = 0; r < R; ++r) lds[base + r * Ns] = x[q][r];
@@ -340,9 +346,9 @@ __device__ __forceinline__ void stage_lds(int t, int T, int L, int Ns, int twste
 // any other radix runs from LDS, and as the last stage brings the result
 // back into registers.
 template <int R, int E, int DIR, typename V>
-__device__ __forceinline__ void stage_rt(V (&v)[E], int t, int T, int L, int Ns, int twstep,
-                                         const V *__restrict__ tw, V *lds, bool from_lds,
-                                         bool last)
+__device__ __forceinline__ void stage_rt(V (&v)[E], int t, int T, int L, int Ns, unsigned mag,
+                                         int twstep, const V *__restrict__ tw, V *lds,
+                                         bool from_lds, bool last)
 {
     if constexpr (E % R == 0) {
         if (from_lds) {
@@ -351,14 +357,14 @@ __device__ __forceinline__ void stage_rt(V (&v)[E], int t, int T, int L, int Ns,
             for (int e = 0; e < E; ++e) v[e] = lds[t + e * T];
             __syncthreads();
         }
-        stage<R, E, DIR>(v, t, T, Ns, twstep, tw, lds, last);
+        stage<R, E, DIR>(v, t, T, Ns, mag, twstep, tw, lds, last);
     } else {
         if (!from_lds) {
 #pragma unroll
             for (int e = 0; e < E; ++e) lds[t + e * T] = v[e];
         }
         __syncthreads();
-        stage_lds<R, E, DIR>(t, T, L, Ns, twstep, tw, lds);
+        stage_lds<R, E, DIR>(t, T, L, Ns, mag, twstep, tw, lds);
         if (last) {
             __syncthreads();
 #pragma unroll
@@ -371,7 +377,9 @@ __device__ __forceinline__ void stage_rt(V (&v)[E], int t, int T, int L, int Ns,
 // the input; on exit it holds elements t + e*T of the output.  `lds` is this
 // transform's LDS segment (>= L points).  twscale = (table length) / L.
 // Every thread of the workgroup must call it (it contains barriers).
-template <int E, int DIR, typename V>
+// BIG: with the radices 11 and 13, whose butterflies need so many registers that
+// kernels without them hold twice the waves.
+template <int E, int DIR, bool BIG, typename V>
 __device__ __forceinline__ void fft_run(V (&v)[E], int t, const pll_fftplan &P,
                                         const V *__restrict__ tw, int twscale, V *lds)
 {
@@ -381,17 +389,23 @@ __device__ __forceinline__ void fft_run(V (&v)[E], int t, const pll_fftplan &P,
         const int R = P.rad[s];
         const bool last = (s == P.nst - 1), fl = s > 0;
         const int twstep = twscale * (L / (Ns * R));
+        const unsigned mag = P.mag[s];
         switch (R) {
-            case 2: stage_rt<2, E, DIR>(v, t, T, L, Ns, twstep, tw, lds, fl, last); break;
-            case 3: stage_rt<3, E, DIR>(v, t, T, L, Ns, twstep, tw, lds, fl, last); break;
-            case 4: stage_rt<4, E, DIR>(v, t, T, L, Ns, twstep, tw, lds, fl, last); break;
-            case 5: stage_rt<5, E, DIR>(v, t, T, L, Ns, twstep, tw, lds, fl, last); break;
-            case 6: stage_rt<6, E, DIR>(v, t, T, L, Ns, twstep, tw, lds, fl, last); break;
-            case 7: stage_rt<7, E, DIR>(v, t, T, L, Ns, twstep, tw, lds, fl, last); break;
-            case 8: stage_rt<8, E, DIR>(v, t, T, L, Ns, twstep, tw, lds, fl, last); break;
-            case 11: stage_rt<11, E, DIR>(v, t, T, L, Ns, twstep, tw, lds, fl, last); break;
-            case 13: stage_rt<13, E, DIR>(v, t, T, L, Ns, twstep, tw, lds, fl, last); break;
-            default: break;
+            case 2: stage_rt<2, E, DIR>(v, t, T, L, Ns, mag, twstep, tw, lds, fl, last); break;
+            case 3: stage_rt<3, E, DIR>(v, t, T, L, Ns, mag, twstep, tw, lds, fl, last); break;
+            case 4: stage_rt<4, E, DIR>(v, t, T, L, Ns, mag, twstep, tw, lds, fl, last); break;
+            case 5: stage_rt<5, E, DIR>(v, t, T, L, Ns, mag, twstep, tw, lds, fl, last); break;
+            case 6: stage_rt<6, E, DIR>(v, t, T, L, Ns, mag, twstep, tw, lds, fl, last); break;
+            case 7: stage_rt<7, E, DIR>(v, t, T, L, Ns, mag, twstep, tw, lds, fl, last); break;
+            case 8: stage_rt<8, E, DIR>(v, t, T, L, Ns, mag, twstep, tw, lds, fl, last); break;
+            default:
+                if constexpr (BIG) {
+                    if (R == 11)
+                        stage_rt<11, E, DIR>(v, t, T, L, Ns, mag, twstep, tw, lds, fl, last);
+                    else if (R == 13)
+                        stage_rt<13, E, DIR>(v, t, T, L, Ns, mag, twstep, tw, lds, fl, last);
+                }
+                break;
         }
         Ns *= R;
     }
@@ -474,6 +488,7 @@ __device__ __forceinline__ void stages_ct(V (&v)[E], int t, const V *__restrict_
 template <int L_, int E_, int... Rs>
 struct CtFFT {
     static constexpr int E = E_;
+    static constexpr bool kBig = false;
     static constexpr int kT = L_ / E_;  // threads per row
     static constexpr bool kSplit = true;
     static __device__ __forceinline__ int threads(const pll_fftplan &) { return L_ / E_; }
@@ -487,9 +502,10 @@ struct CtFFT {
     }
 };
 
-template <int E_>
+template <int E_, bool BIG>
 struct RtFFT {
     static constexpr int E = E_;
+    static constexpr bool kBig = BIG;
     static constexpr int kT = 0;  // threads per row known at run time only
     static constexpr bool kSplit = false;
     static __device__ __forceinline__ int threads(const pll_fftplan &P) { return P.T; }
@@ -498,7 +514,7 @@ struct RtFFT {
     static __device__ __forceinline__ void run(V (&v)[E_], int t, const pll_fftplan &P,
                                                const V *__restrict__ tw, void *lds)
     {
-        fft_run<E_, DIR>(v, t, P, tw, TWSCALE, reinterpret_cast<V *>(lds));
+        fft_run<E_, DIR, BIG>(v, t, P, tw, TWSCALE, reinterpret_cast<V *>(lds));
     }
 };
 
@@ -938,6 +954,15 @@ struct YArgs {
 // FP64 kernels with 12 or more points per thread need more than 128 VGPRs,
 // so their workgroups are capped at 256 threads; FP32 values take half the
 // registers.
+// Waves per SIMD asked of the FP64 kernels with runtime plans (registers are
+// capped accordingly): three for 8 and 12 points per thread without the large
+// radices, which take 166 to 223 registers uncapped.
+template <class F, typename V>
+constexpr int waves_f()
+{
+    return F::kT == 0 && !F::kBig && sizeof(V) == sizeof(double2) && (F::E == 8 || F::E == 12) ? 3 : 1;
+}
+
 template <int E, typename V = double2>
 constexpr int max_threads()
 {
@@ -959,7 +984,7 @@ __device__ __forceinline__ V tw_m(const V *__restrict__ tw, V wt, int e, int T)
 }
 
 template <class F, typename V, class Src>
-__global__ void __launch_bounds__((max_threads_f<F, V>()))
+__global__ void __launch_bounds__((max_threads_f<F, V>()), (waves_f<F, V>()))
 k_xfwd(Src src, V *__restrict__ W, const V *__restrict__ twr, XArgs<V> a)
 {
     using S = typename Sc<V>::T;
@@ -1068,7 +1093,7 @@ k_xfwd(Src src, V *__restrict__ W, const V *__restrict__ twr, XArgs<V> a)
 // x backward: packed half spectrum rows -> real rows * norm, stored by Dst;
 // with NORM, also the workgroup's max |value| and max |result|.
 template <class F, typename V, class Dst, bool NORM = false>
-__global__ void __launch_bounds__((max_threads_f<F, V>()))
+__global__ void __launch_bounds__((max_threads_f<F, V>()), (waves_f<F, V>()))
 k_xbwd(const V *__restrict__ W, Dst dst, const V *__restrict__ twr, XArgs<V> a)
 {
     using S = typename Sc<V>::T;
@@ -1235,7 +1260,7 @@ __global__ void __launch_bounds__(256) k_norm_final(const double *__restrict__ p
 
 // y forward, in place on W: tile of `cols` adjacent columns of one k-plane.
 template <class F, typename V>
-__global__ void __launch_bounds__((max_threads_f<F, V>()))
+__global__ void __launch_bounds__((max_threads_f<F, V>()), (waves_f<F, V>()))
 k_yfwd(V *__restrict__ W, YArgs<V> a)
 {
     using S = typename Sc<V>::T;
@@ -1284,7 +1309,7 @@ k_yfwd(V *__restrict__ W, YArgs<V> a)
 }
 
 template <class F, typename V>
-__global__ void __launch_bounds__((max_threads_f<F, V>()))
+__global__ void __launch_bounds__((max_threads_f<F, V>()), (waves_f<F, V>()))
 k_ybwd(V *__restrict__ W, YArgs<V> a)
 {
     using S = typename Sc<V>::T;
@@ -1445,23 +1470,22 @@ int launch_y(bool fwd, const pll_ppe_dev *d, const void *tw, void *W, hipStream_
 }
 
 // Compile-time plans for the transform lengths of the production grids
-// (x: L = nx/2, y: L = ny).  For a length listed twice the first entry is the
-// default (fewer registers, more waves per SIMD: faster on gfx950 as measured)
-// and PLL_FFT_E selects the other.
+// (x: L = nx/2, y: L = ny).  Points per thread: 12 or 8 (24 needs 228 registers,
+// two waves per SIMD), which also puts enough lanes on a row: at L = 96 with 24
+// points its 4 lanes read 64 bytes at a time (solve at 192x192x128 110 us; 89
+// with 12 points, 8 lanes; 96x96x96 52 -> 46 us with 12 points at L = 48 and 96),
+// at L = 32 8 lanes of 4 points read 128 (64x64x64 24.8 -> 23.6 us).
 #define PLL_CT_PLANS(X)                 \
-    X(32, 8, 8, 4)                      \
-    X(48, 24, 8, 6)                     \
+    X(32, 4, 4, 4, 2)                   \
+    X(48, 12, 4, 4, 3)                  \
     X(64, 8, 8, 8)                      \
-    X(96, 24, 8, 4, 3)                  \
+    X(96, 12, 4, 4, 6)                  \
     X(128, 8, 8, 8, 2)                  \
     X(192, 12, 4, 4, 4, 3)              \
-    X(192, 24, 8, 8, 3)                 \
     X(256, 8, 8, 8, 4)                  \
     X(384, 12, 4, 4, 4, 6)              \
-    X(384, 24, 8, 8, 6)                 \
     X(512, 8, 8, 8, 8)                  \
     X(768, 12, 4, 4, 4, 4, 3)           \
-    X(768, 24, 8, 8, 4, 3)              \
     X(1024, 8, 8, 8, 8, 2)
 
 template <typename G>
@@ -1471,22 +1495,36 @@ int dispatch_plan(const pll_fftplan &P, G &&g)
     if (P.L == L_ && P.E == E_) return g(CtFFT<L_, E_, __VA_ARGS__>{});
     PLL_CT_PLANS(PLL_CT_CASE)
 #undef PLL_CT_CASE
+    bool big = false;
+    for (int i = 0; i < P.nst; ++i) big = big || P.rad[i] > 8;
+#define PLL_RT_CASE(E_) \
+    case E_: return big ? g(RtFFT<E_, true>{}) : g(RtFFT<E_, false>{});
     switch (P.E) {
-        case 2: return g(RtFFT<2>{});
-        case 3: return g(RtFFT<3>{});
-        case 4: return g(RtFFT<4>{});
-        case 5: return g(RtFFT<5>{});
-        case 6: return g(RtFFT<6>{});
-        case 7: return g(RtFFT<7>{});
-        case 8: return g(RtFFT<8>{});
-        case 12: return g(RtFFT<12>{});
-        case 24: return g(RtFFT<24>{});
+        PLL_RT_CASE(2)
+        PLL_RT_CASE(3)
+        PLL_RT_CASE(4)
+        PLL_RT_CASE(5)
+        PLL_RT_CASE(6)
+        PLL_RT_CASE(7)
+        PLL_RT_CASE(8)
+        PLL_RT_CASE(12)
+        PLL_RT_CASE(24)
         default: return -5;
     }
+#undef PLL_RT_CASE
 }
 
 }  // namespace
 
+// The launchers come in four groups, each its own object file (PLL_FFT_UNIT = 1
+// to 4; undefined: all), so that they compile side by side.
+#ifdef PLL_FFT_UNIT
+#define PLL_UNIT(n) (PLL_FFT_UNIT == n)
+#else
+#define PLL_UNIT(n) 1
+#endif
+
+#if PLL_UNIT(1)
 extern "C" int pll_fft_supported_E(int E)
 {
     return E == 2 || E == 3 || E == 4 || E == 5 || E == 6 || E == 7 || E == 8 || E == 12 ||
@@ -1533,7 +1571,6 @@ extern "C" int pll_launch_xfwd(const pll_ppe_dev *d, const double *p, void *W, h
 // The chunked transforms of host-pointer solves are their own instantiations
 // (same code), so that kernel traces keep them apart from whole-array ones.
 struct SrcHalo64Rows : SrcHalo64 {};
-struct DstHalo64Rows : DstHalo64 {};
 
 extern "C" int pll_launch_xfwd_rows(const pll_ppe_dev *d, const double *p, void *W,
                                     long long row0, long long row1, hipStream_t s)
@@ -1563,6 +1600,8 @@ extern "C" int pll_launch_xfwd_div(const pll_ppe_dev *d, const pll_div_src *q, v
     });
 }
 
+#endif
+#if PLL_UNIT(2)
 extern "C" int pll_launch_xbwd(const pll_ppe_dev *d, const void *W, double *p, hipStream_t s)
 {
     const DstHalo64 dst{p, (long long)(d->nx + 2) * (d->ny + 2), d->nx + 2};
@@ -1570,6 +1609,8 @@ extern "C" int pll_launch_xbwd(const pll_ppe_dev *d, const void *W, double *p, h
         return launch_xb<decltype(f), double2>(d, d->tw_x, W, dst, s);
     });
 }
+
+struct DstHalo64Rows : DstHalo64 {};
 
 extern "C" int pll_launch_xbwd_rows(const pll_ppe_dev *d, const void *W, double *p,
                                     long long row0, long long row1, hipStream_t s)
@@ -1601,6 +1642,8 @@ extern "C" int pll_launch_ybwd(const pll_ppe_dev *d, void *W, hipStream_t s)
     return dispatch_plan(d->py, [&](auto f) { return launch_y<decltype(f), double2>(false, d, d->tw_y, W, s); });
 }
 
+#endif
+#if PLL_UNIT(3)
 // ---- FP32 solve of the refined form
 extern "C" int pll_launch_xfwd32(const pll_ppe_dev *d, int src_kind, const void *src, void *W32,
                                  hipStream_t s)
@@ -1614,28 +1657,6 @@ extern "C" int pll_launch_xfwd32(const pll_ppe_dev *d, int src_kind, const void 
     const SrcDense32 in{(const float *)src};
     return dispatch_plan(d->px, [&](auto f) {
         return launch_xf<decltype(f), float2>(d, d->tw_x32, in, W32, s);
-    });
-}
-
-extern "C" int pll_launch_xbwd32(const pll_ppe_dev *d, int dst_kind, const void *W32,
-                                 double *p_halo, double *P_dense, const double *eps,
-                                 hipStream_t s)
-{
-    const long long off1 = (long long)(d->nx + 2) * (d->ny + 2), off2 = d->nx + 2;
-    return dispatch_plan(d->px, [&](auto f) {
-        using F = decltype(f);
-        switch (dst_kind) {
-            case PLL_DST_HALO_SET:
-                return launch_xb<F, float2>(d, d->tw_x32, W32, DstHalo64{p_halo, off1, off2}, s);
-            case PLL_DST_DENSE_SET:
-                return launch_xb<F, float2>(d, d->tw_x32, W32, DstDenseSet{P_dense}, s);
-            case PLL_DST_DENSE_ADD:
-                return launch_xb<F, float2>(d, d->tw_x32, W32, DstDenseAdd{P_dense}, s);
-            case PLL_DST_HALO_FROM_DENSE:
-                return launch_xb<F, float2>(d, d->tw_x32, W32,
-                                            DstHaloFromDense{p_halo, off1, off2, P_dense, eps}, s);
-            default: return -1;
-        }
     });
 }
 
@@ -1674,6 +1695,30 @@ extern "C" int pll_launch_xfwd32_resid(const pll_ppe_dev *d, const double *f, in
     });
 }
 
+#endif
+#if PLL_UNIT(4)
+extern "C" int pll_launch_xbwd32(const pll_ppe_dev *d, int dst_kind, const void *W32,
+                                 double *p_halo, double *P_dense, const double *eps,
+                                 hipStream_t s)
+{
+    const long long off1 = (long long)(d->nx + 2) * (d->ny + 2), off2 = d->nx + 2;
+    return dispatch_plan(d->px, [&](auto f) {
+        using F = decltype(f);
+        switch (dst_kind) {
+            case PLL_DST_HALO_SET:
+                return launch_xb<F, float2>(d, d->tw_x32, W32, DstHalo64{p_halo, off1, off2}, s);
+            case PLL_DST_DENSE_SET:
+                return launch_xb<F, float2>(d, d->tw_x32, W32, DstDenseSet{P_dense}, s);
+            case PLL_DST_DENSE_ADD:
+                return launch_xb<F, float2>(d, d->tw_x32, W32, DstDenseAdd{P_dense}, s);
+            case PLL_DST_HALO_FROM_DENSE:
+                return launch_xb<F, float2>(d, d->tw_x32, W32,
+                                            DstHaloFromDense{p_halo, off1, off2, P_dense, eps}, s);
+            default: return -1;
+        }
+    });
+}
+
 extern "C" int pll_launch_xbwd32_norm(const pll_ppe_dev *d, const void *W32, double *p_halo,
                                       const double *eps, double *norm, hipStream_t s)
 {
@@ -1693,3 +1738,4 @@ extern "C" int pll_launch_ybwd32(const pll_ppe_dev *d, void *W32, hipStream_t s)
 {
     return dispatch_plan(d->py, [&](auto f) { return launch_y<decltype(f), float2>(false, d, d->tw_y32, W32, s); });
 }
+#endif

@@ -20,6 +20,9 @@ extern "C" {
 typedef struct {
     int L, E, T, nst;
     int rad[PLL_MAX_STAGES];
+    /* ceil(2^32 / (rad[0] .. rad[s-1])): n / that product by one high multiply,
+     * exact for n < 65536 (set for runtime plans) */
+    unsigned mag[PLL_MAX_STAGES];
 } pll_fftplan;
 
 /* Everything the PPE kernels need, all pointers on the device.

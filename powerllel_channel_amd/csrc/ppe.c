@@ -43,13 +43,9 @@ int pll_set_error(int code, const char *fmt, ...)
 
 /* ------------------------------------------------------------------ plans */
 /* Factor L = 2^a 3^b 5^c 7^d 11^e 13^f into radix stages from
- * {8,6,4,3,2,5,7,11,13}.  E (points per thread) is the first of
- * {12,8,24,6,4,3,5,7,2} that divides L, keeps L/E threads per row within the
- * kernel's limit and divides every radix of the plan, so that all stages run
- * from registers (E = 24 needs more than 256 VGPRs per lane, so it is the
- * last resort of the large ones).  Lengths that no such E fits (mixed
- * prime factors, such as 2^a 5 or 2^a 3 7) take the first E that divides L;
- * their stages whose radix does not divide E run through LDS. */
+ * {8,6,4,3,2,5,7,11,13} for E points per thread (E divides L): first the
+ * radices that divide E, whose stages run from registers, then the others,
+ * whose stages run through LDS (none with reg_only). */
 static int plan_for_E(int L, int E, const int cnt[4], const int cnt_big[2], int reg_only,
                       pll_fftplan *p)
 {
@@ -79,15 +75,20 @@ static int plan_for_E(int L, int E, const int cnt[4], const int cnt_big[2], int 
     p->T = L / E;
     p->nst = n;
     memcpy(p->rad, rad, sizeof(int) * (size_t)n);
+    for (int s = 0, q = 1; s < n; q *= rad[s], s++)
+        p->mag[s] = (unsigned)((((unsigned long long)1 << 32) + q - 1) / q);
     return 1;
 }
 
-static int make_plan(int L, pll_fftplan *p)
+/* maxT: threads per transform that the kernel would rather not exceed */
+static int make_plan(int L, int maxT, pll_fftplan *p)
 {
     memset(p, 0, sizeof *p);
-    /* PLL_FFT_E selects among compile-time plans of the same length (tuning) */
+    /* PLL_FFT_E (tuning): points per thread, of a compile-time plan when a length
+     * has two, of a runtime plan where it divides the length */
     const char *pe = getenv("PLL_FFT_E");
-    if (pll_fft_ct_plan(L, pe ? atoi(pe) : 0, p)) return PLL_OK;
+    const int want = pe ? atoi(pe) : 0;
+    if (pll_fft_ct_plan(L, want, p)) return PLL_OK;
     memset(p, 0, sizeof *p);
     if (L < 2) return pll_set_error(PLL_EUNSUP, "FFT length %d < 2", L);
     static const int primes[6] = {2, 3, 5, 7, 11, 13};
@@ -99,13 +100,31 @@ static int make_plan(int L, pll_fftplan *p)
                              "FFT length %d has a prime factor above 13 (radices 2, 3, 5, 7, "
                              "11 and 13 are supported)", L);
     const int cnt[4] = {c6[0], c6[1], c6[2], c6[3]}, big[2] = {c6[4], c6[5]};
-    static const int Es[] = {12, 8, 24, 6, 4, 3, 5, 7, 2};
-    for (int reg_only = 1; reg_only >= 0; reg_only--)
-        for (size_t ie = 0; ie < sizeof Es / sizeof Es[0]; ie++) {
-            const int E = Es[ie];
+    /* Points per thread, first fit:
+     * - lengths below 128: few (3 below 100, else 4), so that a row has lanes
+     *   enough to read long pieces and small grids have threads enough, whether
+     *   or not stages go through LDS (solves, 12 points -> this: 72x36x64 41 ->
+     *   25 us, 144x72x64 51 -> 36, 216x108x64 78 -> 62; 80x80x80 8 -> 4: 42 -> 35);
+     * - longer ones with a factor 5: 5 (4 -> 5: 240x140x90 90 -> 81, 320x160x64 90
+     *   -> 78, 640x320x64 265 -> 226; below 120 4 is faster, 200x100x64 52 for 56);
+     * - other longer ones: all stages in registers (288x144x64, 576x288x64: 87 and
+     *   229 us with 12, 88 and 238 with 4), else 4. */
+    static const int Es[4][9] = {{3, 4, 6, 5, 8, 7, 2, 12, 24}, {4, 3, 6, 5, 8, 7, 2, 12, 24},
+                                 {5, 4, 6, 8, 12, 3, 7, 24, 2}, {12, 8, 24, 6, 4, 3, 5, 7, 2}};
+    const int small = L < 128 && !(L % 5 == 0 && L >= 120);
+    const int first = small ? (L < 100 ? 0 : 1) : (L % 5 == 0 ? 2 : 3);
+    for (int pass = 0; pass < 3; pass++) {
+        /* stages in registers only; any stages, at most maxT threads; any */
+        if (pass == 0 && first != 3) continue;
+        const int *es = pass == 0 || first != 3 ? Es[first] : Es[1];
+        for (int ie = 0; ie < 9; ie++) {
+            const int E = es[ie];
             if (L % E != 0 || !pll_fft_supported_E(E) || L / E > pll_fft_max_threads(E)) continue;
-            if (plan_for_E(L, E, cnt, big, reg_only, p)) return PLL_OK;
+            if (pass == 1 && L / E > maxT) continue;
+            if (want > 0 && E != want && L % want == 0) continue;
+            if (plan_for_E(L, E, cnt, big, pass == 0, p)) return PLL_OK;
         }
+    }
     return pll_set_error(PLL_EUNSUP, "no FFT plan for length %d", L);
 }
 
@@ -452,7 +471,7 @@ int pll_ppe_create(pll_ppe **out, int nx, int ny, int nz, double dx, double dy,
     h->nz = nz;
     h->L = nx / 2;
     int rc;
-    if ((rc = make_plan(h->L, &h->d.px)) || (rc = make_plan(ny, &h->d.py)) ||
+    if ((rc = make_plan(h->L, 256, &h->d.px)) || (rc = make_plan(ny, 64, &h->d.py)) ||
         (rc = choose_launch(h))) {
         free(h);
         return rc;
@@ -1259,7 +1278,7 @@ void free_poisson_solver(void) { abort_on(free_poisson_solver_status(), "free_po
 int pll_fft_plan_info(int L, int *E, int *nst, int *rad)
 {
     pll_fftplan p;
-    const int rc = make_plan(L, &p);
+    const int rc = make_plan(L, 256, &p);
     if (rc) return rc;
     *E = p.E;
     *nst = p.nst;

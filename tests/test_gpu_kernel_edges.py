@@ -224,3 +224,33 @@ def test_ragged_z_solve(orc, cuda, shape, bc, monkeypatch):
         a, b = p[inner], q[inner]
         assert float((a - b).abs().max()) <= tol * float(b.abs().max()), solve
         assert torch.equal(p[0], torch.from_numpy(f[0]).to(cuda))
+
+
+# transform plans: every points-per-thread choice of the runtime plans (3, 4, 5,
+# 7, 12; stages in registers and through LDS; rows that leave lanes of the last
+# wavefront idle) and the compile-time lengths 32, 48, 96 in x and y
+@pytest.mark.parametrize("shape", [
+    (72, 54, 6), (216, 108, 4), (240, 120, 4), (288, 144, 4), (450, 100, 3), (24, 96, 8),
+    (192, 48, 5), (96, 32, 5), (64, 140, 4), (98, 210, 3), (220, 26, 4), (432, 216, 3)])
+def test_transform_plans(orc, cuda, shape):
+    """Solve against the oracle (1e-12) and the refined form with two sweeps
+    (1e-11, its bar)."""
+    import torch
+    from powerllel_channel_amd import PoissonSolver
+    from powerllel_channel_amd.mesh import Grid
+    nx, ny, nz = shape
+    print(f"[transform plans] {shape}", flush=True)
+    g = Grid(nx, ny, nz, 6.0, 3.0, 2.0, 1.0)
+    f = np.random.default_rng(13).standard_normal(g.shape)
+    wz = g.dzf[1:-1]
+    inner = (slice(1, -1),) * 3
+    f[inner] -= (f[inner].sum(axis=(1, 2)) * wz).sum() / (wz.sum() * nx * ny)
+    ref = f.copy()
+    orc.OraclePPE(nx, ny, nz, g.dx, g.dy, g.dzf, pin_gauge=True).solve(ref)
+    s = PoissonSolver(nx, ny, nz, g.dx, g.dy, g.dzf)
+    p, q = _dev(torch, cuda, f, f)
+    s.solve(p)
+    s.solve_refined(q, 2)
+    top = np.abs(ref[inner]).max()
+    assert np.abs(p.cpu().numpy() - ref)[inner].max() <= 1e-12 * top
+    assert np.abs(q.cpu().numpy() - ref)[inner].max() <= 1e-11 * top
