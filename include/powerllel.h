@@ -186,6 +186,14 @@ int pll_channel_max_cfl(pll_channel *c, const double *u, const double *v,
  * haloed field is NaN.  Synchronises. */
 int pll_channel_check_nan(pll_channel *c, const double *q, int *has_nan,
                           void *stream);
+/* The run-time check of src/main.f90:213-222 in one pass over the fields:
+ * *has_nan as pll_channel_check_nan of u, (cfl, cfl_ijk) as
+ * pll_channel_max_cfl, (div, div_ijk) as pll_channel_max_div; any of the
+ * results may be NULL.  Synchronises. */
+int pll_channel_check(pll_channel *c, const double *u, const double *v,
+                      const double *w, int *has_nan, double *cfl,
+                      int cfl_ijk[3], double *div, int div_ijk[3],
+                      void *stream);
 /* One whole time step, src/main.f90:137-208: RK1, BC, RK2, BC, calcRHS,
  * PPE (ppe must match the grid), updateBoundP, correctVel, forceVel, BC.
  * With the FP64 solve, calcRHS is formed inside the solve's x transform

@@ -113,11 +113,15 @@ class Channel:
 
     def check(self, u, v, w, cfl_limit, div_limit, stream=None):
         """The run-time check of src/main.f90:213-222: checkNaN(u), calcMaxCFL +
-        checkCFL, calcMaxDiv + checkDiv.  Returns (passed, report); a value
+        checkCFL, calcMaxDiv + checkDiv, in one pass over the fields.  Returns (passed, report); a value
         above its limit or NaN fails, as in checkCFL / checkDiv."""
-        nan = self.check_nan(u, stream)
-        cfl, cfl_at = self.max_cfl(u, v, w, stream)
-        div, div_at = self.max_div(u, v, w, stream)
+        self._chk(u, v, w)
+        flag, vals, at = C.c_int(), (C.c_double(), C.c_double()), ((C.c_int * 3)(), (C.c_int * 3)())
+        check(lib().pll_channel_check(self._h, _p(u), _p(v), _p(w), C.byref(flag),
+                                      C.byref(vals[0]), at[0], C.byref(vals[1]), at[1],
+                                      _stream_ptr(stream)))
+        nan, cfl, div = bool(flag.value), vals[0].value, vals[1].value
+        cfl_at, div_at = tuple(at[0]), tuple(at[1])
         ok_cfl = not (cfl > cfl_limit or cfl != cfl)
         ok_div = not (div > div_limit or div != div)
         report = {"nan": nan, "cfl_max": cfl, "cfl_at": cfl_at, "div_max": div, "div_at": div_at}

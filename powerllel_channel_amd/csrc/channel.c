@@ -27,9 +27,10 @@ struct pll_channel {
     int is_forced[3];
     double vel_force[3];
     double *zarr;      /* device: dzf | dzf_inv | dzc_inv | dzflzi, each nz+2 */
-    double *part;      /* device: ny*nz partials */
-    long long *pidx;   /* device: ny*nz indices  */
-    double *scal;      /* device: 8 scalars (mean, max value, fused-step means at 4, 5) */
+    double *part;      /* device: partials (ny*nz, and what the other passes need) */
+    long long *pidx;   /* device: as many indices */
+    double *scal;      /* device: 16 scalars (mean, max value, fused-step means at 4, 5,
+                        * wall sums at 6, 7, run-time check at 8 .. 12) */
     long long *sidx;   /* device: 1 index */
     double *dzf_h;     /* host copy of dzf_global (nz+2) */
     double lx, ly, lz;
@@ -109,10 +110,11 @@ int pll_channel_create(pll_channel **out, int nx, int ny, int nz, double lx, dou
     size_t nrow = (size_t)ny * nz;
     const size_t nfused = 2 * (size_t)pll_rk_blocks(&c->g); /* fused-step Mean_h partials */
     if (nfused > nrow) nrow = nfused;
+    if (nrow < 3 * PLL_CHECK_BLOCKS) nrow = 3 * PLL_CHECK_BLOCKS;
     if ((e = hipMalloc((void **)&c->zarr, sizeof(double) * 4 * (size_t)n2)) != hipSuccess ||
         (e = hipMalloc((void **)&c->part, sizeof(double) * nrow)) != hipSuccess ||
         (e = hipMalloc((void **)&c->pidx, sizeof(long long) * nrow)) != hipSuccess ||
-        (e = hipMalloc((void **)&c->scal, sizeof(double) * 8)) != hipSuccess ||
+        (e = hipMalloc((void **)&c->scal, sizeof(double) * 16)) != hipSuccess ||
         (e = hipMalloc((void **)&c->sidx, sizeof(long long))) != hipSuccess ||
         (e = hipMemcpy(c->zarr, z, sizeof(double) * 4 * (size_t)n2, hipMemcpyHostToDevice)) !=
             hipSuccess) {
@@ -293,6 +295,36 @@ int pll_channel_check_nan(pll_channel *c, const double *q, int *has_nan, void *s
     int any = 0;
     for (int b = 0; b < nb; b++) any |= flags[b] != 0;
     *has_nan = any;
+    return PLL_OK;
+}
+
+/* The run-time check of src/main.f90:213-222 in one pass over the velocity:
+ * checkNaN of u, calcMaxCFL and calcMaxDiv with the results of the separate
+ * calls. */
+int pll_channel_check(pll_channel *c, const double *u, const double *v, const double *w,
+                      int *has_nan, double *cfl, int cfl_ijk[3], double *div, int div_ijk[3],
+                      void *stream)
+{
+    CHK_C(c);
+    if (!u || !v || !w) return pll_set_error(PLL_EINVAL, "NULL field");
+    hipStream_t s = (hipStream_t)stream;
+    int rc;
+    if ((rc = kl(pll_launch_check(&c->g, u, v, w, c->part, c->pidx, c->scal + 8, s), "check")))
+        return rc;
+    struct { double v[2]; long long i[2], nan; } r;
+    HIPCHK(hipMemcpyAsync(&r, c->scal + 8, sizeof r, hipMemcpyDeviceToHost, s));
+    HIPCHK(hipStreamSynchronize(s));
+    if (has_nan) *has_nan = r.nan != 0;
+    if (cfl) *cfl = (r.v[0] < 0.0 ? 0.0 : r.v[0]) * c->g.dt;
+    if (div) *div = r.v[1] < 0.0 ? 0.0 : r.v[1];
+    int *at[2] = {cfl_ijk, div_ijk};
+    const long long nx = c->g.nx, ny = c->g.ny;
+    for (int f = 0; f < 2; f++)
+        if (at[f]) {
+            at[f][0] = (int)(r.i[f] % nx) + 1;
+            at[f][1] = (int)((r.i[f] / nx) % ny) + 1;
+            at[f][2] = (int)(r.i[f] / (nx * ny)) + 1;
+        }
     return PLL_OK;
 }
 

@@ -238,6 +238,12 @@ int pll_launch_maxdiv_final(int n, const double *pval, const long long *pidx,
 int pll_launch_maxcfl_partials(const pll_grid_dev *g, const double *u,
                                const double *v, const double *w, double *pval,
                                long long *pidx, hipStream_t s);
+/* NaN of u, CFL and divergence maxima in one pass: pval 2, pidx 3 times
+ * PLL_CHECK_BLOCKS; res: 5 values of 8 bytes (max CFL sum, max |div|, their
+ * linear indices, NaN flag of u) */
+#define PLL_CHECK_BLOCKS 8192
+int pll_launch_check(const pll_grid_dev *g, const double *u, const double *v, const double *w,
+                     double *pval, long long *pidx, double *res, hipStream_t s);
 /* flags[0 .. nblocks) = 1 where a block's share of the haloed field holds a NaN */
 int pll_launch_nan_partials(const pll_grid_dev *g, const double *q, long long *flags,
                             int nblocks, hipStream_t s);

@@ -389,11 +389,13 @@ __global__ void __launch_bounds__(256) k_mean_part(G g, const double *__restrict
     for (int i = threadIdx.x + 1; i <= g.nx; i += blockDim.x) s = s + q[base + i] * wk;
     sh[threadIdx.x] = s;
     __syncthreads();
-    for (int h = blockDim.x / 2; h > 0; h >>= 1) {
-        if ((int)threadIdx.x < h) sh[threadIdx.x] += sh[threadIdx.x + h];
-        __syncthreads();
+    if (threadIdx.x < 128) sh[threadIdx.x] += sh[threadIdx.x + 128];
+    __syncthreads();
+    if (threadIdx.x < 64) {
+        double r = sh[threadIdx.x] + sh[threadIdx.x + 64];
+        for (int h = 32; h > 0; h >>= 1) r += __shfl_down(r, h);
+        if (threadIdx.x == 0) part[blockIdx.x] = r;
     }
-    if (threadIdx.x == 0) part[blockIdx.x] = sh[0];
 }
 
 __global__ void __launch_bounds__(1024) k_mean_final(int n, const double *__restrict__ part,
@@ -402,14 +404,30 @@ __global__ void __launch_bounds__(1024) k_mean_final(int n, const double *__rest
 {
     __shared__ double sh[1024];
     double s = 0.0;
-    for (int t = threadIdx.x; t < n; t += blockDim.x) s += part[t];
+    // eight partials in flight per thread, added in order (98304 partials, one
+    // at a time: 38 us)
+    const int nb = blockDim.x;
+    int t = threadIdx.x;
+    for (; t + 7 * nb < n; t += 8 * nb) {
+        double o[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) o[q] = part[t + q * nb];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) s += o[q];
+    }
+    for (; t < n; t += nb) s += part[t];
     sh[threadIdx.x] = s;
     __syncthreads();
-    for (int h = blockDim.x / 2; h > 0; h >>= 1) {
+    for (int h = blockDim.x / 2; h > 32; h >>= 1) {
         if ((int)threadIdx.x < h) sh[threadIdx.x] += sh[threadIdx.x + h];
         __syncthreads();
     }
-    if (threadIdx.x == 0) out[0] = sh[0] / nx / ny;
+    if (threadIdx.x < 64) {
+        double r = sh[threadIdx.x];
+        r = threadIdx.x < 32 ? r + sh[threadIdx.x + 32] : r;
+        for (int h = 16; h > 0; h >>= 1) r += __shfl_down(r, h);
+        if (threadIdx.x == 0) out[0] = r / nx / ny;
+    }
 }
 
 __global__ void __launch_bounds__(256) k_force_shift(G g, double *__restrict__ q, double vel_force,
@@ -630,6 +648,125 @@ __global__ void __launch_bounds__(1024) k_maxdiv_final(int n, const double *__re
     if (threadIdx.x == 0) {
         oval[0] = sv[0];
         oidx[0] = si[0];
+    }
+}
+
+// The run-time checks in one pass over u, v, w: calcMaxCFL's sum (value 0),
+// calcMaxDiv's (value 1), both with location as k_maxloc_part, and checkNaN of
+// u (ghost cells included).  Up to CHK workgroups share the rows, in y slabs per XCD
+// as there; each leaves one partial of either maximum (pval, pidx: value 0 of
+// every workgroup, then value 1) and a NaN flag (after both locations).
+// Bound by HBM: 24 N bytes for the 56 N of the three separate passes;
+// 768x384x256 0.40 ms (4.6 TB/s) for 0.34 + 0.34 + 0.17 and their final passes.
+constexpr int CHK = PLL_CHECK_BLOCKS;
+
+struct MaxLoc {
+    double v;
+    long long i;
+};
+__device__ __forceinline__ void take(MaxLoc &a, double v, long long i)
+{
+    if (v > a.v || (v == a.v && i < a.i)) {
+        a.v = v;
+        a.i = i;
+    }
+}
+__device__ __forceinline__ void take_wave(MaxLoc &a)
+{
+    for (int h = 32; h > 0; h >>= 1) {
+        const double v = __shfl_xor(a.v, h);
+        const long long i = __shfl_xor(a.i, h);
+        take(a, v, i);
+    }
+}
+
+__global__ void __launch_bounds__(256) k_check_part(G g, const double *__restrict__ u,
+                                                    const double *__restrict__ v,
+                                                    const double *__restrict__ w, long long nshell,
+                                                    double *__restrict__ pval,
+                                                    long long *__restrict__ pidx)
+{
+    MaxLoc c{-1.0, 0}, d{-1.0, 0};
+    int bad = 0;
+    const bool slab = g.ny % 8 == 0;
+    const int sl = g.ny >> 3, x = blockIdx.x & 7;
+    const long long rows = slab ? (long long)sl * g.nz : (long long)g.ny * g.nz;
+    const long long r0 = slab ? blockIdx.x >> 3 : blockIdx.x, dr = slab ? gridDim.x >> 3 : gridDim.x;
+    for (long long r = r0; r < rows; r += dr) {
+        const int k = (int)(r / (slab ? sl : g.ny)) + 1;
+        const int j = slab ? x * sl + (int)(r % sl) + 1 : (int)(r % g.ny) + 1;
+        const long long base = g.sy * j + g.sz * k;
+        const double dzi = g.dzf_inv[k];
+        for (int i = threadIdx.x + 1; i <= g.nx; i += 256) {
+            const long long e = base + i;
+            const double uc = u[e], um = u[e - 1], vc = v[e], vm = v[e - g.sy], wc = w[e],
+                         wm = w[e - g.sz];
+            bad |= uc != uc;
+            const double cfl = fabs((uc + um) * 0.5) * g.dx_inv + fabs((vc + vm) * 0.5) * g.dy_inv +
+                               fabs((wc + wm) * 0.5) * dzi;
+            const double div = fabs((uc - um) * g.dx_inv + (vc - vm) * g.dy_inv + (wc - wm) * dzi);
+            const long long at = ((long long)(k - 1) * g.ny + (j - 1)) * g.nx + (i - 1);
+            take(c, cfl, at);
+            take(d, div, at);
+        }
+    }
+    const int planes[2] = {0, g.nz + 1};
+    for (long long t = (long long)blockIdx.x * 256 + threadIdx.x; t < nshell;
+         t += gridDim.x * 256LL) {
+        int i, j, k;
+        if (shell_pos(g, t, i, j, k, 2, planes)) {
+            const double q = u[i + g.sy * j + g.sz * k];
+            bad |= q != q;
+        }
+    }
+    __shared__ MaxLoc red[2][4];
+    take_wave(c);
+    take_wave(d);
+    if ((threadIdx.x & 63) == 0) {
+        red[0][threadIdx.x >> 6] = c;
+        red[1][threadIdx.x >> 6] = d;
+    }
+    bad = __syncthreads_or(bad);
+    if (threadIdx.x == 0) {
+        for (int q = 1; q < 4; ++q) {
+            take(c, red[0][q].v, red[0][q].i);
+            take(d, red[1][q].v, red[1][q].i);
+        }
+        pval[blockIdx.x] = c.v;
+        pidx[blockIdx.x] = c.i;
+        pval[gridDim.x + blockIdx.x] = d.v;
+        pidx[gridDim.x + blockIdx.x] = d.i;
+        pidx[2 * gridDim.x + blockIdx.x] = bad;
+    }
+}
+
+// res: two maxima, then their locations and the NaN flag (8 bytes each)
+__global__ void __launch_bounds__(1024) k_check_final(int n, const double *__restrict__ pval,
+                                                      const long long *__restrict__ pidx,
+                                                      double *__restrict__ res)
+{
+    MaxLoc m[2] = {{-1.0, 0}, {-1.0, 0}};
+    int bad = 0;
+#pragma unroll 4
+    for (int t = threadIdx.x; t < n; t += 1024) {
+        take(m[0], pval[t], pidx[t]);
+        take(m[1], pval[n + t], pidx[n + t]);
+        bad |= pidx[2 * n + t] != 0;
+    }
+    __shared__ MaxLoc red[2][16];
+    for (int f = 0; f < 2; ++f) {
+        take_wave(m[f]);
+        if ((threadIdx.x & 63) == 0) red[f][threadIdx.x >> 6] = m[f];
+    }
+    bad = __syncthreads_or(bad);
+    if (threadIdx.x == 0) {
+        long long *ri = reinterpret_cast<long long *>(res);
+        for (int f = 0; f < 2; ++f) {
+            for (int q = 1; q < 16; ++q) take(m[f], red[f][q].v, red[f][q].i);
+            res[f] = m[f].v;
+            ri[2 + f] = m[f].i;
+        }
+        ri[4] = bad;
     }
 }
 
@@ -861,5 +998,27 @@ extern "C" int pll_launch_maxdiv_final(int n, const double *pval, const long lon
                                        double *oval, long long *oidx, hipStream_t s)
 {
     hipLaunchKernelGGL(k_maxdiv_final, dim3(1), dim3(1024), 0, s, n, pval, pidx, oval, oidx);
+    return ok();
+}
+
+extern "C" int pll_launch_check(const pll_grid_dev *gd, const double *u, const double *v,
+                                const double *w, double *pval, long long *pidx, double *res,
+                                hipStream_t s)
+{
+    const G g = make_g(gd);
+    const long long shell = 2LL * (g.nx + 2) * (g.ny + 2) + 2LL * (g.nx + 2) * g.nz +
+                            2LL * g.ny * g.nz;
+    const long long rows = (long long)g.ny * g.nz;
+    // about twelve rows per workgroup, 2048 to 8192 of them (768x384x256 643 us per
+    // check with 2048, 619 with 8192, 684 with 65536; 192x192x128 137, 159, 202:
+    // more workgroups drift apart less, which keeps the neighbour rows in the
+    // L2, but leave more partials and start-up)
+    long long n8 = rows / 12;
+    n8 = n8 < 2048 ? 2048 : (n8 > CHK ? CHK : n8);
+    n8 = n8 < rows ? n8 : rows;
+    const int n = (int)((n8 + 7) / 8 * 8);
+    hipLaunchKernelGGL(k_check_part, dim3(n), dim3(256), 0, s, g, u, v, w, shell, pval, pidx);
+    if (ok()) return -3;
+    hipLaunchKernelGGL(k_check_final, dim3(1), dim3(1024), 0, s, n, pval, pidx, res);
     return ok();
 }

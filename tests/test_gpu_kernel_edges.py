@@ -254,3 +254,40 @@ def test_transform_plans(orc, cuda, shape):
     top = np.abs(ref[inner]).max()
     assert np.abs(p.cpu().numpy() - ref)[inner].max() <= 1e-12 * top
     assert np.abs(q.cpu().numpy() - ref)[inner].max() <= 1e-11 * top
+
+
+# one-pass check: rows in XCD slabs (ny a multiple of 8) and in plain order,
+# fewer rows than workgroups and more, rows shorter and longer than a workgroup
+@pytest.mark.parametrize("shape", [(4, 2, 2), (300, 24, 7), (20, 30, 90), (64, 128, 40)])
+def test_check_equals_separate_calls(cuda, shape):
+    """NaN flag, maxima and locations equal to check_nan, max_cfl, max_div; ties
+    go to the first cell, NaN cells never win, infinities do."""
+    import torch
+    from powerllel_channel_amd import Channel
+    from powerllel_channel_amd.mesh import Grid
+    nx, ny, nz = shape
+    print(f"[check] {shape}", flush=True)
+    g = Grid(nx, ny, nz, 4.0, 2.0, 2.0, 2.0)
+    ch = Channel(nx, ny, nz, 4.0, 2.0, 2.0, g.dzf, 1e-3, 1e-3)
+    gen = torch.Generator().manual_seed(2)
+    f = [torch.randn(g.shape, generator=gen, dtype=torch.float64).to(cuda) for _ in range(3)]
+
+    def compare(u, v, w):
+        _, rep = ch.check(u, v, w, 1.0, 1.0)
+        cfl, div = ch.max_cfl(u, v, w), ch.max_div(u, v, w)
+        assert rep["nan"] == ch.check_nan(u)
+        assert (rep["cfl_max"], rep["cfl_at"]) == cfl
+        assert (rep["div_max"], rep["div_at"]) == div
+        return rep
+    assert not compare(*f)["nan"]
+    const = [torch.ones_like(t) for t in f]  # every cell ties
+    assert compare(*const)["cfl_at"][:2] == (1, 1)
+    for at in ((0, 0, 0), (nz + 1, ny + 1, nx + 1), (1, 0, nx), (nz, ny, nx + 1), (nz, ny, nx)):
+        u = f[0].clone()
+        u[at] = float("nan")
+        assert compare(u, *f[1:])["nan"]
+    w = f[2].clone()
+    w[nz, ny, 1] = float("inf")
+    assert compare(f[0], f[1], w)["div_max"] == float("inf")
+    everywhere = torch.full_like(f[0], float("nan"))
+    assert compare(everywhere, *f[1:])["cfl_max"] == 0.0
