@@ -170,7 +170,8 @@ int pll_channel_correct_vel(pll_channel *c, const double *p, double *u, double *
 {
     CHK_C(c);
     const double *q[3] = {u, v, w};
-    return kl(pll_launch_correct_vel(&c->g, p, q, u, v, w, 0, 0.0, 0.0, NULL, (hipStream_t)stream),
+    return kl(pll_launch_correct_vel(&c->g, p, q, u, v, w, 0, 0.0, 0.0, NULL, 0,
+                                     (hipStream_t)stream),
               "correct_vel");
 }
 
@@ -360,9 +361,9 @@ static int step_impl(pll_channel *c, pll_ppe *ppe, double *u, double *v, double 
                     return rc;
     /* The boundary fill of the RK2 output is read by calcRHS only, unless the
      * separate forcing passes follow (Mean_h of w includes its wall row): the
-     * fused calcRHS takes the values it would leave from the interior, and the
-     * fill at the end of the step writes the ghosts and w's wall row (one fill
-     * less per step: 64x64x64 75 -> 64 us, 192x192x128 358 -> 342 us). */
+     * fused calcRHS takes the values it would leave from the interior, and
+     * correctVel at the end of the step writes the ghosts and w's wall row (one
+     * fill less per step: 64x64x64 75 -> 64 us, 192x192x128 358 -> 342 us). */
     const int fp64 = pll_ppe_refinement(ppe) < 0, unfilled = fp64 && (fuse || none);
     if (!unfilled && (rc = pll_channel_bc_vel(c, u, v, w, stream))) return rc;
     if (fp64) {
@@ -379,14 +380,12 @@ static int step_impl(pll_channel *c, pll_ppe *ppe, double *u, double *v, double 
     }
     if (fuse || none) {
         const double *q[3] = {u, v, w};
-        if ((rc = kl(pll_launch_correct_vel(&c->g, p, q, u, v, w, fuse ? fmask : 0, c->vel_force[0],
-                                            c->vel_force[1], fuse ? c->scal + 4 : NULL, s),
-                     "correct_vel")))
-            return rc;
-    } else {
-        if ((rc = pll_channel_correct_vel(c, p, u, v, w, stream))) return rc;
-        if ((rc = pll_channel_force_vel(c, u, v, w, stream))) return rc;
+        return kl(pll_launch_correct_vel(&c->g, p, q, u, v, w, fuse ? fmask : 0, c->vel_force[0],
+                                         c->vel_force[1], fuse ? c->scal + 4 : NULL, 1, s),
+                  "correct_vel");
     }
+    if ((rc = pll_channel_correct_vel(c, p, u, v, w, stream))) return rc;
+    if ((rc = pll_channel_force_vel(c, u, v, w, stream))) return rc;
     return pll_channel_bc_vel(c, u, v, w, stream);
 }
 
@@ -458,11 +457,9 @@ static int run_chain(pll_channel *c, pll_ppe *ppe, int m, double *u, double *v, 
         if ((rc = forcing_means(c, fmask, s)) || (rc = solve_unfilled(c, ppe, q, p, s))) return rc;
     }
     const double *q[3] = {X[0], X[1], X[2]};
-    if ((rc = kl(pll_launch_correct_vel(&c->g, p, q, u, v, w, fmask, c->vel_force[0],
-                                        c->vel_force[1], mean, s),
-                 "correct_vel")))
-        return rc;
-    return pll_channel_bc_vel(c, u, v, w, s);
+    return kl(pll_launch_correct_vel(&c->g, p, q, u, v, w, fmask, c->vel_force[0],
+                                     c->vel_force[1], mean, 1, s),
+              "correct_vel");
 }
 
 int pll_channel_run(pll_channel *c, pll_ppe *ppe, int nsteps, double *u, double *v, double *w,
@@ -514,12 +511,11 @@ int pll_channel_step_from(pll_channel *c, pll_ppe *ppe, const double *const src[
     if ((rc = kl(pll_launch_rk12(&c->g, src, tmp, NULL, fmask ? c->part : NULL, fmask, 0.0, 0.0,
                                  NULL, body, s),
                  "rk1 + rk2")) ||
-        (rc = forcing_means(c, fmask, s)) || (rc = solve_unfilled(c, ppe, q, p, s)) ||
-        (rc = kl(pll_launch_correct_vel(&c->g, p, q, dst[0], dst[1], dst[2], fmask,
-                                        c->vel_force[0], c->vel_force[1], mean, s),
-                 "correct_vel")))
+        (rc = forcing_means(c, fmask, s)) || (rc = solve_unfilled(c, ppe, q, p, s)))
         return rc;
-    return pll_channel_bc_vel(c, dst[0], dst[1], dst[2], stream);
+    return kl(pll_launch_correct_vel(&c->g, p, q, dst[0], dst[1], dst[2], fmask, c->vel_force[0],
+                                     c->vel_force[1], mean, 1, s),
+              "correct_vel");
 }
 
 int pll_channel_step_body(pll_channel *c, pll_ppe *ppe, double *u, double *v, double *w,

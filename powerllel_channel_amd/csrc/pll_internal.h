@@ -212,10 +212,11 @@ int pll_launch_calc_rhs(const pll_grid_dev *g, const double *u, const double *v,
                         const double *w, double *p, hipStream_t s);
 /* (u, v, w) := q corrected, q = the same arrays or others; mean non-NULL and
  * fmask != 0: then also += vel_force - mean[d] for the forced components
- * (bit 0 u with vfu, bit 1 v with vfv). */
+ * (bit 0 u with vfu, bit 1 v with vfv); with fill, the boundary fill of the
+ * result too. */
 int pll_launch_correct_vel(const pll_grid_dev *g, const double *p, const double *const q[3],
                            double *u, double *v, double *w, int fmask, double vfu, double vfv,
-                           const double *mean, hipStream_t s);
+                           const double *mean, int fill, hipStream_t s);
 /* partial sums of q*dzflzi per (j,k) row into part[ny*nz]; then a single
  * workgroup reduces them to out[0] = sum / nx / ny (Mean_h). */
 int pll_launch_mean_partials(const pll_grid_dev *g, const double *q, double *part,

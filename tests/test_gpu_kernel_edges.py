@@ -291,3 +291,37 @@ def test_check_equals_separate_calls(cuda, shape):
     assert compare(f[0], f[1], w)["div_max"] == float("inf")
     everywhere = torch.full_like(f[0], float("nan"))
     assert compare(everywhere, *f[1:])["cfl_max"] == 0.0
+
+
+# the corrected velocity's ghosts written by the projection: the smallest grid,
+# tiles cut by the edge, k chunks with short ends
+@pytest.mark.parametrize("shape,forced,u_crf", [
+    ((4, 2, 2), (True, False, False), 0.3),
+    ((10, 6, 3), (True, True, False), 0.3),
+    ((66, 26, 17), (False, False, False), 0.2),
+    ((64, 256, 131), (True, False, False), 0.0)])
+def test_step_fills_boundary(orc, cuda, shape, forced, u_crf):
+    """A step and a run leave the ghosts that the fill makes of their result."""
+    import torch
+    from powerllel_channel_amd import PoissonSolver
+    nx, ny, nz = shape
+    print(f"[step fills] {shape} forced={forced}", flush=True)
+    g, G, ch, (u, v, w, *_) = _channel(orc, nx, ny, nz, u_crf=u_crf, is_forced=forced,
+                                       vel_force=(1.0, 0.2, 0.0), dt=1e-4)
+    orc.bc_vel(G, u, v, w, u_crf)
+    z = np.zeros(g.shape)
+    s = PoissonSolver(nx, ny, nz, g.dx, g.dy, g.dzf)
+    for n in (1, 2):
+        a = _dev(torch, cuda, u, v, w, z, z, z, z)
+        ch.run(s, n, *a)
+        b = [q.clone() for q in a[:3]]
+        inner = np.full(g.shape, np.nan)
+        inner[1:-1, 1:-1, 1:-1] = 0.0
+        m = torch.from_numpy(inner).to(cuda)
+        for q in b:
+            q += m
+        ch.bc_vel(*b)
+        torch.cuda.synchronize()
+        for x, y in zip(a[:3], b):
+            assert torch.isfinite(y).all()
+            assert torch.equal(x, y)
