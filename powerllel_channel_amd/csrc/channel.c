@@ -329,6 +329,19 @@ int pll_channel_check(pll_channel *c, const double *u, const double *v, const do
     return PLL_OK;
 }
 
+/* The FP64 solve with calcRHS of a velocity whose boundary fill is not made; its
+ * x transform also reduces Mean_h of that velocity's components in fmask, from
+ * RK2's partial sums, to scal[4], scal[5]. */
+static int solve_unfilled(pll_channel *c, pll_ppe *ppe, const double *const q[3], double *p,
+                          int fmask, hipStream_t s)
+{
+    const double dti = 1.0 / c->g.dt;
+    const pll_div_src d = {q[0], q[1], q[2], c->g.dzf_inv, dti, dti * c->g.dx_inv,
+                           dti * c->g.dy_inv, 1, fmask ? c->part : NULL,
+                           pll_rk_blocks(&c->g), fmask, c->scal + 4};
+    return pll_ppe_solve_div(ppe, &d, p, s);
+}
+
 static int step_impl(pll_channel *c, pll_ppe *ppe, double *u, double *v, double *w, double *u1,
                      double *v1, double *w1, double *p, const double *const *body, void *stream)
 {
@@ -345,20 +358,12 @@ static int step_impl(pll_channel *c, pll_ppe *ppe, double *u, double *v, double 
     const int fmask = (c->is_forced[0] ? 1 : 0) | (c->is_forced[1] ? 2 : 0);
     const int fuse = fmask && !c->is_forced[2];
     const int none = !fmask && !c->is_forced[2];
-    const int nb = pll_rk_blocks(&c->g);
     if ((rc = kl(pll_launch_rk1(&c->g, u, v, w, u1, v1, w1, body, s), "rk1"))) return rc;
     /* RK2 reads u1's boundary values from its interior (no fill pass) */
     if ((rc = kl(pll_launch_rk2(&c->g, u, v, w, u1, v1, w1, fuse ? c->part : NULL,
                                 fuse ? fmask : 0, body, 1, s),
                  "rk2")))
         return rc;
-    if (fuse)
-        for (int d = 0; d < 2; d++)
-            if ((fmask >> d) & 1)
-                if ((rc = kl(pll_launch_mean_final(nb, c->part + (size_t)d * nb, c->scal + 4 + d,
-                                                   c->g.nx, c->g.ny, s),
-                             "mean final")))
-                    return rc;
     /* The boundary fill of the RK2 output is read by calcRHS only, unless the
      * separate forcing passes follow (Mean_h of w includes its wall row): the
      * fused calcRHS takes the values it would leave from the interior, and
@@ -366,24 +371,34 @@ static int step_impl(pll_channel *c, pll_ppe *ppe, double *u, double *v, double 
      * fill less per step: 64x64x64 75 -> 64 us, 192x192x128 358 -> 342 us). */
     const int fp64 = pll_ppe_refinement(ppe) < 0, unfilled = fp64 && (fuse || none);
     if (!unfilled && (rc = pll_channel_bc_vel(c, u, v, w, stream))) return rc;
-    if (fp64) {
+    if (fuse && !unfilled)
+        for (int d = 0; d < 2; d++)
+            if ((fmask >> d) & 1) {
+                const int nb = pll_rk_blocks(&c->g);
+                if ((rc = kl(pll_launch_mean_final(nb, c->part + (size_t)d * nb, c->scal + 4 + d,
+                                                   c->g.nx, c->g.ny, s),
+                             "mean final")))
+                    return rc;
+            }
+    const double *q[3] = {u, v, w};
+    if (unfilled) {
         /* calcRHS fused into the solve's x forward transform: the right-hand
          * side is never stored (mod_calcRHS.f90:28-30, same arithmetic) */
+        if ((rc = solve_unfilled(c, ppe, q, p, fuse ? fmask : 0, s))) return rc;
+    } else if (fp64) {
         const double dti = 1.0 / c->g.dt;
-        pll_div_src q = {u, v, w, c->g.dzf_inv, dti, dti * c->g.dx_inv, dti * c->g.dy_inv,
-                         unfilled};
-        if ((rc = pll_ppe_solve_div(ppe, &q, p, stream))) return rc;  /* + updateBoundP */
+        const pll_div_src d = {u, v, w, c->g.dzf_inv, dti, dti * c->g.dx_inv, dti * c->g.dy_inv, 0,
+                               NULL, 0, 0, NULL};
+        if ((rc = pll_ppe_solve_div(ppe, &d, p, stream))) return rc;  /* + updateBoundP */
     } else {
         if ((rc = pll_channel_calc_rhs(c, u, v, w, p, stream))) return rc;
         if ((rc = pll_ppe_solve(ppe, p, stream))) return rc;
         if ((rc = pll_channel_bc_p(c, p, stream))) return rc;
     }
-    if (fuse || none) {
-        const double *q[3] = {u, v, w};
+    if (fuse || none)
         return kl(pll_launch_correct_vel(&c->g, p, q, u, v, w, fuse ? fmask : 0, c->vel_force[0],
                                          c->vel_force[1], fuse ? c->scal + 4 : NULL, 1, s),
                   "correct_vel");
-    }
     if ((rc = pll_channel_correct_vel(c, p, u, v, w, stream))) return rc;
     if ((rc = pll_channel_force_vel(c, u, v, w, stream))) return rc;
     return pll_channel_bc_vel(c, u, v, w, stream);
@@ -393,30 +408,6 @@ int pll_channel_step(pll_channel *c, pll_ppe *ppe, double *u, double *v, double 
                      double *v1, double *w1, double *p, void *stream)
 {
     return step_impl(c, ppe, u, v, w, u1, v1, w1, p, NULL, stream);
-}
-
-/* Mean_h of the RK2 output from its partial sums, into scal[4], scal[5] */
-static int forcing_means(pll_channel *c, int fmask, hipStream_t s)
-{
-    const int nb = pll_rk_blocks(&c->g);
-    for (int d = 0; d < 2; d++)
-        if ((fmask >> d) & 1) {
-            const int rc = kl(pll_launch_mean_final(nb, c->part + (size_t)d * nb, c->scal + 4 + d,
-                                                    c->g.nx, c->g.ny, s),
-                              "mean final");
-            if (rc) return rc;
-        }
-    return PLL_OK;
-}
-
-/* the FP64 solve with calcRHS of a velocity whose boundary fill is not made */
-static int solve_unfilled(pll_channel *c, pll_ppe *ppe, const double *const q[3], double *p,
-                          hipStream_t s)
-{
-    const double dti = 1.0 / c->g.dt;
-    const pll_div_src d = {q[0], q[1], q[2], c->g.dzf_inv, dti, dti * c->g.dx_inv,
-                           dti * c->g.dy_inv, 1};
-    return pll_ppe_solve_div(ppe, &d, p, s);
 }
 
 /* m steps whose projections are carried into the next step.  Step 0 takes
@@ -454,7 +445,7 @@ static int run_chain(pll_channel *c, pll_ppe *ppe, int m, double *u, double *v, 
             X = Y;
         }
         const double *q[3] = {X[0], X[1], X[2]};
-        if ((rc = forcing_means(c, fmask, s)) || (rc = solve_unfilled(c, ppe, q, p, s))) return rc;
+        if ((rc = solve_unfilled(c, ppe, q, p, fmask, s))) return rc;
     }
     const double *q[3] = {X[0], X[1], X[2]};
     return kl(pll_launch_correct_vel(&c->g, p, q, u, v, w, fmask, c->vel_force[0],
@@ -511,7 +502,7 @@ int pll_channel_step_from(pll_channel *c, pll_ppe *ppe, const double *const src[
     if ((rc = kl(pll_launch_rk12(&c->g, src, tmp, NULL, fmask ? c->part : NULL, fmask, 0.0, 0.0,
                                  NULL, body, s),
                  "rk1 + rk2")) ||
-        (rc = forcing_means(c, fmask, s)) || (rc = solve_unfilled(c, ppe, q, p, s)))
+        (rc = solve_unfilled(c, ppe, q, p, fmask, s)))
         return rc;
     return kl(pll_launch_correct_vel(&c->g, p, q, dst[0], dst[1], dst[2], fmask, c->vel_force[0],
                                      c->vel_force[1], mean, 1, s),

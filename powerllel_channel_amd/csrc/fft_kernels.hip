@@ -725,6 +725,7 @@ struct SrcDiv {  // PPE right-hand side formed from the velocity on the fly
 };
 struct SrcDivUnfilled {  // SrcDiv on a velocity whose boundary fill is not made
     static constexpr bool kLow = false;
+    static constexpr bool kMeans = true;
     pll_div_src q;
     long long off1, off2;
     int nx, ny, nz;
@@ -908,11 +909,11 @@ struct XArgs {
 // that each XCD runs one contiguous range of tiles puts neighbouring column
 // tiles (which share 128-byte lines when a tile row is narrower than a
 // line) on one L2.
-__device__ __forceinline__ unsigned xcd_block()
+__device__ __forceinline__ unsigned xcd_block(unsigned b, unsigned n)
 {
-    const unsigned b = blockIdx.x, n = gridDim.x;
     return (n & 7) ? b : (b & 7) * (n >> 3) + (b >> 3);
 }
+__device__ __forceinline__ unsigned xcd_block() { return xcd_block(blockIdx.x, gridDim.x); }
 
 // First row of an x kernel's workgroup (row = k ny + j).  With a.slab, XCD x
 // (= blockIdx & 7) takes the rows j in [x ny/8, (x+1) ny/8) of every plane,
@@ -923,14 +924,14 @@ __device__ __forceinline__ unsigned xcd_block()
 // neighbours, more than the 4 MB L2; round-robin splits the y neighbours
 // over XCDs.  Needs row0 = 0, nrows = ny nz and ny % (8 rows_per_wg) = 0.
 template <typename V>
-__device__ __forceinline__ long long x_row_first(const XArgs<V> &a)
+__device__ __forceinline__ long long x_row_first(const XArgs<V> &a, unsigned b, unsigned n)
 {
     if (a.slab) {
-        const unsigned b = blockIdx.x, x = b & 7, p = b >> 3;
+        const unsigned x = b & 7, p = b >> 3;
         const unsigned k = p / (unsigned)a.slab, q = p - k * (unsigned)a.slab;
         return (long long)k * a.ny + (long long)(x * (unsigned)a.slab + q) * a.rows_per_wg;
     }
-    return a.row0 + (long long)(a.xcd ? xcd_block() : blockIdx.x) * a.rows_per_wg;
+    return a.row0 + (long long)(a.xcd ? xcd_block(b, n) : b) * a.rows_per_wg;
 }
 
 // Sources that read neighbouring rows and planes (stencils) take the slab
@@ -943,6 +944,48 @@ template <class S>
 struct is_stencil<S, decltype((void)S::kStencil)> {
     static constexpr bool value = S::kStencil;
 };
+
+// Sources whose launch has a workgroup (the first) for Mean_h's partial sums.
+template <class S, class = void>
+struct has_means {
+    static constexpr bool value = false;
+};
+template <class S>
+struct has_means<S, decltype((void)S::kMeans)> {
+    static constexpr bool value = S::kMeans;
+};
+
+// That workgroup: mean[d] of the components in fmask.  The transform does not
+// need the result (the projection after the solve does), so the sums, a launch of
+// 4.6 us of their own otherwise, run beside it (step at 64x64x64 50.7 -> 48.3 us,
+// ten of 240x140x90 2.01 -> 1.95 ms).
+__device__ __forceinline__ void means_block(const pll_div_src &q, double nx, double ny, double *sh)
+{
+    const int t = threadIdx.x, nb = blockDim.x;
+    for (int d = 0; d < 2; ++d) {
+        if (!((q.fmask >> d) & 1)) continue;
+        const double *p = q.mpart + (long long)d * q.nmp;
+        double s = 0.0;
+        int i = t;
+        // eight partials in flight per thread, summed in pairs (fewer threads
+        // than k_mean_final, so as few additions in a row by this)
+        for (; i + 7 * nb < q.nmp; i += 8 * nb) {
+            double o[8];
+#pragma unroll
+            for (int r = 0; r < 8; ++r) o[r] = p[i + r * nb];
+            s += ((o[0] + o[1]) + (o[2] + o[3])) + ((o[4] + o[5]) + (o[6] + o[7]));
+        }
+        for (; i < q.nmp; i += nb) s += p[i];
+        sh[t] = s;
+        __syncthreads();
+        for (int h = 256; h > 0; h >>= 1) {  // at most 512 threads, any number
+            if (t < h && t + h < nb) sh[t] += sh[t + h];
+            __syncthreads();
+        }
+        if (t == 0) q.mean[d] = sh[0] / nx / ny;
+        __syncthreads();
+    }
+}
 
 template <typename V>
 struct YArgs {
@@ -990,9 +1033,20 @@ k_xfwd(Src src, V *__restrict__ W, const V *__restrict__ twr, XArgs<V> a)
     using S = typename Sc<V>::T;
     extern __shared__ unsigned char lds_raw[];
     constexpr int E = F::E;
+    unsigned b = blockIdx.x, n = gridDim.x;
+    if constexpr (has_means<Src>::value) {
+        if (src.q.mpart) {
+            if (b == 0) {
+                means_block(src.q, (double)src.nx, (double)src.ny,
+                            reinterpret_cast<double *>(lds_raw));
+                return;
+            }
+            --b, --n;
+        }
+    }
     const int T = F::threads(a.P), L = F::length(a.P);
     const int rl = threadIdx.x / T, t = threadIdx.x - rl * T;
-    const long long row = x_row_first(a) + rl;
+    const long long row = x_row_first(a, b, n) + rl;
     const bool valid = row < a.nrows;
     unsigned char *ml = lds_raw + (size_t)rl * a.pitch * lds_elem<F, V>();
     const long long j = valid ? row % a.ny : 0, k = valid ? row / a.ny : 0;
@@ -1101,7 +1155,7 @@ k_xbwd(const V *__restrict__ W, Dst dst, const V *__restrict__ twr, XArgs<V> a)
     constexpr int E = F::E;
     const int T = F::threads(a.P), L = F::length(a.P);
     const int rl = threadIdx.x / T, t = threadIdx.x - rl * T;
-    const long long row = x_row_first(a) + rl;
+    const long long row = x_row_first(a, blockIdx.x, gridDim.x) + rl;
     const bool valid = row < a.nrows;
     unsigned char *ml = lds_raw + (size_t)rl * a.pitch * lds_elem<F, V>();
     const long long j = valid ? row % a.ny : 0, k = valid ? row / a.ny : 0;
@@ -1392,7 +1446,8 @@ int launch_xf(const pll_ppe_dev *d, const void *tw, Src src, void *W, hipStream_
         a.nrows = row1;
     }
     const int threads = a.rows_per_wg * a.P.T;
-    const long long blocks = (a.nrows - a.row0 + a.rows_per_wg - 1) / a.rows_per_wg;
+    long long blocks = (a.nrows - a.row0 + a.rows_per_wg - 1) / a.rows_per_wg;
+    if constexpr (has_means<Src>::value) blocks += src.q.mpart != nullptr;
     const size_t shm = (size_t)a.rows_per_wg * a.pitch * lds_elem<F, V>();
     if (threads > max_threads_f<F, V>() || shm > 65536 || blocks > 0x7fffffffLL) return -1;
     a.xcd = d->x_xcd >= 2 || (d->x_xcd == 1 && sizeof(V) == sizeof(float2));

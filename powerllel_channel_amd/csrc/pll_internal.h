@@ -91,6 +91,12 @@ typedef struct {
      * what it would have left (u(0) = u(nx), v(j=0) = v(ny), w = 0 on the
      * wall rows k = 0 and nz) */
     int unfilled;
+    /* unfilled only, mpart NULL: none.  One workgroup more reduces the partial
+     * sums of Mean_h of component d (fmask bit d: u, v), nmp of them at
+     * mpart + d nmp, to mean[d] = sum / nx / ny */
+    const double *mpart;
+    int nmp, fmask;
+    double *mean;
 } pll_div_src;
 int pll_launch_xfwd_div(const pll_ppe_dev *d, const pll_div_src *q, void *W, hipStream_t s);
 

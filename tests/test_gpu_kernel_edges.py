@@ -325,3 +325,29 @@ def test_step_fills_boundary(orc, cuda, shape, forced, u_crf):
         for x, y in zip(a[:3], b):
             assert torch.isfinite(y).all()
             assert torch.equal(x, y)
+
+
+# Mean_h reduced by a workgroup of the x transform: fewer partial sums than
+# threads, thread counts that are no power of two, many partial sums
+@pytest.mark.parametrize("shape", [(4, 4, 2), (10, 6, 3), (66, 26, 17), (300, 140, 29),
+                                   (64, 256, 131), (384, 384, 66)])
+def test_forced_means(orc, cuda, shape):
+    """The forcing sets Mean_h of u and v.  Their partial sums run over at most
+    a few hundred terms each of size |u| <= 6 (and the pressure gradient's sum
+    telescopes), so the mean is off by less than 1000 roundings of 6: 1.4e-12."""
+    import torch
+    from powerllel_channel_amd import PoissonSolver
+    nx, ny, nz = shape
+    print(f"[forced means] {shape}", flush=True)
+    g, G, ch, (u, v, w, *_) = _channel(orc, nx, ny, nz, is_forced=(True, True, False),
+                                       vel_force=(1.0, 0.2, 0.0), dt=1e-4)
+    orc.bc_vel(G, u, v, w, 0.0)
+    z = np.zeros(g.shape)
+    s = PoissonSolver(nx, ny, nz, g.dx, g.dy, g.dzf)
+    for n in (1, 3):
+        a = _dev(torch, cuda, u, v, w, z, z, z, z)
+        ch.run(s, n, *a)
+        for q, m in ((a[0], 1.0), (a[1], 0.2)):
+            wk = torch.from_numpy(np.asarray(g.dzf[1:-1])).to(cuda).reshape(-1, 1, 1)
+            got = float((q[1:-1, 1:-1, 1:-1] * wk).sum() / wk.sum() / (nx * ny))
+            assert abs(got - m) < 1.4e-12, (n, got - m)
