@@ -1126,12 +1126,18 @@ static int host_setup(pll_ppe *h)
 {
     if (h->host_ready) return PLL_OK;
     const size_t plane = sizeof(double) * (size_t)(h->nx + 2) * (h->ny + 2);
-    /* slots of at most 20 MiB (whole planes): small chunks start the first
-     * transform and the last download sooner (768x384x256: 8 planes 24.0 ms
-     * per solve, 26 planes 25.3 ms) */
-    size_t cp = ((size_t)20 << 20) / plane;
+    /* Chunks: a copy and the transfer of the chunk before it run side by side, so
+     * only the first copy up and the last one down stand alone, and each chunk
+     * costs some 30 us of waits.  Five chunks, each of at least 6 and at most 20
+     * MiB (whole planes); us per solve, slots of 20 MiB against this: 128x128x96
+     * (2 chunks) 833 -> 700, 240x140x90 (3) 1426 -> 1180, 192x192x128 (5) 1838 ->
+     * 1740, 384x192x128 (5) 3309 -> 3300; 3 MiB chunks 748, 1309, 1962, 3353. */
+    const size_t all = plane * (size_t)h->nz;
+    size_t nch = all / ((size_t)6 << 20);
+    nch = nch < 1 ? 1 : nch > 5 ? 5 : nch;
+    size_t cp = ((size_t)h->nz + nch - 1) / nch;
+    if (cp > ((size_t)20 << 20) / plane) cp = ((size_t)20 << 20) / plane;
     if (cp < 1) cp = 1;
-    if (cp > (size_t)h->nz) cp = (size_t)h->nz;
     const char *pc = getenv("PLL_HOST_CHUNK"); /* tuning: planes per chunk */
     if (pc && atoi(pc) > 0) cp = (size_t)atoi(pc) < (size_t)h->nz ? (size_t)atoi(pc) : (size_t)h->nz;
     for (int i = 0; i < PLL_HOST_SLOTS; i++)

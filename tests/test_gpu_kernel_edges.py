@@ -351,3 +351,27 @@ def test_forced_means(orc, cuda, shape):
             wk = torch.from_numpy(np.asarray(g.dzf[1:-1])).to(cuda).reshape(-1, 1, 1)
             got = float((q[1:-1, 1:-1, 1:-1] * wk).sum() / wk.sum() / (nx * ny))
             assert abs(got - m) < 1.4e-12, (n, got - m)
+
+
+# host-pointer solves of one chunk, two, three and five uneven ones
+@pytest.mark.parametrize("shape", [(4, 4, 2), (128, 128, 97), (240, 140, 91), (192, 192, 129)])
+def test_host_solve_chunks(cuda, shape):
+    """The chunked host-pointer solve against the solve on the device."""
+    import torch
+    from powerllel_channel_amd import (PoissonSolver, execute_poisson_solver,
+                                       free_poisson_solver, init_poisson_solver)
+    from powerllel_channel_amd.mesh import Grid
+    from powerllel_channel_amd.workloads import LX, LY, LZ
+    print(f"[host chunks] {shape}", flush=True)
+    g = Grid(*shape, LX, LY, LZ, 1.5)
+    rhs = np.random.default_rng(3).standard_normal(g.shape)
+    d = torch.from_numpy(rhs.copy()).to(cuda)
+    PoissonSolver(*shape, g.dx, g.dy, g.dzf).solve(d)
+    init_poisson_solver(*shape, g.dx, g.dy, g.dzf)
+    try:
+        for _ in range(2):
+            h = rhs.copy()
+            execute_poisson_solver(h)
+            assert np.array_equal(h, d.cpu().numpy())
+    finally:
+        free_poisson_solver()
