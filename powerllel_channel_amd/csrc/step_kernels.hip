@@ -325,11 +325,12 @@ __global__ void __launch_bounds__(RK_TX *RK_TY, (FULL && !SECOND ? 4 : (SECOND &
 // Reads (qu, qv, qw) and writes (u, v, w), which may be the same arrays.
 // FILL: then the boundary fill of the result (k_bc_vel, which every ghost value
 // is a copy or reflection of one corrected cell in): a cell next to a face
-// stores its images too, and w's wall row is zero.  Against a pass of its own,
-// whose few threads wait for one strided load and store each: 64x64x64 6.4 +
-// 11.9 -> 8.2 us (step 64 -> 51 us), 256x192x128 70 + 21 -> 80 us.  The images
-// are a loop, not unrolled (nine kept addresses per field: 204 VGPRs, two waves
-// per SIMD).
+// stores its images too, and w's wall row is zero.  Bound by its memory traffic
+// (4.6 TB/s at 768x384x256; the next plane loaded ahead: 2% slower).  Against a
+// fill of its own, whose few threads wait for one strided load and store each:
+// 64x64x64 6.4 + 11.9 -> 8.2 us, 256x192x128 70 + 18 -> 72, 768x384x256 917 + 59
+// -> 980.  At 1536x1024x384 the images cost more than the pass (7.3 + 0.15 ms,
+// together 7.9), so grids above 2^27 cells take the two.
 template <bool FORCE, bool FILL>
 __global__ void __launch_bounds__(RK_TX *RK_TY) k_correct(G g, Tiles t, const double *__restrict__ p,
                                                           const double *qu, const double *qv,
@@ -352,27 +353,26 @@ __global__ void __launch_bounds__(RK_TX *RK_TY) k_correct(G g, Tiles t, const do
         if (fmask & 2) fv = vfv - mean[1];
     }
     // (un, vn, wn) at e and at the cell's images across the periodic faces
-    const bool edge = FILL && (i == 1 || i == g.nx || j == 1 || j == g.ny);
-    auto store = [&](long long a, double un, double vn, double wn) {
+    // (nx, ny >= 2: at most one in each direction)
+    const long long ox = i == 1 ? g.nx : (i == g.nx ? -g.nx : 0);
+    const long long oy = (j == 1 ? g.ny : (j == g.ny ? -g.ny : 0)) * sy;
+    auto put = [&](long long a, double un, double vn, double wn) {
         u[a] = un;
         v[a] = vn;
         w[a] = wn;
-        if (edge)
-#pragma unroll 1
-            for (int q = 0; q < 9; ++q) {
-                const int x = q % 3 - 1, y = q / 3 - 1;
-                if (q == 4 || (x > 0 && i != 1) || (x < 0 && i != g.nx) || (y > 0 && j != 1) ||
-                    (y < 0 && j != g.ny))
-                    continue;
-                const long long b = a + x * g.nx + y * g.ny * sy;
-                u[b] = un;
-                v[b] = vn;
-                w[b] = wn;
-            }
+    };
+    auto store = [&](long long a, double un, double vn, double wn) {
+        put(a, un, vn, wn);
+        if (FILL && ox) put(a + ox, un, vn, wn);
+        if (FILL && oy) {
+            put(a + oy, un, vn, wn);
+            if (ox) put(a + oy + ox, un, vn, wn);
+        }
     };
     const double bcu = 0.0 - g.u_crf;
     double pc = p[e];
     for (int k = k0; k <= k1; ++k, e += sz) {
+        if (FILL) asm volatile("" : "+v"(e));  // no kept address per field and image
         const double pz = p[e + sz];
         double un = qu[e] - (p[e + 1] - pc) * dtdxi;
         double vn = qv[e] - (p[e + sy] - pc) * dtdyi;
@@ -942,12 +942,14 @@ extern "C" int pll_launch_correct_vel(const pll_grid_dev *gd, const double *p,
     const double dtdxi = g.dt * g.dx_inv, dtdyi = g.dt * g.dy_inv;  // mod_calcVel.f90:436-437
     const dim3 grid((unsigned)(t.ntx * t.nty * t.nkc));
     const bool force = mean && fmask;
-    return with_flags(force, fill, false, [&](auto Fo, auto Fi, auto) {
+    const bool in = fill && (long long)g.nx * g.ny * g.nz <= 1LL << 27;
+    const int rc = with_flags(force, in, false, [&](auto Fo, auto Fi, auto) {
         hipLaunchKernelGGL((k_correct<decltype(Fo)::value, decltype(Fi)::value>), grid,
                            dim3(RK_TX * RK_TY), 0, s, g, t, p, q[0], q[1], q[2], u, v, w, dtdxi,
                            dtdyi, force ? fmask : 0, vfu, vfv, force ? mean : nullptr);
         return ok();
     });
+    return rc || !fill || in ? rc : pll_launch_bc_vel(gd, u, v, w, s);
 }
 
 extern "C" int pll_launch_mean_partials(const pll_grid_dev *gd, const double *q, double *part,
