@@ -43,7 +43,7 @@ struct Body {
 };
 
 // Projection of the input as it is read: correctVel with the forcing shift
-// and the boundary fill, as the projecting RK1 of step_kernels.hip forms it.
+// and the boundary fill.
 struct Proj {
     const double *p;
     double dtdxi, dtdyi;
