@@ -322,19 +322,27 @@ static int choose_launch(pll_ppe *h)
  * one wavefront), S columns per tile (16, 8 or 4 doubles = one 128/64/32-byte
  * row segment); LDS holds the tile twice (values and, for low-mode tiles,
  * pivots).  Returns 0 (streaming solve) if nothing fits. */
-static int part_fits(int nx, int nz, int m, int *M, int *P, int *S)
+static int part_fits(int nx, int ny, int nz, int m, int *M, int *P, int *S)
 {
     /* widest first: a tile row of 32 FP64 columns is 256 contiguous bytes,
      * which HBM serves faster than 128-byte pieces (768x384x256: 0.270 ->
-     * 0.253 ms against 16 columns, same box) */
+     * 0.253 ms against 16 columns, same box).  Not where W stays in the 256 MiB
+     * Infinity Cache and tiles are tall: there twice the tiles, two to a CU,
+     * hide each other's waits and leave a shorter last round.  us per solve, 32
+     * against 16 columns: 96x96x256 73 / 68, 192x192x128 88 / 85, 192x192x256
+     * 145 / 136, 512x384x128 370 / 348, refined 192x192x128 203 / 192; no gain
+     * up to 16 MiB or 96 planes (128x128x128 58.8 / 59.4, 384x192x96 117 / 120)
+     * and beyond the cache (512x256x256 462 / 462, 768x384x192 833 / 836). */
     static const int Ss[] = {32, 16, 8, 4};
+    const size_t w = sizeof(double) * (size_t)nx * ny * nz;
+    const int narrow = nz >= 128 && w > (size_t)16 << 20 && w <= (size_t)256 << 20;
     if (m <= 0 || nz % m || !pll_trid_part_supported(m)) return 0;
     const int p = nz / m;
     if (p < 2 || p > 64 || (p & (p - 1))) return 0;
     const char *ps = getenv("PLL_TRID_S"); /* tuning override of the tile width */
     for (size_t j = 0; j < sizeof Ss / sizeof Ss[0]; j++) {
         const int sc = Ss[j];
-        if (ps && atoi(ps) != sc) continue;
+        if (ps ? atoi(ps) != sc : narrow && sc == 32) continue;
         if (nx % sc || sc * p > 512 || (size_t)nz * sc * 8 + (size_t)nz * 24 + (size_t)p * 8 > 163840)
             continue;
         *M = m;
@@ -345,16 +353,16 @@ static int part_fits(int nx, int nz, int m, int *M, int *P, int *S)
     return 0;
 }
 
-static int choose_part(int nx, int nz, int *M, int *P, int *S)
+static int choose_part(int nx, int ny, int nz, int *M, int *P, int *S)
 {
     static const int Ms[] = {8, 12, 16, 4};
     const char *pm = getenv("PLL_TRID_M"); /* tuning override of the rows per lane */
-    if (pm) return part_fits(nx, nz, atoi(pm), M, P, S);
+    if (pm) return part_fits(nx, ny, nz, atoi(pm), M, P, S);
     /* prefer P = 16 lanes per column (one DPP row) unless PLL_TRID_DPP=0 */
     const char *pd = getenv("PLL_TRID_DPP");
-    if (!(pd && atoi(pd) == 0) && nz % 16 == 0 && part_fits(nx, nz, nz / 16, M, P, S)) return 1;
+    if (!(pd && atoi(pd) == 0) && nz % 16 == 0 && part_fits(nx, ny, nz, nz / 16, M, P, S)) return 1;
     for (size_t i = 0; i < sizeof Ms / sizeof Ms[0]; i++)
-        if (part_fits(nx, nz, Ms[i], M, P, S)) return 1;
+        if (part_fits(nx, ny, nz, Ms[i], M, P, S)) return 1;
     return 0;
 }
 
@@ -560,7 +568,7 @@ int pll_ppe_create(pll_ppe **out, int nx, int ny, int nz, double dx, double dy,
     h->d.dz = (const double *)h->bz + nz;
     {
         int M, P, S, rM, rP = 0, rS;
-        int part = choose_part(nx, nz, &M, &P, &S);
+        int part = choose_part(nx, ny, nz, &M, &P, &S);
         /* Ragged tiles where the regular layout does not exist, or has 4 columns
          * (32-byte row segments): 500x250x128 498 -> 442 us per solve, 100x100x64
          * 43 -> 40.  With 8 columns and more the regular one is faster:

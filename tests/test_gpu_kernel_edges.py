@@ -375,3 +375,31 @@ def test_host_solve_chunks(cuda, shape):
             assert np.array_equal(h, d.cpu().numpy())
     finally:
         free_poisson_solver()
+
+
+# 16-column z tiles on grids that stay in the Infinity Cache: one group per tile
+# (16 rows per lane) and two (8 and 12), just above the rule's lower end
+@pytest.mark.parametrize("shape", [(160, 128, 128), (96, 128, 192), (96, 96, 256), (64, 132, 256)])
+def test_narrow_z_tiles(cuda, shape, monkeypatch):
+    """The solve and its transpose against the streaming recurrence (1e-12, the
+    solve's tolerance), the refined solve against the FP64 one (1e-9 with one
+    sweep on these grids' wide tiles)."""
+    import torch
+    from powerllel_channel_amd import PoissonSolver
+    from powerllel_channel_amd.mesh import Grid
+    nx, ny, nz = shape
+    print(f"[narrow z tiles] {shape}", flush=True)
+    g = Grid(nx, ny, nz, 6.0, 3.0, 2.0, 2.0)
+    f = np.random.default_rng(12).standard_normal(g.shape)
+    wz = g.dzf[1:-1]
+    inner = (slice(1, -1),) * 3
+    f[inner] -= (f[inner].sum(axis=(1, 2)) * wz).sum() / (wz.sum() * nx * ny)
+    s = PoissonSolver(nx, ny, nz, g.dx, g.dy, g.dzf)
+    monkeypatch.setenv("PLL_TRID_STREAMING", "1")
+    streaming = PoissonSolver(nx, ny, nz, g.dx, g.dy, g.dzf)
+    for solve, tol in (("solve", 1e-12), ("solve_adjoint", 1e-12), ("solve_refined", 1e-9)):
+        p, q = _dev(torch, cuda, f, f)
+        getattr(s, solve)(p, *((1,) if solve == "solve_refined" else ()))
+        getattr(streaming, "solve" if solve == "solve_refined" else solve)(q)
+        a, b = p[inner], q[inner]
+        assert float((a - b).abs().max()) <= tol * float(b.abs().max()), solve
