@@ -268,6 +268,16 @@ static int choose_launch(pll_ppe *h)
     const pll_fftplan *px = &h->d.px, *py = &h->d.py;
     int maxt = pll_fft_max_threads(px->E);
     int rw = 256 / px->T;
+    /* small grids (2^21 cells): at most 16 rows, but a whole wavefront.  There a
+     * pass is as long as its workgroups, and barriers among fewer wavefronts are
+     * shorter; us per solve, 256 lanes against this: 40x40x40 27.6 -> 26.4,
+     * 64x64x64 23.5 -> 22.6, 96x96x96 45.6 -> 42.7, 128x128x128 59.1 -> 58.1,
+     * refined 96x96x96 100.5 -> 97.6; larger ones gain nothing or lose
+     * (192x192x128 85.6 / 84.7 but ten steps 2381 / 2400, 144x384x192 179 / 217) */
+    if ((long long)h->nx * h->ny * h->nz <= 1LL << 21) {
+        const int few = px->T < 4 ? 64 / px->T : 16;
+        if (rw > few) rw = few;
+    }
     {
         const char *pr = getenv("PLL_X_ROWS"); /* tuning override of the rows per workgroup */
         if (pr && atoi(pr) > 0) rw = atoi(pr);

@@ -403,3 +403,27 @@ def test_narrow_z_tiles(cuda, shape, monkeypatch):
         getattr(streaming, "solve" if solve == "solve_refined" else solve)(q)
         a, b = p[inner], q[inner]
         assert float((a - b).abs().max()) <= tol * float(b.abs().max()), solve
+
+
+# rows per workgroup of the x transforms: the rule's 16 and 64 / T, a single row,
+# counts that leave lanes of a wavefront and rows of a workgroup idle
+@pytest.mark.parametrize("shape", [(4, 4, 2), (10, 6, 5), (60, 50, 21), (64, 64, 64), (96, 30, 10)])
+def test_x_rows_bitwise(cuda, shape, monkeypatch):
+    """The solves do not depend on the rows per workgroup."""
+    import torch
+    from powerllel_channel_amd import PoissonSolver
+    from powerllel_channel_amd.mesh import Grid
+    print(f"[x rows] {shape}", flush=True)
+    g = Grid(*shape, 6.0, 3.0, 2.0, 2.0)
+    f = torch.from_numpy(np.random.default_rng(13).standard_normal(g.shape)).to(cuda)
+    got = []
+    for rows in (None, "1", "7", "64"):
+        if rows:
+            monkeypatch.setenv("PLL_X_ROWS", rows)
+        s = PoissonSolver(*shape, g.dx, g.dy, g.dzf)
+        p, q = f.clone(), f.clone()
+        s.solve(p)
+        s.solve_refined(q, 1)
+        got.append((p, q))
+    for p, q in got[1:]:
+        assert torch.equal(p, got[0][0]) and torch.equal(q, got[0][1])
