@@ -55,22 +55,24 @@ typedef struct {
     const double *bz;          /* [nz] diagonal before adding the eigenvalue */
     const double *dz;          /* [nz] row sums a + bz + c (zero up to rounding) */
     const double *piv;         /* [nz][ny/2+1][L+1] factorised diagonal */
-    struct {                   /* partitioned z solve (P = 0: streaming solve) */
+    /* partitioned z solve, in regular tiles (tp) or ragged ones (rg); where both
+     * are there, FP64 storage takes rg and FP32 tp; neither: streaming solve */
+    const double *lamx;        /* [L+1]    */
+    const double *lamy;        /* [ny/2+1] */
+    struct {                   /* P = 0: none */
         int M, P, S;           /* rows per lane, lanes per column, columns per tile */
         int dpp16;             /* P == 16: interface reduction by DPP row shifts */
         int qx, iyx;           /* tiles with q0 < qx and iy < iyx: exact path */
-        const double *bz;      /* [nz] diagonal before adding the eigenvalue */
-        const double *lamx;    /* [L+1]    */
-        const double *lamy;    /* [ny/2+1] */
         const int *order;      /* [tiles] launch order, exact tiles first */
         int h32;               /* FP32 storage: 2 = tiles of 2 S columns (0/1: S) */
         int h64;               /* FP64 storage: the same, at S = 16 only */
         int qx32;              /* qx for those tiles */
         const int *order32;    /* [nx/(2S) ny] their launch order */
-        int rag;               /* tiles of S columns of the plane's nx ny, P M >= nz
-                                  rows; order: ceil(nx ny / S) entries, exact tiles
-                                  marked (qx, iyx, h32, h64, order32 unused) */
     } tp;
+    struct {                   /* FP64 storage only; P = 0: none */
+        int M, P, S;           /* tiles of S columns of the plane's nx ny, P M >= nz rows */
+        const int *order;      /* [ceil(nx ny / S)] launch order, exact tiles marked */
+    } rg;
     /* refined form: the lowest modes (kx in {0,1}, ky in {0,1,ny-1}) of each
      * FP32 solve in FP64 (low_on = 0: off).  low_rx [ny nz][2] the x sums of
      * the FP64 rows, low_y [nz][6] their y sums, low_x [nz][6] the solved

@@ -195,7 +195,7 @@ struct pll_ppe {
     int nx, ny, nz, L;
     pll_ppe_dev d;
     void *W, *tw_x, *tw_y, *a, *c, *piv;
-    void *bz, *lamx, *lamy, *order, *order32;  /* partitioned z solve */
+    void *bz, *lamx, *lamy, *order, *order32, *rorder;  /* partitioned z solve */
     void *tw_x32, *tw_y32, *W32, *P64, *r32; /* refined form (allocated on first use) */
     void *gauge;                      /* top-plane partial sums + mean (refined form) */
     void *low_rx, *low_y, *low_x;     /* lowest modes in FP64 (refined form) */
@@ -232,13 +232,32 @@ static int dmalloc(pll_ppe *h, void **p, size_t bytes)
     return PLL_OK;
 }
 
+/* device copy of a host table */
+static int upload(pll_ppe *h, void **p, const void *src, size_t bytes)
+{
+    const int rc = dmalloc(h, p, bytes);
+    if (rc) return rc;
+    const hipError_t e = hipMemcpy(*p, src, bytes, hipMemcpyHostToDevice);
+    return e == hipSuccess ? PLL_OK
+                           : pll_set_error(PLL_EHIP, "hipMemcpy H2D failed: %s", hipGetErrorString(e));
+}
+
+/* device copy of a tile list of n entries, which is freed (NULL: out of memory) */
+static int put_order(pll_ppe *h, void **p, int *order, int n)
+{
+    const int rc = order ? upload(h, p, order, sizeof(int) * (size_t)n)
+                         : pll_set_error(PLL_ENOMEM, "host allocation failed");
+    free(order);
+    return rc;
+}
+
 int pll_ppe_destroy(pll_ppe *h)
 {
     if (!h) return PLL_OK;
     void *bufs[] = {h->W, h->tw_x, h->tw_y, h->a, h->c, h->piv, h->stage,
                     h->bz, h->lamx, h->lamy, h->order, h->tw_x32, h->tw_y32,
                     h->W32, h->P64, h->r32, h->gauge, h->nrm, h->low_rx, h->low_y,
-                    h->low_x, h->order32};
+                    h->low_x, h->order32, h->rorder};
     for (size_t i = 0; i < sizeof bufs / sizeof bufs[0]; i++)
         if (bufs[i]) hipFree(bufs[i]);
     if (h->timing)
@@ -579,21 +598,23 @@ int pll_ppe_create(pll_ppe **out, int nx, int ny, int nz, double dx, double dy,
     {
         int M, P, S, rM, rP = 0, rS;
         int part = choose_part(nx, ny, nz, &M, &P, &S);
-        /* Ragged tiles where the regular layout does not exist, or has 4 columns
-         * (32-byte row segments): 500x250x128 498 -> 442 us per solve, 100x100x64
-         * 43 -> 40.  With 8 columns and more the regular one is faster:
+        /* Ragged tiles for FP64 where the regular layout does not exist, or has 4
+         * columns (32-byte row segments): 500x250x128 498 -> 442 us per solve,
+         * 100x100x64 43 -> 40.  With 8 columns and more the regular one is faster:
          * 360x128x128 159 us (ragged 166), 400x256x128 242 (257).
-         * PLL_TRID_RAG (tuning): 0 never, 1 always */
+         * PLL_TRID_RAG (tuning): 0 never, 1 always and nothing else */
         const char *pr = getenv("PLL_TRID_RAG");
         int rag = choose_rag(nz, &rM, &rP, &rS) && (pr ? atoi(pr) != 0 : !part || S < 8);
-        if (rag) {
-            M = rM;
-            P = rP;
-            S = rS;
-            part = 1;
-        }
-        if (!getenv("PLL_TRID_STREAMING") && part) {
-            const int ntx = nx / S, ntiles = rag ? (nx * ny + S - 1) / S : ntx * ny;
+        /* FP32 storage then keeps the regular tiles of 4 columns: a workgroup of
+         * 4 P lanes, against the streaming solve's one lane per two columns and one
+         * chain of nz rows, which many columns and few planes favour.  us per
+         * refined solve with one sweep, streaming against regular: P = 16
+         * 100x100x64 159 / 77, 500x250x128 817 / 727, 900x400x128 1969 / 1712,
+         * 660x330x128 1478 / 1516, 1500x500x128 4275 / 5038; P = 8 500x250x96
+         * 573 / 529, 660x330x96 1115 / 1162; P = 4 300x150x48 192 / 155,
+         * 900x400x48 727 / 834; P = 2 100x100x16 82 / 72, 500x250x16 133 / 192 */
+        if (rag) part = part && !pr && (long long)nx * ny <= 24576LL * P;
+        if (!getenv("PLL_TRID_STREAMING") && (part || rag)) {
             /* exact-path thresholds: |lambda| < tau * max|bz| */
             double bmax = 0.0;
             for (int k = 0; k < nz; k++) bmax = fabs(bz[k]) > bmax ? fabs(bz[k]) : bmax;
@@ -602,85 +623,59 @@ int pll_ppe_create(pll_ppe **out, int nx, int ny, int nz, double dx, double dy,
             while (iyx < nyh && fabs(ly[iyx]) < thr) iyx++;
             int ixmax = -1;
             while (ixmax + 1 <= L && fabs(lx[ixmax + 1]) < thr) ixmax++;
-            int qx = iyx > 0 ? 2 * (ixmax + 1) : 0;
-            const int qx0 = qx;
-            qx = ((qx0 + S - 1) / S) * S;
-            int *order = rag ? rag_order(nx, ny, S, qx0, iyx) : tile_order(nx, ny, S, qx, iyx);
-            if (!order) {
-                rc = pll_set_error(PLL_ENOMEM, "host allocation failed");
+            const int qx0 = iyx > 0 ? 2 * (ixmax + 1) : 0;
+            if ((rc = upload(h, &h->lamx, lx, sizeof(double) * (size_t)(L + 1))) ||
+                (rc = upload(h, &h->lamy, ly, sizeof(double) * (size_t)nyh)))
                 goto fail;
-            }
-            /* FP32 storage: tiles of 2 S columns (256-byte row segments at
-             * S = 32), if their LDS fits (PLL_TRID32_H=1: S columns) */
-            const char *ph = getenv("PLL_TRID32_H");
-            const int h32 = (!rag && S >= 16 && nx % (2 * S) == 0 &&
-                             (size_t)nz * 2 * S * 8 + (size_t)nz * 24 + (size_t)P * 8 <= 163840 &&
-                             !(ph && atoi(ph) == 1)) ? 2 : 1;
-            const int qx32 = ((qx0 + 2 * S - 1) / (2 * S)) * (2 * S);
-            if (h32 == 2) {
-                int *order32 = tile_order(nx, ny, 2 * S, qx32, iyx);
-                if (!order32 || (rc = dmalloc(h, &h->order32, sizeof(int) * (size_t)(ntiles / 2)))) {
-                    free(order32);
-                    free(order);
-                    if (!rc) rc = pll_set_error(PLL_ENOMEM, "host allocation failed");
+            h->d.lamx = (const double *)h->lamx;
+            h->d.lamy = (const double *)h->lamy;
+            if (rag) {
+                if ((rc = put_order(h, &h->rorder, rag_order(nx, ny, rS, qx0, iyx),
+                                    (nx * ny + rS - 1) / rS)))
                     goto fail;
-                }
-                const hipError_t e32 = hipMemcpy(h->order32, order32, sizeof(int) * (size_t)(ntiles / 2),
-                                                 hipMemcpyHostToDevice);
-                free(order32);
-                if (e32 != hipSuccess) {
-                    free(order);
-                    rc = pll_set_error(PLL_EHIP, "copy of z-solve tables failed");
+                h->d.rg.M = rM;
+                h->d.rg.P = rP;
+                h->d.rg.S = rS;
+                h->d.rg.order = (const int *)h->rorder;
+            }
+            if (part) {
+                const int ntiles = nx / S * ny;
+                const int qx = ((qx0 + S - 1) / S) * S;
+                /* FP32 storage: tiles of 2 S columns (256-byte row segments at
+                 * S = 32), if their LDS fits (PLL_TRID32_H=1: S columns) */
+                const char *ph = getenv("PLL_TRID32_H");
+                const int h32 = (S >= 16 && nx % (2 * S) == 0 &&
+                                 (size_t)nz * 2 * S * 8 + (size_t)nz * 24 + (size_t)P * 8 <= 163840 &&
+                                 !(ph && atoi(ph) == 1)) ? 2 : 1;
+                const int qx32 = ((qx0 + 2 * S - 1) / (2 * S)) * (2 * S);
+                if ((rc = put_order(h, &h->order, tile_order(nx, ny, S, qx, iyx), ntiles)) ||
+                    (h32 == 2 && (rc = put_order(h, &h->order32,
+                                                 tile_order(nx, ny, 2 * S, qx32, iyx), ntiles / 2))))
                     goto fail;
+                h->d.tp.h32 = h32;
+                {
+                    /* FP64 storage: two 16-column groups make the 256-byte row
+                     * segments that 32-column tiles give where P = 32 lanes per
+                     * column leave room for 16 columns only (nz = 384); at M = 16
+                     * rows per lane the second group's values would spill
+                     * (PLL_TRID64_H=1: one group) */
+                    const char *p64 = getenv("PLL_TRID64_H");
+                    h->d.tp.h64 =
+                        (h32 == 2 && S == 16 && M <= 12 && !(p64 && atoi(p64) == 1)) ? 2 : 1;
                 }
+                h->d.tp.qx32 = qx32;
+                h->d.tp.order32 = (const int *)h->order32;
+                h->d.tp.M = M;
+                h->d.tp.P = P;
+                h->d.tp.S = S;
+                {
+                    const char *pd = getenv("PLL_TRID_DPP");
+                    h->d.tp.dpp16 = (P == 16) && !(pd && atoi(pd) == 0);
+                }
+                h->d.tp.qx = qx;
+                h->d.tp.iyx = iyx;
+                h->d.tp.order = (const int *)h->order;
             }
-            h->d.tp.h32 = h32;
-            {
-                /* FP64 storage: two 16-column groups make the 256-byte row
-                 * segments that 32-column tiles give where P = 32 lanes per
-                 * column leave room for 16 columns only (nz = 384); at M = 16
-                 * rows per lane the second group's values would spill
-                 * (PLL_TRID64_H=1: one group) */
-                const char *p64 = getenv("PLL_TRID64_H");
-                h->d.tp.h64 =
-                    (h32 == 2 && S == 16 && M <= 12 && !(p64 && atoi(p64) == 1)) ? 2 : 1;
-            }
-            h->d.tp.qx32 = qx32;
-            h->d.tp.order32 = (const int *)h->order32;
-            double *lxh = (double *)malloc(sizeof(double) * (size_t)(L + 1));
-            if (!lxh) {
-                free(order);
-                rc = pll_set_error(PLL_ENOMEM, "host allocation failed");
-                goto fail;
-            }
-            for (int i = 0; i <= L; i++) lxh[i] = lx[i];
-            if ((rc = dmalloc(h, &h->lamx, sizeof(double) * (size_t)(L + 1))) ||
-                (rc = dmalloc(h, &h->lamy, sizeof(double) * (size_t)nyh)) ||
-                (rc = dmalloc(h, &h->order, sizeof(int) * (size_t)ntiles)) ||
-                (hipMemcpy(h->lamx, lxh, sizeof(double) * (size_t)(L + 1), hipMemcpyHostToDevice) != hipSuccess) ||
-                (hipMemcpy(h->lamy, ly, sizeof(double) * (size_t)nyh, hipMemcpyHostToDevice) != hipSuccess) ||
-                (hipMemcpy(h->order, order, sizeof(int) * (size_t)ntiles, hipMemcpyHostToDevice) != hipSuccess)) {
-                free(order);
-                free(lxh);
-                if (!rc) rc = pll_set_error(PLL_EHIP, "copy of z-solve tables failed");
-                goto fail;
-            }
-            free(order);
-            free(lxh);
-            h->d.tp.rag = rag;
-            h->d.tp.M = M;
-            h->d.tp.P = P;
-            h->d.tp.S = S;
-            {
-                const char *pd = getenv("PLL_TRID_DPP");
-                h->d.tp.dpp16 = (P == 16) && !(pd && atoi(pd) == 0);
-            }
-            h->d.tp.qx = qx;
-            h->d.tp.iyx = iyx;
-            h->d.tp.bz = (const double *)h->bz;
-            h->d.tp.lamx = (const double *)h->lamx;
-            h->d.tp.lamy = (const double *)h->lamy;
-            h->d.tp.order = (const int *)h->order;
         }
     }
     free(a); free(c); free(bz); free(lx); free(ly); free(piv); free(twx); free(twy);

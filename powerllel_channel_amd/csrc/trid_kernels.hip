@@ -577,34 +577,35 @@ unsigned persistent_grid(const void *fn, int threads, size_t shm, int ntiles)
     return (unsigned)(n < ntiles ? n : ntiles);
 }
 
-// FP64 storage only.  FP32 storage on such grids keeps the streaming solve: with
-// ragged tiles the error left after one refinement sweep is 13 +- 5% larger
-// (150 right-hand sides on six grids; 515 for 773 us at 360x200x150).
+// FP64 storage only.  FP32 storage on such grids keeps the regular tiles, if there
+// are any, or the streaming solve: with ragged tiles the error left after one
+// refinement sweep is 13 +- 5% larger (150 right-hand sides on six grids; 515
+// for 773 us at 360x200x150).
 int launch_rag(const pll_ppe_dev *d, void *W, hipStream_t s)
 {
     using St = double;
     PArgs g;
     g.a = d->a;
     g.c = d->c;
-    g.bz = d->tp.bz;
-    g.lamx = d->tp.lamx;
-    g.lamy = d->tp.lamy;
+    g.bz = d->bz;
+    g.lamx = d->lamx;
+    g.lamy = d->lamy;
     g.piv = d->piv;
-    g.order = d->tp.order;
+    g.order = d->rg.order;
     g.L = d->L;
     g.nx = d->nx;
     g.ny = d->ny;
     g.nz = d->nz;
-    g.P = d->tp.P;
+    g.P = d->rg.P;
     g.lP = 0;
     while ((1 << g.lP) < g.P) g.lP++;
-    g.S = d->tp.S;
+    g.S = d->rg.S;
     g.ncol = d->nx * d->ny;
     g.ntx = 1;
     g.ntiles = (g.ncol + g.S - 1) / g.S;
     g.pin_gauge = d->pin_gauge;
     g.qx = g.iyx = 0;
-    const int M = d->tp.M, threads = g.S * g.P;
+    const int M = d->rg.M, threads = g.S * g.P;
     const size_t shm = sizeof(double) * ((size_t)M * g.P * g.S + (3 * (size_t)M + 1) * g.P);
     if ((1 << g.lP) != g.P || M * g.P < d->nz || threads > 512 || shm > 163840 || !g.order) return -1;
 #define PLL_RAG_L(M_, S_, D_)                                                                      \
@@ -643,8 +644,8 @@ int launch_rag(const pll_ppe_dev *d, void *W, hipStream_t s)
 template <typename St, typename C>
 int launch_trid(const pll_ppe_dev *d, void *W, hipStream_t s)
 {
-    if (d->tp.rag && sizeof(St) == sizeof(double)) return launch_rag(d, W, s);
-    if (d->tp.P > 0 && !d->tp.rag) {
+    if (d->rg.P > 0 && sizeof(St) == sizeof(double)) return launch_rag(d, W, s);
+    if (d->tp.P > 0) {
         // FP32 storage with wide tiles: H = 2 groups of S columns per tile
         const int H = ((sizeof(St) == sizeof(float) ? d->tp.h32 : d->tp.h64) == 2) ? 2 : 1;
         // H = 2: FP32 storage at S = 16 and 32, FP64 storage at S = 16 only (FP64
@@ -653,9 +654,9 @@ int launch_trid(const pll_ppe_dev *d, void *W, hipStream_t s)
         PArgs g;
         g.a = d->a;
         g.c = d->c;
-        g.bz = d->tp.bz;
-        g.lamx = d->tp.lamx;
-        g.lamy = d->tp.lamy;
+        g.bz = d->bz;
+        g.lamx = d->lamx;
+        g.lamy = d->lamy;
         g.piv = d->piv;
         g.order = H == 2 ? d->tp.order32 : d->tp.order;
         g.L = d->L;

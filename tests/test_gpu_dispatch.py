@@ -1,0 +1,50 @@
+"""Which kernel a solve takes where several could, against a solver that is
+held to one of them."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+# nx a multiple of 4 but not of 8: FP32 sweeps on regular tiles of 4 columns (2 to
+# 64 lanes per column), streaming above 24576 columns per lane; FP64 ragged
+@pytest.mark.parametrize("shape,held", [
+    ((20, 12, 16), "PLL_TRID_RAG=0"), ((12, 14, 48), "PLL_TRID_RAG=0"),
+    ((100, 10, 64), "PLL_TRID_RAG=0"), ((28, 6, 96), "PLL_TRID_RAG=0"),
+    ((20, 16, 128), "PLL_TRID_RAG=0"), ((12, 8, 192), "PLL_TRID_RAG=0"),
+    ((36, 6, 256), "PLL_TRID_RAG=0"), ((12, 6, 512), "PLL_TRID_RAG=0"),
+    ((260, 192, 16), "PLL_TRID_STREAMING=1")])
+def test_refined_z_tiles_of_4_columns(cuda, shape, held, monkeypatch):
+    """The refined solve is bit for bit that of a solver held to the z solve the
+    rule names; the FP64 solve and its transpose agree with the streaming
+    recurrence (1e-12, the solve's tolerance)."""
+    import torch
+    from powerllel_channel_amd import PoissonSolver
+    from powerllel_channel_amd.mesh import Grid
+    nx, ny, nz = shape
+    print(f"[refined, 4-column z tiles] {shape}", flush=True)
+    g = Grid(nx, ny, nz, 6.0, 3.0, 2.0, 2.0)
+    f = np.random.default_rng(17).standard_normal(g.shape)
+    wz = g.dzf[1:-1]
+    inner = (slice(1, -1),) * 3
+    f[inner] -= (f[inner].sum(axis=(1, 2)) * wz).sum() / (wz.sum() * nx * ny)
+
+    def solver(env=None):
+        if env:
+            monkeypatch.setenv(*env.split("="))
+        s = PoissonSolver(nx, ny, nz, g.dx, g.dy, g.dzf)
+        if env:
+            monkeypatch.delenv(env.split("=")[0])
+        return s
+
+    def run(s, name, *args):
+        p = torch.from_numpy(f.copy()).to(cuda)
+        getattr(s, name)(p, *args)
+        return p[inner]
+    default, alone, streaming = solver(), solver(held), solver("PLL_TRID_STREAMING=1")
+    for sweeps in (0, 1):
+        assert torch.equal(run(default, "solve_refined", sweeps),
+                           run(alone, "solve_refined", sweeps)), sweeps
+    for name in ("solve", "solve_adjoint"):
+        a, b = run(default, name), run(streaming, name)
+        assert float((a - b).abs().max()) <= 1e-12 * float(b.abs().max()), name
