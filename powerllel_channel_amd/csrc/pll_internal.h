@@ -181,8 +181,10 @@ int pll_fft_max_threads32(int E);
 /* compile-time plan for length L, if one exists (returns 1 and fills p);
  * among several, the one with E == prefer_E, else the first listed */
 int pll_fft_ct_plan(int L, int prefer_E, pll_fftplan *p);
-/* the plan the solver uses for length L (host only): E, stage count, radices */
+/* the plan the solver uses for an x transform of length L, a y transform of
+ * length ny (host only): E, stage count, radices */
 int pll_fft_plan_info(int L, int *E, int *nst, int *rad);
+int pll_fft_plan_info_y(int ny, int *E, int *nst, int *rad);
 
 /* Grid constants for the step kernels (device pointers for z arrays). */
 typedef struct {

@@ -10,6 +10,7 @@
  * evaluated here with the reference's formulas.  The solver state stays on
  * the GPU for the lifetime of the handle.
  */
+#include <limits.h>
 #include <math.h>
 #include <stdarg.h>
 #include <stdio.h>
@@ -80,7 +81,10 @@ static int plan_for_E(int L, int E, const int cnt[4], const int cnt_big[2], int 
     return 1;
 }
 
-/* maxT: threads per transform that the kernel would rather not exceed */
+/* Threads per transform that the kernels would rather not exceed: a workgroup of x
+ * rows, a y tile of 8 columns. */
+enum { PLL_MAXT_X = 256, PLL_MAXT_Y = 64 };
+
 static int make_plan(int L, int maxT, pll_fftplan *p)
 {
     memset(p, 0, sizeof *p);
@@ -100,7 +104,7 @@ static int make_plan(int L, int maxT, pll_fftplan *p)
                              "FFT length %d has a prime factor above 13 (radices 2, 3, 5, 7, "
                              "11 and 13 are supported)", L);
     const int cnt[4] = {c6[0], c6[1], c6[2], c6[3]}, big[2] = {c6[4], c6[5]};
-    /* Points per thread, first fit:
+    /* Points per thread E, first fit in a class's list:
      * - lengths below 128: few (3 below 100, else 4), so that a row has lanes
      *   enough to read long pieces and small grids have threads enough, whether
      *   or not stages go through LDS (solves, 12 points -> this: 72x36x64 41 ->
@@ -108,23 +112,42 @@ static int make_plan(int L, int maxT, pll_fftplan *p)
      * - longer ones with a factor 5: 5 (4 -> 5: 240x140x90 90 -> 81, 320x160x64 90
      *   -> 78, 640x320x64 265 -> 226; below 120 4 is faster, 200x100x64 52 for 56);
      * - other longer ones: all stages in registers (288x144x64, 576x288x64: 87 and
-     *   229 us with 12, 88 and 238 with 4), else 4. */
-    static const int Es[4][9] = {{3, 4, 6, 5, 8, 7, 2, 12, 24}, {4, 3, 6, 5, 8, 7, 2, 12, 24},
-                                 {5, 4, 6, 8, 12, 3, 7, 24, 2}, {12, 8, 24, 6, 4, 3, 5, 7, 2}};
-    const int small = L < 128 && !(L % 5 == 0 && L >= 120);
-    const int first = small ? (L < 100 ? 0 : 1) : (L % 5 == 0 ? 2 : 3);
-    for (int pass = 0; pass < 3; pass++) {
-        /* stages in registers only; any stages, at most maxT threads; any */
-        if (pass == 0 && first != 3) continue;
-        const int *es = pass == 0 || first != 3 ? Es[first] : Es[1];
-        for (int ie = 0; ie < 9; ie++) {
-            const int E = es[ie];
-            if (L % E != 0 || !pll_fft_supported_E(E) || L / E > pll_fft_max_threads(E)) continue;
-            if (pass == 1 && L / E > maxT) continue;
+     *   229 us with 12, 88 and 238 with 4), else 4;
+     * - lengths with a factor 11 or 13, any size: many, 12, 8 or 6, as long as a
+     *   workgroup holds two rows: the registers that the large butterflies need
+     *   are there either way (both y passes at 256 x ny x 64, 3 to 5 points
+     *   against this: 104 40 / 33 us, 312 89 / 55, 462 149 / 98, 832 224 / 155,
+     *   1092 494 / 202; x passes at 2 L x 128 x 64: 330 109 / 84, 660 254 / 149,
+     *   1404 390 / 298; the one case the other way, x at 1040: 308 / 343).
+     * Then the width of a y tile: at most 64 threads a column leave room for 8
+     * columns (4 from 12 points on); where no E of the list does that, tiles of
+     * two columns and more are wide enough for fewer points to be faster (640: 4
+     * columns of 5 points 92 us, 6 of 8 117), but one column, 16 bytes of a row,
+     * is not (1400: 5 points 361, 8 points 318; 1440: 402, with 12 295; 1568: 4
+     * points 394, 8 points 351).
+     * 24 points take 228 registers, two waves per SIMD (960: 245, with 5 160;
+     * x 3360: 1678, with 8 1010): only where nothing else divides the length. */
+    static const int few100[9] = {3, 4, 6, 5, 8, 7, 2, 12}, few[9] = {4, 6, 3, 5, 8, 7, 2, 12},
+                     five[9] = {5, 4, 6, 8, 12, 3, 7, 2}, regs[9] = {12, 8, 24, 6, 4, 3, 5, 7, 2},
+                     twice[9] = {5, 4, 12, 8, 6, 7, 3, 2}, many[9] = {12, 8, 6, 5, 3, 7, 4, 2},
+                     one[9] = {12, 6, 4, 3, 5, 8, 7, 2}, last[9] = {24};
+    const int large = c6[4] || c6[5], small = L < 128 && !(L % 5 == 0 && L >= 120);
+    const int *list = small ? (L < 100 ? few100 : few) : (L % 5 == 0 ? five : few);
+    const struct { const int *list; int reg_only, maxT, half; } pass[5] = {
+        /* stages in registers only; at most maxT threads; room for two rows; any */
+        {!large && !small && L % 5 ? regs : NULL, 1, INT_MAX, 0},
+        {large ? NULL : list, 0, maxT, 0},
+        {large ? many : twice, 0, INT_MAX, 1},
+        {large ? one : list, 0, INT_MAX, 0},
+        {last, 0, INT_MAX, 0}};
+    for (int i = 0; i < 5; i++)
+        for (const int *e = pass[i].list; e && e < pass[i].list + 9 && *e; e++) {
+            const int E = *e, T = L / E;
+            if (L % E != 0 || !pll_fft_supported_E(E)) continue;
+            if (T > pass[i].maxT || (pass[i].half ? 2 * T : T) > pll_fft_max_threads(E)) continue;
             if (want > 0 && E != want && L % want == 0) continue;
-            if (plan_for_E(L, E, cnt, big, pass == 0, p)) return PLL_OK;
+            if (plan_for_E(L, E, cnt, big, pass[i].reg_only, p)) return PLL_OK;
         }
-    }
     return pll_set_error(PLL_EUNSUP, "no FFT plan for length %d", L);
 }
 
@@ -508,7 +531,7 @@ int pll_ppe_create(pll_ppe **out, int nx, int ny, int nz, double dx, double dy,
     h->nz = nz;
     h->L = nx / 2;
     int rc;
-    if ((rc = make_plan(h->L, 256, &h->d.px)) || (rc = make_plan(ny, 64, &h->d.py)) ||
+    if ((rc = make_plan(h->L, PLL_MAXT_X, &h->d.px)) || (rc = make_plan(ny, PLL_MAXT_Y, &h->d.py)) ||
         (rc = choose_launch(h))) {
         free(h);
         return rc;
@@ -1292,15 +1315,26 @@ void execute_poisson_solver(double *var)
 
 void free_poisson_solver(void) { abort_on(free_poisson_solver_status(), "free_poisson_solver"); }
 
-/* Host-only query of the FFT plan chosen for length L (no device needed):
- * points per thread, stage count and radices (rad: PLL_MAX_STAGES ints). */
-int pll_fft_plan_info(int L, int *E, int *nst, int *rad)
+/* Host-only query of the plan the solver uses for an x transform of length L
+ * (= nx/2) or a y transform of length ny (no device needed): points per thread,
+ * stage count and radices (rad: PLL_MAX_STAGES ints). */
+static int plan_info(int L, int maxT, int *E, int *nst, int *rad)
 {
     pll_fftplan p;
-    const int rc = make_plan(L, 256, &p);
+    const int rc = make_plan(L, maxT, &p);
     if (rc) return rc;
     *E = p.E;
     *nst = p.nst;
     for (int s = 0; s < p.nst; s++) rad[s] = p.rad[s];
     return PLL_OK;
+}
+
+int pll_fft_plan_info(int L, int *E, int *nst, int *rad)
+{
+    return plan_info(L, PLL_MAXT_X, E, nst, rad);
+}
+
+int pll_fft_plan_info_y(int ny, int *E, int *nst, int *rad)
+{
+    return plan_info(ny, PLL_MAXT_Y, E, nst, rad);
 }

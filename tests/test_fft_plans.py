@@ -1,0 +1,63 @@
+"""Points per thread that the transform plans take (no GPU needed)."""
+import ctypes as C
+
+import pytest
+
+
+@pytest.fixture(scope="module")
+def lib():
+    from powerllel_channel_amd import lib as L
+    return L()
+
+
+def _points(fn, L):
+    E, n, rad = C.c_int(), C.c_int(), (C.c_int * 12)()
+    return E.value if fn(L, C.byref(E), C.byref(n), rad) == 0 else 0
+
+
+def _smooth(L, primes):
+    for q in primes:
+        while L % q == 0:
+            L //= q
+    return L == 1
+
+
+def _limit(E):
+    return 256 if E >= 12 else 512
+
+
+ALL = (2, 3, 4, 5, 6, 7, 8, 12, 24)
+
+
+@pytest.mark.parametrize("axis", ["x", "y"])
+def test_plan_points_per_thread(lib, axis):
+    """Of a length's usable points per thread E (E divides it, at most 512
+    threads a row, 256 from E = 12 on): 24 only where nothing else is usable;
+    y tiles of two columns and more where any E but 24 gives them (from 128
+    on); with a factor 11 or 13, the first of 12, 8, 6 that leaves room for two
+    rows in a workgroup.  Lengths 2^a 3^b have plans of their own."""
+    fn = lib.pll_fft_plan_info if axis == "x" else lib.pll_fft_plan_info_y
+    for L in range(2, 4096 if axis == "x" else 5120, 1 if axis == "x" else 2):
+        usable = [E for E in ALL if L % E == 0 and L // E <= _limit(E)]
+        E = _points(fn, L)
+        assert (E in usable) == (_smooth(L, (2, 3, 5, 7, 11, 13)) and bool(usable)), L
+        if not E or _smooth(L, (2, 3)):
+            continue
+        assert E != 24 or usable == [24], (L, E)
+        two = [e for e in usable if e != 24 and 2 * (L // e) <= _limit(e)]
+        if axis == "y" and L >= 128 and two:
+            assert E in two, (L, E, two)
+        if not _smooth(L, (2, 3, 5, 7)):
+            first = [e for e in (12, 8, 6) if e in two]
+            assert not first or E == first[0], (L, E, first)
+
+
+@pytest.mark.parametrize("axis,L,E", [
+    ("y", 640, 5), ("y", 800, 5), ("y", 960, 5), ("y", 1344, 12), ("y", 1400, 8),
+    ("y", 1568, 8), ("y", 126, 6), ("y", 462, 6), ("y", 832, 8), ("y", 936, 12),
+    ("x", 126, 6), ("x", 294, 6), ("x", 660, 12), ("x", 726, 6), ("x", 1500, 6),
+    ("x", 1300, 4), ("x", 1584, 8), ("x", 3360, 8)])
+def test_plan_measured(lib, axis, L, E):
+    """Lengths on either side of the rule's lines, as they were measured."""
+    fn = lib.pll_fft_plan_info if axis == "x" else lib.pll_fft_plan_info_y
+    assert _points(fn, L) == E

@@ -48,3 +48,32 @@ def test_refined_z_tiles_of_4_columns(cuda, shape, held, monkeypatch):
     for name in ("solve", "solve_adjoint"):
         a, b = run(default, name), run(streaming, name)
         assert float((a - b).abs().max()) <= 1e-12 * float(b.abs().max()), name
+
+
+# transform plans: lengths with a factor 11 or 13 at 12, 8, 7, 6 and 4 points per
+# thread, long y transforms in tiles of two columns and of one
+@pytest.mark.parametrize("shape", [
+    (132, 66, 4), (264, 156, 3), (176, 104, 4), (462, 78, 3), (660, 132, 3), (252, 126, 4),
+    (12, 1400, 3), (20, 1344, 2), (16, 960, 3), (8, 1300, 2), (24, 1764, 2), (10, 1560, 2)])
+def test_plans_against_oracle(orc, cuda, shape):
+    """Solve against the oracle (1e-12) and the refined form with two sweeps
+    (1e-11, its bar)."""
+    import torch
+    from powerllel_channel_amd import PoissonSolver
+    from powerllel_channel_amd.mesh import Grid
+    nx, ny, nz = shape
+    print(f"[plans] {shape}", flush=True)
+    g = Grid(nx, ny, nz, 0.05 * nx, 0.05 * ny, 2.0, 1.0)
+    f = np.random.default_rng(19).standard_normal(g.shape)
+    wz = g.dzf[1:-1]
+    inner = (slice(1, -1),) * 3
+    f[inner] -= (f[inner].sum(axis=(1, 2)) * wz).sum() / (wz.sum() * nx * ny)
+    ref = f.copy()
+    orc.OraclePPE(nx, ny, nz, g.dx, g.dy, g.dzf, pin_gauge=True).solve(ref)
+    s = PoissonSolver(nx, ny, nz, g.dx, g.dy, g.dzf)
+    p, q = (torch.from_numpy(f.copy()).to(cuda) for _ in range(2))
+    s.solve(p)
+    s.solve_refined(q, 2)
+    top = np.abs(ref[inner]).max()
+    assert np.abs(p.cpu().numpy() - ref)[inner].max() <= 1e-12 * top
+    assert np.abs(q.cpu().numpy() - ref)[inner].max() <= 1e-11 * top
