@@ -89,7 +89,7 @@ static int make_plan(int L, int maxT, pll_fftplan *p)
 {
     memset(p, 0, sizeof *p);
     /* PLL_FFT_E (tuning): points per thread, of a compile-time plan when a length
-     * has two, of a runtime plan where it divides the length */
+     * has two, of a runtime plan where it divides the length and has a kernel */
     const char *pe = getenv("PLL_FFT_E");
     const int want = pe ? atoi(pe) : 0;
     if (pll_fft_ct_plan(L, want, p)) return PLL_OK;
@@ -131,6 +131,9 @@ static int make_plan(int L, int maxT, pll_fftplan *p)
                      five[9] = {5, 4, 6, 8, 12, 3, 7, 2}, regs[9] = {12, 8, 24, 6, 4, 3, 5, 7, 2},
                      twice[9] = {5, 4, 12, 8, 6, 7, 3, 2}, many[9] = {12, 8, 6, 5, 3, 7, 4, 2},
                      one[9] = {12, 6, 4, 3, 5, 8, 7, 2}, last[9] = {24};
+    if (pll_fft_supported_E(want) && L % want == 0 && L / want <= pll_fft_max_threads(want) &&
+        plan_for_E(L, want, cnt, big, 0, p))
+        return PLL_OK;
     const int large = c6[4] || c6[5], small = L < 128 && !(L % 5 == 0 && L >= 120);
     const int *list = small ? (L < 100 ? few100 : few) : (L % 5 == 0 ? five : few);
     const struct { const int *list; int reg_only, maxT, half; } pass[5] = {
@@ -145,7 +148,6 @@ static int make_plan(int L, int maxT, pll_fftplan *p)
             const int E = *e, T = L / E;
             if (L % E != 0 || !pll_fft_supported_E(E)) continue;
             if (T > pass[i].maxT || (pass[i].half ? 2 * T : T) > pll_fft_max_threads(E)) continue;
-            if (want > 0 && E != want && L % want == 0) continue;
             if (plan_for_E(L, E, cnt, big, pass[i].reg_only, p)) return PLL_OK;
         }
     return pll_set_error(PLL_EUNSUP, "no FFT plan for length %d", L);

@@ -61,3 +61,14 @@ def test_plan_measured(lib, axis, L, E):
     """Lengths on either side of the rule's lines, as they were measured."""
     fn = lib.pll_fft_plan_info if axis == "x" else lib.pll_fft_plan_info_y
     assert _points(fn, L) == E
+
+
+@pytest.mark.parametrize("want,L,taken", [("8", 80, True), ("2", 130, True), ("10", 80, False),
+                                          ("2", 2000, False), ("9", 2268, False),
+                                          ("x", 80, False), ("12", 64, False)])
+def test_plan_override(lib, monkeypatch, want, L, taken):
+    """PLL_FFT_E is taken where a kernel of as many points divides the length
+    within its thread limit; otherwise the plan is the one without it."""
+    plain = _points(lib.pll_fft_plan_info_y, L)
+    monkeypatch.setenv("PLL_FFT_E", want)
+    assert _points(lib.pll_fft_plan_info_y, L) == (int(want) if taken else plain) != 0
