@@ -498,12 +498,14 @@ __global__ void __launch_bounds__(256) k_rhs_adj(G g, const double *__restrict__
 // on its wall row), and the transposed forcing l -= dzflzi(k) tot of the
 // components in fmask is applied as l is read (tot: sum of l over the interior
 // / (nx ny)).  In the pressure gradient it cancels for u and v.
-#define PLL_CELL                                                   \
+// A workgroup's column of cells: planes blockIdx.z + 1, + gridDim.z, ... (a grid's
+// z extent ends at 65535).
+#define PLL_COLUMN                                                 \
     const int i = blockIdx.x * blockDim.x + threadIdx.x + 1;       \
     const int j = blockIdx.y * blockDim.y + threadIdx.y + 1;       \
-    const int k = blockIdx.z + 1;                                  \
     if (i > g.nx || j > g.ny) return;                              \
-    const long long sy = g.sy, sz = g.sz, e = i + sy * j + sz * k;
+    const long long sy = g.sy, sz = g.sz;                          \
+    for (int k = blockIdx.z + 1; k <= g.nz; k += gridDim.z)
 
 __global__ void __launch_bounds__(256) k_correct_adj_fold(G g, const double *__restrict__ lu,
                                                           const double *__restrict__ lv,
@@ -512,12 +514,16 @@ __global__ void __launch_bounds__(256) k_correct_adj_fold(G g, const double *__r
                                                           double dtdyi, int fmask,
                                                           const double *__restrict__ tot)
 {
-    PLL_CELL
     const double sw = (fmask & 4) ? tot[2] : 0.0;
-    const double um = lu[i == 1 ? e - 1 + g.nx : e - 1], vm = lv[j == 1 ? e + sy * (g.ny - 1) : e - sy];
-    const double wt = k < g.nz ? g.dzc_inv[k] * (lw[e] - g.dzflzi[k] * sw) : 0.0;
-    const double wb = k > 1 ? g.dzc_inv[k - 1] * (lw[e - sz] - g.dzflzi[k - 1] * sw) : 0.0;
-    lp[e] = dtdxi * (lu[e] - um) + dtdyi * (lv[e] - vm) + g.dt * (wt - wb);
+    PLL_COLUMN
+    {
+        const long long e = i + sy * j + sz * k;
+        const double um = lu[i == 1 ? e - 1 + g.nx : e - 1],
+                     vm = lv[j == 1 ? e + sy * (g.ny - 1) : e - sy];
+        const double wt = k < g.nz ? g.dzc_inv[k] * (lw[e] - g.dzflzi[k] * sw) : 0.0;
+        const double wb = k > 1 ? g.dzc_inv[k - 1] * (lw[e - sz] - g.dzflzi[k - 1] * sw) : 0.0;
+        lp[e] = dtdxi * (lu[e] - um) + dtdyi * (lv[e] - vm) + g.dt * (wt - wb);
+    }
 }
 
 __global__ void __launch_bounds__(256) k_rhs_adj_fold(G g, const double *__restrict__ lr,
@@ -527,15 +533,24 @@ __global__ void __launch_bounds__(256) k_rhs_adj_fold(G g, const double *__restr
                                                       double dtidxi, double dtidyi, int fmask,
                                                       const double *__restrict__ tot)
 {
-    PLL_CELL
-    const double wk = g.dzflzi[k];
-    const double rc = lr[e], rx = lr[i == g.nx ? e + 1 - g.nx : e + 1];
-    const double ry = lr[j == g.ny ? e - sy * (g.ny - 1) : e + sy], rz = k < g.nz ? lr[e + sz] : 0.0;
-    const double tu = (fmask & 1) ? wk * tot[0] : 0.0, tv = (fmask & 2) ? wk * tot[1] : 0.0,
-                 tw = (fmask & 4) ? wk * tot[2] : 0.0;
-    lu[e] = (lu[e] - tu) + dtidxi * (rc - rx);
-    lv[e] = (lv[e] - tv) + dtidyi * (rc - ry);
-    lw[e] = k == g.nz ? 0.0 : (lw[e] - tw) + dti * (g.dzf_inv[k] * rc - g.dzf_inv[k + 1] * rz);
+    PLL_COLUMN
+    {
+        const long long e = i + sy * j + sz * k;
+        const double wk = g.dzflzi[k];
+        const double rc = lr[e], rx = lr[i == g.nx ? e + 1 - g.nx : e + 1];
+        const double ry = lr[j == g.ny ? e - sy * (g.ny - 1) : e + sy],
+                     rz = k < g.nz ? lr[e + sz] : 0.0;
+        const double tu = (fmask & 1) ? wk * tot[0] : 0.0, tv = (fmask & 2) ? wk * tot[1] : 0.0,
+                     tw = (fmask & 4) ? wk * tot[2] : 0.0;
+        lu[e] = (lu[e] - tu) + dtidxi * (rc - rx);
+        lv[e] = (lv[e] - tv) + dtidyi * (rc - ry);
+        lw[e] = k == g.nz ? 0.0 : (lw[e] - tw) + dti * (g.dzf_inv[k] * rc - g.dzf_inv[k + 1] * rz);
+    }
+}
+
+inline dim3 column_grid(const G &g)
+{
+    return dim3((g.nx + 63) / 64, (g.ny + 3) / 4, g.nz < 65535 ? g.nz : 65535);
 }
 
 // ------------------------------------------------------------ forcing
@@ -803,9 +818,8 @@ extern "C" int pll_launch_correct_adj_fold(const pll_grid_dev *gd, const double 
                                            double *lp, int fmask, const double *tot, hipStream_t s)
 {
     const G g = make_g(gd);
-    hipLaunchKernelGGL(k_correct_adj_fold, dim3((g.nx + 63) / 64, (g.ny + 3) / 4, g.nz),
-                       dim3(64, 4, 1), 0, s, g, l[0], l[1], l[2], lp, g.dt * g.dx_inv,
-                       g.dt * g.dy_inv, fmask, tot);
+    hipLaunchKernelGGL(k_correct_adj_fold, column_grid(g), dim3(64, 4, 1), 0, s, g, l[0], l[1],
+                       l[2], lp, g.dt * g.dx_inv, g.dt * g.dy_inv, fmask, tot);
     return ok();
 }
 
@@ -815,9 +829,8 @@ extern "C" int pll_launch_rhs_adj_fold(const pll_grid_dev *gd, const double *lr,
 {
     const G g = make_g(gd);
     const double dti = 1.0 / g.dt;
-    hipLaunchKernelGGL(k_rhs_adj_fold, dim3((g.nx + 63) / 64, (g.ny + 3) / 4, g.nz),
-                       dim3(64, 4, 1), 0, s, g, lr, l[0], l[1], l[2], dti, dti * g.dx_inv,
-                       dti * g.dy_inv, fmask, tot);
+    hipLaunchKernelGGL(k_rhs_adj_fold, column_grid(g), dim3(64, 4, 1), 0, s, g, lr, l[0], l[1],
+                       l[2], dti, dti * g.dx_inv, dti * g.dy_inv, fmask, tot);
     return ok();
 }
 

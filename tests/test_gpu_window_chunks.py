@@ -69,3 +69,61 @@ def test_window_gradient_does_not_depend_on_chunks(cuda, shape, forced, monkeypa
     for other in got[1:]:
         for a, b in zip(other, got[0]):
             assert float((a - b).abs().max()) <= 1e-11 * top
+
+
+def test_window_gradient_many_planes(cuda):
+    """More planes than a launch grid's z extent: the window's reversed steps
+    against the public transposes applied one after the other.  The mean mode's
+    pressure is summed over 65600 planes up to 65600 times its own difference
+    from plane to plane, so those differences are good to some 65600 roundings,
+    7e-12 of the largest; 1e-9."""
+    import torch
+    from powerllel_channel_amd import Channel, PoissonSolver
+    from powerllel_channel_amd.adjoint import WallShearWindow
+    from powerllel_channel_amd.mesh import Grid
+    nx, ny, nz, nu, dt, n = 4, 2, 65600, 1e-2, 1e-3, 2
+    print(f"[window gradient] {(nx, ny, nz)}", flush=True)
+    g = Grid(nx, ny, nz, 0.1 * nx, 0.1 * ny, 0.1 * nz, 0.0)
+    ch = Channel(nx, ny, nz, g.lx, g.ly, g.lz, g.dzf, nu, dt, is_forced=(False, False, False))
+    s = PoissonSolver(nx, ny, nz, g.dx, g.dy, g.dzf)
+    gen = torch.Generator().manual_seed(6)
+    f = [0.3 * torch.randn(g.shape, generator=gen, dtype=torch.float64).to(cuda) for _ in range(6)]
+    ch.bc_vel(*f[:3])
+    win = WallShearWindow(ch, s, n, 1)
+    win.forward(*f)
+    got = [torch.full_like(f[0], 9.0) for _ in range(3)]
+    win.backward(*got)
+
+    def zeros(m):
+        return [torch.zeros_like(f[0]) for _ in range(m)]
+
+    def seed(lam):
+        for k in (1, nz):
+            lam[0][k, 1:-1, 1:-1] += nu / (n * nx * ny) / g.dzf[k]
+    inner = (slice(1, -1),) * 3
+    second = [t.clone() for t in f[:3]]
+    ch.step_body(s, *second, *zeros(4), *f[3:])
+    lam, grad = zeros(3), zeros(3)
+    seed(lam)
+    for state in (second, f[:3]):
+        u1, (lp,), l1 = zeros(3), zeros(1), zeros(3)
+        ch.rk1(*state, *u1)
+        for t, b in zip(u1, f[3:]):
+            t[inner] += dt * b[inner]
+        ch.bc_vel(*u1)
+        ch.bc_vel_adj(*lam)
+        ch.correct_vel_adj(*lam, lp)
+        ch.bc_p_adj(lp)
+        s.solve_adjoint(lp)
+        ch.calc_rhs_adj(lp, *lam)
+        ch.bc_vel_adj(*lam)
+        ch.rk_vjp(u1, lam, l1, 0.5 * dt, 0.5, 0.0)
+        ch.bc_vel_adj(*l1)
+        for q, a, d in zip(grad, lam, l1):
+            q += 0.5 * dt * a + dt * d
+        ch.rk_vjp(state, l1, lam, dt, 1.0, 0.5)
+        seed(lam)
+    for q, want in zip(got, grad):
+        top = float(want.abs().max())
+        assert float(want[65540:, 1:-1, 1:-1].abs().max()) > 0.01 * top > 0.0
+        assert float((q - want).abs().max()) <= 1e-9 * top
