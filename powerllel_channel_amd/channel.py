@@ -113,8 +113,9 @@ class Channel:
 
     def check(self, u, v, w, cfl_limit, div_limit, stream=None):
         """The run-time check of src/main.f90:213-222: checkNaN(u), calcMaxCFL +
-        checkCFL, calcMaxDiv + checkDiv, in one pass over the fields.  Returns (passed, report); a value
-        above its limit or NaN fails, as in checkCFL / checkDiv."""
+        checkCFL, calcMaxDiv + checkDiv, in one pass over the fields.  Returns
+        (passed, report); a value above its limit or NaN fails, as in checkCFL /
+        checkDiv."""
         self._chk(u, v, w)
         flag, vals, at = C.c_int(), (C.c_double(), C.c_double()), ((C.c_int * 3)(), (C.c_int * 3)())
         check(lib().pll_channel_check(self._h, _p(u), _p(v), _p(w), C.byref(flag),
@@ -133,8 +134,10 @@ class Channel:
                                      _p(w1), _p(p), _stream_ptr(stream)))
 
     def run(self, ppe: PoissonSolver, nsteps, u, v, w, u1, v1, w1, p, stream=None):
-        """nsteps steps, equal to nsteps calls of step(); with the FP64 solve
-        the projection of each step is formed in the next step's RK1."""
+        """nsteps steps, equal to nsteps calls of step() bit for bit in u, v, w
+        and p; with the FP64 solve and w not forced each step's projection is
+        formed as the next step reads the velocity.  u1, v1, w1 are work space:
+        what they hold after the call is unspecified."""
         self._chk(u, v, w, u1, v1, w1, p)
         check(lib().pll_channel_run(self._h, ppe.handle, int(nsteps), _p(u), _p(v), _p(w),
                                     _p(u1), _p(v1), _p(w1), _p(p), _stream_ptr(stream)))

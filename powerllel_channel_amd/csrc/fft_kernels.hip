@@ -1589,7 +1589,7 @@ extern "C" int pll_fft_supported_E(int E)
 extern "C" int pll_fft_max_threads(int E) { return E >= 12 ? 256 : 512; }
 extern "C" int pll_fft_max_threads32(int) { return 512; }
 
-extern "C" int pll_fft_ct_plan(int L, int prefer_E, pll_fftplan *p)
+extern "C" int pll_fft_ct_plan(int L, pll_fftplan *p)
 {
     const int plans[][8] = {
 #define PLL_CT_ROW(L_, E_, ...) {L_, E_, __VA_ARGS__},
@@ -1597,10 +1597,8 @@ extern "C" int pll_fft_ct_plan(int L, int prefer_E, pll_fftplan *p)
 #undef PLL_CT_ROW
     };
     int pick = -1;
-    for (size_t i = 0; i < sizeof plans / sizeof plans[0]; i++) {
-        if (plans[i][0] != L) continue;
-        if (pick < 0 || plans[i][1] == prefer_E) pick = (int)i;
-    }
+    for (size_t i = 0; i < sizeof plans / sizeof plans[0]; i++)
+        if (plans[i][0] == L) pick = (int)i;
     if (pick < 0) return 0;
     p->L = L;
     p->E = plans[pick][1];

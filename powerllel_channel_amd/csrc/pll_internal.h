@@ -178,9 +178,8 @@ int pll_fft_supported_E(int E);
  * the FP32 ones take pll_fft_max_threads32) */
 int pll_fft_max_threads(int E);
 int pll_fft_max_threads32(int E);
-/* compile-time plan for length L, if one exists (returns 1 and fills p);
- * among several, the one with E == prefer_E, else the first listed */
-int pll_fft_ct_plan(int L, int prefer_E, pll_fftplan *p);
+/* compile-time plan for length L, if one exists (returns 1 and fills p) */
+int pll_fft_ct_plan(int L, pll_fftplan *p);
 /* the plan the solver uses for an x transform of length L, a y transform of
  * length ny (host only): E, stage count, radices */
 int pll_fft_plan_info(int L, int *E, int *nst, int *rad);

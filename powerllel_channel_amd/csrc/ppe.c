@@ -88,11 +88,11 @@ enum { PLL_MAXT_X = 256, PLL_MAXT_Y = 64 };
 static int make_plan(int L, int maxT, pll_fftplan *p)
 {
     memset(p, 0, sizeof *p);
-    /* PLL_FFT_E (tuning): points per thread, of a compile-time plan when a length
-     * has two, of a runtime plan where it divides the length and has a kernel */
+    /* PLL_FFT_E (tuning): points per thread of a runtime plan, where it divides the
+     * length and has a kernel */
     const char *pe = getenv("PLL_FFT_E");
     const int want = pe ? atoi(pe) : 0;
-    if (pll_fft_ct_plan(L, want, p)) return PLL_OK;
+    if (pll_fft_ct_plan(L, p)) return PLL_OK;
     memset(p, 0, sizeof *p);
     if (L < 2) return pll_set_error(PLL_EUNSUP, "FFT length %d < 2", L);
     static const int primes[6] = {2, 3, 5, 7, 11, 13};
@@ -371,22 +371,26 @@ static int choose_launch(pll_ppe *h)
     return PLL_OK;
 }
 
-/* Layout of the partitioned z solve: M rows per lane (M in {8,12,16,4}),
- * P = nz/M lanes per column (a power of two, 2..64, so a column's lanes share
- * one wavefront), S columns per tile (16, 8 or 4 doubles = one 128/64/32-byte
- * row segment); LDS holds the tile twice (values and, for low-mode tiles,
- * pivots).  Returns 0 (streaming solve) if nothing fits. */
+/* Regular layout of the partitioned z solve: M rows per lane (M in
+ * {8,12,16,4}), P = nz/M lanes per column (a power of two, 2..64, so a column's
+ * lanes share one wavefront), S columns per tile (32, 16, 8 or 4 doubles = a
+ * 256/128/64/32-byte row segment); LDS holds the tile's values and the z
+ * coefficients.  Returns 0 if nothing fits. */
 static int part_fits(int nx, int ny, int nz, int m, int *M, int *P, int *S)
 {
     /* widest first: a tile row of 32 FP64 columns is 256 contiguous bytes,
      * which HBM serves faster than 128-byte pieces (768x384x256: 0.270 ->
      * 0.253 ms against 16 columns, same box).  Not where W stays in the 256 MiB
-     * Infinity Cache and tiles are tall: there twice the tiles, two to a CU,
-     * hide each other's waits and leave a shorter last round.  us per solve, 32
-     * against 16 columns: 96x96x256 73 / 68, 192x192x128 88 / 85, 192x192x256
-     * 145 / 136, 512x384x128 370 / 348, refined 192x192x128 203 / 192; no gain
-     * up to 16 MiB or 96 planes (128x128x128 58.8 / 59.4, 384x192x96 117 / 120)
-     * and beyond the cache (512x256x256 462 / 462, 768x384x192 833 / 836). */
+     * Infinity Cache and tiles are tall: there S = 16 makes workgroups of 256
+     * threads, two or three to a CU where 512 threads are alone, which hide each
+     * other's waits and leave a shorter last round.  At M = 16 (nz = 256) their
+     * tiles are 16 columns wide, twice as many; at M = 8 and 12, where nx is a
+     * multiple of 32, 32 columns as before, solved as two groups in turn (h64).
+     * us per solve, S = 32 against 16: M = 16 96x96x256 73 / 68, 192x192x256
+     * 144 / 134; M = 8 192x192x128 89 / 86, 512x384x128 364 / 342, refined
+     * 192x192x128 205 / 194; M = 12 96x128x192 67 / 67; no gain up to 16 MiB or
+     * 96 planes (128x128x128 58.8 / 59.4, 384x192x96 117 / 120) and beyond the
+     * cache (512x256x256 462 / 462, 768x384x192 833 / 836). */
     static const int Ss[] = {32, 16, 8, 4};
     const size_t w = sizeof(double) * (size_t)nx * ny * nz;
     const int narrow = nz >= 128 && w > (size_t)16 << 20 && w <= (size_t)256 << 20;

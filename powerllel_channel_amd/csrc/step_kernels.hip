@@ -825,11 +825,11 @@ inline int ok() { return hipGetLastError() == hipSuccess ? 0 : -3; }
 // 16: 2.64), and one size up or down from its choice is 0 to 20% slower.
 constexpr int RK_WG_MIN = 2048, RK_KC_MAX = 64;
 
-Tiles rk_tiles(const G &g, int ty = RK_TY)
+Tiles rk_tiles(const G &g)
 {
     Tiles t;
     t.ntx = (g.nx + RK_TX - 1) / RK_TX;
-    t.nty = (g.ny + ty - 1) / ty;
+    t.nty = (g.ny + RK_TY - 1) / RK_TY;
     const long long cols = (long long)t.ntx * t.nty;
     t.kc = RK_KC_MAX;
     while (t.kc > 1 && cols * ((g.nz + t.kc - 1) / t.kc) < RK_WG_MIN) t.kc >>= 1;
