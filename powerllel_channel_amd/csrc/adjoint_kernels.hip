@@ -660,7 +660,7 @@ inline unsigned nblk(long long n) { return (unsigned)((n + 255) / 256); }
 // Tiles of an nx x ny x nz box: k chunks of up to 32 planes, shorter on small
 // boxes so that 1536 workgroups run (two rounds of the three that fit a CU):
 // 256x192x128 145 us with 16 planes, 161 with 32, 148 with 8; 512x384x256
-// 974 us with 32, 985 with 16.
+// 974 us with 32, 985 with 16.  Then even chunks, as the stencil tiles.
 JTiles jt_tiles(int nx, int ny, int nz, int kc)
 {
     JTiles t;
@@ -669,7 +669,8 @@ JTiles jt_tiles(int nx, int ny, int nz, int kc)
     const long long cols = (long long)t.ntx * t.nty;
     t.kc = 32;
     while (t.kc > 1 && cols * ((nz + t.kc - 1) / t.kc) < 1536) t.kc >>= 1;
-    if (kc > 0) t.kc = kc;
+    const int n = (nz + t.kc - 1) / t.kc;
+    t.kc = kc > 0 ? kc : (nz + n - 1) / n;
     t.nkc = (nz + t.kc - 1) / t.kc;
     t.xcd = (cols * t.nkc) % 8 == 0;
     return t;

@@ -813,8 +813,8 @@ __global__ void __launch_bounds__(256) k_nan_part(const double *__restrict__ q, 
 
 inline int ok() { return hipGetLastError() == hipSuccess ? 0 : -3; }
 
-// Planes per k chunk (PLL_RK_KC overrides): the largest power of two up to 64
-// that leaves at least 2048 workgroups.  A chunk costs two planes of loads
+// Planes per k chunk (PLL_RK_KC overrides): at first the largest power of two up
+// to 64 that leaves at least 2048 workgroups.  A chunk costs two planes of loads
 // before its first result, so long chunks are cheaper per plane; but the chip
 // holds 4 workgroups per CU, 1024, and with fewer than two rounds of them it
 // idles (a 64-plane chunk of a 64x64x64 grid makes 16 workgroups).  Measured,
@@ -823,6 +823,9 @@ inline int ok() { return hipGetLastError() == hipSuccess ? 0 : -3; }
 // 240x140x90 492 -> 347 us (4), 384x384x192 1.81 -> 1.51 ms (32; 64 leaves
 // 1728 workgroups); at 512x384x256 the rule keeps 64 (2.61 ms, 32: 2.62,
 // 16: 2.64), and one size up or down from its choice is 0 to 20% slower.
+// The planes are then spread evenly over as many chunks: with the XCD numbering
+// an XCD runs the tiles of one or two chunks, and short ones leave it idle (step
+// at 768x384x39 as 32 + 7 planes 884 us, as 20 + 19 726, as one chunk 728).
 constexpr int RK_WG_MIN = 2048, RK_KC_MAX = 64;
 
 Tiles rk_tiles(const G &g)
@@ -833,7 +836,8 @@ Tiles rk_tiles(const G &g)
     const long long cols = (long long)t.ntx * t.nty;
     t.kc = RK_KC_MAX;
     while (t.kc > 1 && cols * ((g.nz + t.kc - 1) / t.kc) < RK_WG_MIN) t.kc >>= 1;
-    if (g.kc > 0) t.kc = g.kc;
+    const int n = (g.nz + t.kc - 1) / t.kc;
+    t.kc = g.kc > 0 ? g.kc : (g.nz + n - 1) / n;
     t.nkc = (g.nz + t.kc - 1) / t.kc;
     t.xcd = (cols * t.nkc) % 8 == 0;
     return t;

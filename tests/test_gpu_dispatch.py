@@ -77,3 +77,32 @@ def test_plans_against_oracle(orc, cuda, shape):
     top = np.abs(ref[inner]).max()
     assert np.abs(p.cpu().numpy() - ref)[inner].max() <= 1e-12 * top
     assert np.abs(q.cpu().numpy() - ref)[inner].max() <= 1e-11 * top
+
+
+# k chunks of odd and even lengths, several and short last ones, with and without
+# partial sums of Mean_h
+@pytest.mark.parametrize("kc", ["3", "5", "10", "13"])
+@pytest.mark.parametrize("forced", [(True, True, False), (False, False, False)])
+def test_run_equals_steps_on_chunks(cuda, forced, kc, monkeypatch):
+    """pll_channel_run against as many calls of pll_channel_step, bit for bit."""
+    import torch
+    from powerllel_channel_amd import Channel, PoissonSolver
+    from powerllel_channel_amd.mesh import Grid
+    monkeypatch.setenv("PLL_RK_KC", kc)
+    nx, ny, nz = 70, 26, 29
+    print(f"[run = steps] kc={kc} forced={forced}", flush=True)
+    g = Grid(nx, ny, nz, 0.1 * nx, 0.1 * ny, 2.0, 2.0)
+    ch = Channel(nx, ny, nz, g.lx, g.ly, g.lz, g.dzf, 1e-3, 1e-3, u_crf=0.2, is_forced=forced,
+                 vel_force=(1.0, 0.2, 0.0))
+    s = PoissonSolver(nx, ny, nz, g.dx, g.dy, g.dzf)
+    gen = torch.Generator().manual_seed(8)
+    f = [0.3 * torch.randn(g.shape, generator=gen, dtype=torch.float64).to(cuda) for _ in range(3)]
+    ch.bc_vel(*f)
+    a = [t.clone() for t in f] + [torch.zeros_like(f[0]) for _ in range(4)]
+    b = [t.clone() for t in a]
+    ch.run(s, 4, *a)
+    for _ in range(4):
+        ch.step(s, *b)
+    for q in (0, 1, 2, 6):
+        assert torch.isfinite(b[q]).all()
+        assert torch.equal(a[q], b[q]), q
