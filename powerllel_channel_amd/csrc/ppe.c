@@ -628,12 +628,16 @@ int pll_ppe_create(pll_ppe **out, int nx, int ny, int nz, double dx, double dy,
         int M, P, S, rM, rP = 0, rS;
         int part = choose_part(nx, ny, nz, &M, &P, &S);
         /* Ragged tiles for FP64 where the regular layout does not exist, or has 4
-         * columns (32-byte row segments): 500x250x128 498 -> 442 us per solve,
-         * 100x100x64 43 -> 40.  With 8 columns and more the regular one is faster:
-         * 360x128x128 159 us (ragged 166), 400x256x128 242 (257).
+         * columns (32-byte row segments) and the plane has columns enough for the
+         * chip.  us per solve, regular against ragged: 100x100x64 40.9 / 39.1,
+         * 84x84x128 48.9 / 47.4, 180x180x256 246 / 209, 500x250x128 366 / 303;
+         * 60x60x64 27.2 / 28.2, 60x60x256 49.5 / 55.3, 28x16x256 27.6 / 37.7.
+         * With 8 columns and more the regular one is faster: 360x128x128 159 us
+         * (ragged 166), 400x256x128 242 (257).
          * PLL_TRID_RAG (tuning): 0 never, 1 always and nothing else */
         const char *pr = getenv("PLL_TRID_RAG");
-        int rag = choose_rag(nz, &rM, &rP, &rS) && (pr ? atoi(pr) != 0 : !part || S < 8);
+        int rag = choose_rag(nz, &rM, &rP, &rS) &&
+                  (pr ? atoi(pr) != 0 : !part || (S < 8 && (long long)nx * ny >= 5000));
         /* FP32 storage then keeps the regular tiles of 4 columns: a workgroup of
          * 4 P lanes, against the streaming solve's one lane per two columns and one
          * chain of nz rows, which many columns and few planes favour.  us per

@@ -106,3 +106,28 @@ def test_run_equals_steps_on_chunks(cuda, forced, kc, monkeypatch):
     for q in (0, 1, 2, 6):
         assert torch.isfinite(b[q]).all()
         assert torch.equal(a[q], b[q]), q
+
+
+# regular tiles of 4 columns below 5000 columns, ragged ones from there on and
+# where there are no regular ones
+@pytest.mark.parametrize("shape,rag", [((4, 4, 256), "0"), ((28, 16, 192), "0"), ((60, 80, 64), "0"),
+                                       ((60, 84, 64), "1"), ((100, 100, 128), "1"),
+                                       ((12, 10, 50), "1")])
+def test_fp64_z_tiles_of_4_columns(cuda, shape, rag, monkeypatch):
+    """The solve and its transpose are bit for bit those of a solver held to the
+    tiles the rule names."""
+    import torch
+    from powerllel_channel_amd import PoissonSolver
+    from powerllel_channel_amd.mesh import Grid
+    nx, ny, nz = shape
+    print(f"[fp64, 4-column z tiles] {shape}", flush=True)
+    g = Grid(nx, ny, nz, 6.0, 3.0, 2.0, 2.0)
+    f = torch.from_numpy(np.random.default_rng(23).standard_normal(g.shape)).to(cuda)
+    default = PoissonSolver(nx, ny, nz, g.dx, g.dy, g.dzf)
+    monkeypatch.setenv("PLL_TRID_RAG", rag)
+    held = PoissonSolver(nx, ny, nz, g.dx, g.dy, g.dzf)
+    for name in ("solve", "solve_adjoint"):
+        p, q = f.clone(), f.clone()
+        getattr(default, name)(p)
+        getattr(held, name)(q)
+        assert torch.isfinite(q).all() and torch.equal(p, q), name
