@@ -180,10 +180,11 @@ int pll_fft_max_threads(int E);
 int pll_fft_max_threads32(int E);
 /* compile-time plan for length L, if one exists (returns 1 and fills p) */
 int pll_fft_ct_plan(int L, pll_fftplan *p);
-/* the plan the solver uses for an x transform of length L, a y transform of
- * length ny (host only): E, stage count, radices */
+/* the plan the solver of a grid of so many cells uses for an x transform of length
+ * L (y = 0), a y transform of length L (y = 1) (host only): E, stage count,
+ * radices; the first one: x, a large grid */
 int pll_fft_plan_info(int L, int *E, int *nst, int *rad);
-int pll_fft_plan_info_y(int ny, int *E, int *nst, int *rad);
+int pll_fft_plan_info_grid(int L, int y, long long cells, int *E, int *nst, int *rad);
 
 /* Grid constants for the step kernels (device pointers for z arrays). */
 typedef struct {

@@ -85,7 +85,8 @@ static int plan_for_E(int L, int E, const int cnt[4], const int cnt_big[2], int 
  * rows, a y tile of 8 columns. */
 enum { PLL_MAXT_X = 256, PLL_MAXT_Y = 64 };
 
-static int make_plan(int L, int maxT, pll_fftplan *p)
+/* cells: of the grid */
+static int make_plan(int L, int maxT, long long cells, pll_fftplan *p)
 {
     memset(p, 0, sizeof *p);
     /* PLL_FFT_E (tuning): points per thread of a runtime plan, where it divides the
@@ -112,35 +113,45 @@ static int make_plan(int L, int maxT, pll_fftplan *p)
      * - longer ones with a factor 5: 5 (4 -> 5: 240x140x90 90 -> 81, 320x160x64 90
      *   -> 78, 640x320x64 265 -> 226; below 120 4 is faster, 200x100x64 52 for 56);
      * - other longer ones: all stages in registers (288x144x64, 576x288x64: 87 and
-     *   229 us with 12, 88 and 238 with 4), else 4;
-     * - lengths with a factor 11 or 13, any size: many, 12, 8 or 6, as long as a
+     *   229 us with 12, 88 and 238 with 4), else 4.
+     * 24 points take 228 registers, two waves per SIMD (both y passes at 256x960x64
+     * 245 us, with 5 160; x passes at 6720x128x64 1678, with 8 1010): only where
+     * nothing else divides the length.
+     * That is all up to 2^20 cells, where the length of a thread's work counts.
+     * Larger grids fill the chip with fewer threads to a row too, and then:
+     * - lengths with a factor 11 or 13 take many points, 12, 8 or 6, as long as a
      *   workgroup holds two rows: the registers that the large butterflies need
      *   are there either way (both y passes at 256 x ny x 64, 3 to 5 points
      *   against this: 104 40 / 33 us, 312 89 / 55, 462 149 / 98, 832 224 / 155,
      *   1092 494 / 202; x passes at 2 L x 128 x 64: 330 109 / 84, 660 254 / 149,
-     *   1404 390 / 298; the one case the other way, x at 1040: 308 / 343).
-     * Then the width of a y tile: at most 64 threads a column leave room for 8
-     * columns (4 from 12 points on); where no E of the list does that, tiles of
-     * two columns and more are wide enough for fewer points to be faster (640: 4
-     * columns of 5 points 92 us, 6 of 8 117), but one column, 16 bytes of a row,
-     * is not (1400: 5 points 361, 8 points 318; 1440: 402, with 12 295; 1568: 4
-     * points 394, 8 points 351).
-     * 24 points take 228 registers, two waves per SIMD (960: 245, with 5 160;
-     * x 3360: 1678, with 8 1010): only where nothing else divides the length. */
-    static const int few100[9] = {3, 4, 6, 5, 8, 7, 2, 12}, few[9] = {4, 6, 3, 5, 8, 7, 2, 12},
-                     five[9] = {5, 4, 6, 8, 12, 3, 7, 2}, regs[9] = {12, 8, 24, 6, 4, 3, 5, 7, 2},
+     *   1404 390 / 298; the one case the other way, x at 1040: 308 / 343);
+     * - 6 comes before 3 (882 242 / 131; x at 294 74 / 57);
+     * - a y tile has two columns and more: 64 threads a column leave room for 8 (4
+     *   from 12 points on), and where no E of the list does that, tiles of two are
+     *   wide enough for fewer points to be faster (640: 4 columns of 5 points 92
+     *   us, 6 of 8 117), but one column, 16 bytes of a row, is not (1400: 5 points
+     *   361, 8 points 318; 1440: 402, with 12 295; 1568: 4 points 394, 8 points 351).
+     * Where the line lies (solve, few points / this): 264x32x64 35 / 43, 264x64x64
+     * 57 / 54; 64x132x64 34 / 39, 128x132x64 56 / 53; 16x882x32 36 / 38, 32x882x32
+     * 48 / 47; 16x1400x32 45 / 49, 32x1400x32 65 / 66, 32x1400x64 99 / 91; x at 702
+     * 0.69M cells 44 / 45, 1.37M 73 / 62. */
+    const int wide = cells > 1LL << 20;
+    static const int few100[9] = {3, 4, 6, 5, 8, 7, 2, 12}, few3[9] = {4, 3, 6, 5, 8, 7, 2, 12},
+                     few6[9] = {4, 6, 3, 5, 8, 7, 2, 12}, five[9] = {5, 4, 6, 8, 12, 3, 7, 2},
+                     regs[9] = {12, 8, 24, 6, 4, 3, 5, 7, 2},
                      twice[9] = {5, 4, 12, 8, 6, 7, 3, 2}, many[9] = {12, 8, 6, 5, 3, 7, 4, 2},
                      one[9] = {12, 6, 4, 3, 5, 8, 7, 2}, last[9] = {24};
+    const int *few = wide ? few6 : few3;
     if (pll_fft_supported_E(want) && L % want == 0 && L / want <= pll_fft_max_threads(want) &&
         plan_for_E(L, want, cnt, big, 0, p))
         return PLL_OK;
-    const int large = c6[4] || c6[5], small = L < 128 && !(L % 5 == 0 && L >= 120);
+    const int large = wide && (c6[4] || c6[5]), small = L < 128 && !(L % 5 == 0 && L >= 120);
     const int *list = small ? (L < 100 ? few100 : few) : (L % 5 == 0 ? five : few);
     const struct { const int *list; int reg_only, maxT, half; } pass[5] = {
         /* stages in registers only; at most maxT threads; room for two rows; any */
         {!large && !small && L % 5 ? regs : NULL, 1, INT_MAX, 0},
         {large ? NULL : list, 0, maxT, 0},
-        {large ? many : twice, 0, INT_MAX, 1},
+        {large ? many : (wide ? twice : NULL), 0, INT_MAX, 1},
         {large ? one : list, 0, INT_MAX, 0},
         {last, 0, INT_MAX, 0}};
     for (int i = 0; i < 5; i++)
@@ -536,8 +547,10 @@ int pll_ppe_create(pll_ppe **out, int nx, int ny, int nz, double dx, double dy,
     h->ny = ny;
     h->nz = nz;
     h->L = nx / 2;
+    const long long cells = (long long)nx * ny * nz;
     int rc;
-    if ((rc = make_plan(h->L, PLL_MAXT_X, &h->d.px)) || (rc = make_plan(ny, PLL_MAXT_Y, &h->d.py)) ||
+    if ((rc = make_plan(h->L, PLL_MAXT_X, cells, &h->d.px)) ||
+        (rc = make_plan(ny, PLL_MAXT_Y, cells, &h->d.py)) ||
         (rc = choose_launch(h))) {
         free(h);
         return rc;
@@ -1325,13 +1338,14 @@ void execute_poisson_solver(double *var)
 
 void free_poisson_solver(void) { abort_on(free_poisson_solver_status(), "free_poisson_solver"); }
 
-/* Host-only query of the plan the solver uses for an x transform of length L
- * (= nx/2) or a y transform of length ny (no device needed): points per thread,
- * stage count and radices (rad: PLL_MAX_STAGES ints). */
-static int plan_info(int L, int maxT, int *E, int *nst, int *rad)
+/* Host-only query of the plan the solver of a grid of so many cells uses for an x
+ * transform of length L (= nx/2), y = 0, or a y transform of length ny, y = 1 (no
+ * device needed): points per thread, stage count and radices (rad: PLL_MAX_STAGES
+ * ints). */
+int pll_fft_plan_info_grid(int L, int y, long long cells, int *E, int *nst, int *rad)
 {
     pll_fftplan p;
-    const int rc = make_plan(L, maxT, &p);
+    const int rc = make_plan(L, y ? PLL_MAXT_Y : PLL_MAXT_X, cells, &p);
     if (rc) return rc;
     *E = p.E;
     *nst = p.nst;
@@ -1339,12 +1353,8 @@ static int plan_info(int L, int maxT, int *E, int *nst, int *rad)
     return PLL_OK;
 }
 
+/* x plan of a large grid */
 int pll_fft_plan_info(int L, int *E, int *nst, int *rad)
 {
-    return plan_info(L, PLL_MAXT_X, E, nst, rad);
-}
-
-int pll_fft_plan_info_y(int ny, int *E, int *nst, int *rad)
-{
-    return plan_info(ny, PLL_MAXT_Y, E, nst, rad);
+    return pll_fft_plan_info_grid(L, 0, LLONG_MAX, E, nst, rad);
 }

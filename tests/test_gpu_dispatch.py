@@ -50,11 +50,14 @@ def test_refined_z_tiles_of_4_columns(cuda, shape, held, monkeypatch):
         assert float((a - b).abs().max()) <= 1e-12 * float(b.abs().max()), name
 
 
-# transform plans: lengths with a factor 11 or 13 at 12, 8, 7, 6 and 4 points per
-# thread, long y transforms in tiles of two columns and of one
+# transform plans: lengths with a factor 11 or 13 and long y transforms, at many
+# threads a row (small grids), and above 2^20 cells at 12, 8, 7, 6 and 4 points per
+# thread in y tiles of two columns and more, and of one
 @pytest.mark.parametrize("shape", [
-    (132, 66, 4), (264, 156, 3), (176, 104, 4), (462, 78, 3), (660, 132, 3), (252, 126, 4),
-    (12, 1400, 3), (20, 1344, 2), (16, 960, 3), (8, 1300, 2), (24, 1764, 2), (10, 1560, 2)])
+    (132, 66, 4), (264, 156, 3), (660, 132, 3), (252, 126, 4), (12, 1400, 3), (16, 960, 3),
+    (8, 1300, 2), (132, 66, 122), (264, 156, 26), (176, 104, 58), (462, 78, 30), (660, 132, 13),
+    (252, 126, 34), (12, 1400, 64), (20, 1344, 40), (16, 960, 70), (8, 1300, 102), (24, 1764, 26),
+    (10, 1560, 68)])
 def test_plans_against_oracle(orc, cuda, shape):
     """Solve against the oracle (1e-12) and the refined form with two sweeps
     (1e-11, its bar)."""
@@ -63,7 +66,7 @@ def test_plans_against_oracle(orc, cuda, shape):
     from powerllel_channel_amd.mesh import Grid
     nx, ny, nz = shape
     print(f"[plans] {shape}", flush=True)
-    g = Grid(nx, ny, nz, 0.05 * nx, 0.05 * ny, 2.0, 1.0)
+    g = Grid(nx, ny, nz, 6.0, 3.0, 2.0, 1.0)
     f = np.random.default_rng(19).standard_normal(g.shape)
     wz = g.dzf[1:-1]
     inner = (slice(1, -1),) * 3
