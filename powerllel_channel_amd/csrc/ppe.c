@@ -1188,9 +1188,10 @@ static int host_setup(pll_ppe *h)
     /* Chunks: a copy and the transfer of the chunk before it run side by side, so
      * only the first copy up and the last one down stand alone, and each chunk
      * costs some 30 us of waits.  Five chunks, each of at least 6 and at most 20
-     * MiB (whole planes); us per solve, slots of 20 MiB against this: 128x128x96
-     * (2 chunks) 833 -> 700, 240x140x90 (3) 1426 -> 1180, 192x192x128 (5) 1838 ->
-     * 1740, 384x192x128 (5) 3309 -> 3300; 3 MiB chunks 748, 1309, 1962, 3353. */
+     * MiB (whole planes); us per solve on one box, slots of 20 MiB against this:
+     * 128x128x96 (2 chunks) 833 -> 700, 240x140x90 (3) 1426 -> 1180, 192x192x128
+     * (5) 1838 -> 1740 (on others 1926 -> 1855), 384x192x128 (5) 3309 -> 3300; 3
+     * MiB chunks 748, 1309, 1962, 3353. */
     const size_t all = plane * (size_t)h->nz;
     size_t nch = all / ((size_t)6 << 20);
     nch = nch < 1 ? 1 : nch > 5 ? 5 : nch;

@@ -113,9 +113,9 @@ def test_run_equals_steps_on_chunks(cuda, forced, kc, monkeypatch):
 
 # regular tiles of 4 columns below 5000 columns, ragged ones from there on and
 # where there are no regular ones
-@pytest.mark.parametrize("shape,rag", [((4, 4, 256), "0"), ((28, 16, 192), "0"), ((60, 80, 64), "0"),
-                                       ((60, 84, 64), "1"), ((100, 100, 128), "1"),
-                                       ((12, 10, 50), "1")])
+@pytest.mark.parametrize("shape,rag", [((4, 4, 256), "0"), ((28, 16, 192), "0"),
+                                       ((60, 80, 64), "0"), ((60, 84, 64), "1"),
+                                       ((100, 100, 128), "1"), ((12, 10, 50), "1")])
 def test_fp64_z_tiles_of_4_columns(cuda, shape, rag, monkeypatch):
     """The solve and its transpose are bit for bit those of a solver held to the
     tiles the rule names."""
